@@ -40,8 +40,9 @@
 // fp16 pair keeps ~22 bits whatever its range); the rest (prep scores, phase 4
 // of the chunk kernel) on v_mfma_f32_16x16x4f32.  Decay factors of
 // off-diagonal 16-row tiles are anchored at the row tile's first row
-// (2^(G_c - G_a) * 2^(G_a - G_i), both <= 1); diagonal tiles likewise when
-// the tile's decay span allows (kDiagAnchorLog2), else per element.
+// (2^(G_c - G_a) * 2^(G_a - G_i), both <= 1; the chunk kernel also at the key
+// tile's last row); diagonal tiles likewise when the tile's decay span allows
+// (kDiagAnchorLog2), else per element.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -55,9 +56,13 @@ namespace {
 
 constexpr int kC = 64;
 constexpr int kThreads = 256;
-// The per-chunk adjoint runs 512 threads (two waves per SIMD): it is bound by
-// latency at one workgroup per CU (its LDS), so the second wave per SIMD hides it.
-constexpr int kChunkThreads = 512;
+// The per-chunk adjoint runs one workgroup per CU (its LDS) and is bound by
+// latency: a wave per (row tile, two column tiles), so d = 128 has four waves
+// per SIMD, each with half the gradients' partial sums of a two-wave form.
+template <int D>
+struct ChunkThreads {
+  static constexpr int value = (D == 128) ? 1024 : 512;
+};
 // Scan workgroups: one per (chain, 32-column slice).  The scans are bound by
 // the latency of their serial chunk steps (operand splits into LDS, three
 // barriers and two short MFMA chains per step), so d = 128 runs 16 waves (four
@@ -72,14 +77,17 @@ constexpr int kScanThreads = 512;   // threads of the 64-column transposed tiles
 // the two halves of the workgroup).
 constexpr int kPrepThreads = 512;
 
-__device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
+// The value, unknown to the compiler from here on (it recomputes what was
+// derived from it instead of keeping the derived values in registers).
+__device__ __forceinline__ int fresh_tid() {   // threadIdx.x, likewise
+  int x = threadIdx.x;
+  asm volatile("" : "+v"(x));
+  return x;
+}
+__device__ __forceinline__ void opaque(int& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void opaque(float& x) { asm volatile("" : "+v"(x)); }
 
-template <int D>
-struct BwdDims {
-  static constexpr int P = D + 1;     // LDS pitch of [rows][D] arrays
-  static constexpr int PC = kC + 1;   // LDS pitch of [rows][64] arrays
-  static constexpr int NJ = D / 16;   // columns per thread of a [64][D] product
-};
+__device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
@@ -179,7 +187,7 @@ struct Tile {
   __device__ __forceinline__ void fetch(const void* src, int src_ld, int col0) {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = threadIdx.x + p * NTH;
+      const int e = fresh_tid() + p * NTH;
       if (N % NTH == 0 || e < N) {
         const int row = e / V, c4 = e - row * V;
         const int64_t i = static_cast<int64_t>(row) * src_ld + col0 + 4 * c4;
@@ -193,7 +201,7 @@ struct Tile {
   __device__ __forceinline__ void put(float* dst) const {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = threadIdx.x + p * NTH;
+      const int e = fresh_tid() + p * NTH;
       if (N % NTH == 0 || e < N) {
         const int row = e / V, c4 = e - row * V;
         const float4 x = get(p);
@@ -264,14 +272,14 @@ __device__ __forceinline__ void lds_load_in(float* dst, const void* src, int64_t
   float tmp[PER][8];
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
-    const int e = threadIdx.x + p * NTH;
+    const int e = fresh_tid() + p * NTH;
     const int r = e / V, c8 = e - r * V;
     const bool ok = (N % NTH == 0 || e < N) && r < len;
     ld8<DT>(src, ((row0 + (ok ? r : 0)) * H + h) * D + col0 + 8 * (ok ? c8 : 0), tmp[p]);
   }
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
-    const int e = threadIdx.x + p * NTH;
+    const int e = fresh_tid() + p * NTH;
     if (N % NTH == 0 || e < N) {
       const int r = e / V, c8 = e - r * V;
       const bool ok = r < len;
@@ -293,7 +301,7 @@ struct InTile {
   __device__ __forceinline__ void fetch(const void* src, int64_t row0, int len, int H, int h, int col0) {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = threadIdx.x + p * NTH;
+      const int e = fresh_tid() + p * NTH;
       const int r = e / V, c8 = e - r * V;
       const bool ok = (N % NTH == 0 || e < N) && r < len;
       const int64_t i = ((row0 + (ok ? r : 0)) * H + h) * D + col0 + 8 * c8;
@@ -311,11 +319,30 @@ struct InTile {
       }
     }
   }
+  // the elements as they are, rows of PITCH elements
+  template <int PITCH>
+  __device__ __forceinline__ void put_raw(typename InT<DT>::t* dst) const {
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int e = fresh_tid() + p * NTH;
+      if (N % NTH == 0 || e < N) {
+        const int r = e / V, c8 = e - r * V;
+        u32x4* o = reinterpret_cast<u32x4*>(dst + r * PITCH + 8 * c8);
+        auto vec = [](const uint4& x) { return u32x4{x.x, x.y, x.z, x.w}; };
+        if constexpr (DT == 0) {
+          o[0] = vec(w[2 * p]);
+          o[1] = vec(w[2 * p + 1]);
+        } else {
+          o[0] = vec(w[p]);
+        }
+      }
+    }
+  }
   template <int PITCH>
   __device__ __forceinline__ void put(float* dst, float mul) const {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = threadIdx.x + p * NTH;
+      const int e = fresh_tid() + p * NTH;
       if (N % NTH == 0 || e < N) {
         const int r = e / V, c8 = e - r * V;
         float x[8];
@@ -699,7 +726,7 @@ __device__ __forceinline__ void put_hl(const Tile<ROWS, COLS, NTH, ET>& tl, __bf
   typedef Tile<ROWS, COLS, NTH, ET> TT;
 #pragma unroll
   for (int p = 0; p < TT::PER; ++p) {
-    const int e = threadIdx.x + p * NTH;
+    const int e = fresh_tid() + p * NTH;
     if (TT::N % NTH == 0 || e < TT::N) {
       const int row = e / TT::V, c4 = e - row * TT::V;
       const float4 x = tl.get(p);
@@ -716,7 +743,7 @@ __device__ __forceinline__ void put_hl(const InTile<DT, D, COLS, NTH>& tl, __bf1
   typedef InTile<DT, D, COLS, NTH> TT;
 #pragma unroll
   for (int p = 0; p < TT::PER; ++p) {
-    const int e = threadIdx.x + p * NTH;
+    const int e = fresh_tid() + p * NTH;
     if (TT::N % NTH == 0 || e < TT::N) {
       const int r = e / TT::V, c8 = e - r * TT::V;
       float x[8];
@@ -753,37 +780,37 @@ struct TTile {
   typedef typename WsPiece<ET>::t Piece;
   Piece r[PER][2];
   __device__ __forceinline__ void fetch(const void* src, int src_ld, int col0) {
+    const int tf = fresh_tid(), rp = tf & 31, cg = tf >> 5;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) fetch_block(src, src_ld, col0, j);
+    for (int j = 0; j < PER; ++j)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const int64_t i = static_cast<int64_t>(2 * rp + y) * src_ld + col0 + 4 * (cg + G * j);
+        if constexpr (ET == 0) r[j][y] = *reinterpret_cast<const float4*>(static_cast<const float*>(src) + i);
+        else r[j][y] = *reinterpret_cast<const uint2*>(static_cast<const u16*>(src) + i);
+      }
   }
-  // column block j alone: columns col0 + 4 (cg + G j) .. + 3 of the row pair
-  __device__ __forceinline__ void fetch_block(const void* src, int src_ld, int col0, int j) {
-    const int rp = threadIdx.x & 31, cg = threadIdx.x >> 5;
+  // columns HW hp .. HW hp + HW - 1 row-major into hi / lo planes of pitch PB
+  // (a [rows][HW] pass of a product over the columns; PER == 1)
+  template <int PB, int HW>
+  __device__ __forceinline__ void put_rows_hl(int hp, __bf16* h, __bf16* l) const {
+    static_assert(PER == 1 && HW % 4 == 0, "one column group per thread");
+    const int tf = fresh_tid(), rp = tf & 31, cg = tf >> 5;
+    if (cg / (HW / 4) != hp) return;
+    const int c = 4 * (cg - hp * (HW / 4));
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
-      const int64_t i = static_cast<int64_t>(2 * rp + y) * src_ld + col0 + 4 * (cg + G * j);
-      if constexpr (ET == 0) r[j][y] = *reinterpret_cast<const float4*>(static_cast<const float*>(src) + i);
-      else r[j][y] = *reinterpret_cast<const uint2*>(static_cast<const u16*>(src) + i);
-    }
-  }
-  // block j row-major into hi / lo planes of pitch PB, block-local columns
-  // 4 cg .. 4 cg + 3 (a [rows][4 G] pass of a product over the columns)
-  template <int PB>
-  __device__ __forceinline__ void put_rows_hl(int j, __bf16* h, __bf16* l) const {
-    const int rp = threadIdx.x & 31, cg = threadIdx.x >> 5;
-#pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const float4 x = ws_unpack<ET>(r[j][y]);
+      const float4 x = ws_unpack<ET>(r[0][y]);
       uint2 hh, ll;
       split2_bf16(x.x, x.y, hh.x, ll.x);
       split2_bf16(x.z, x.w, hh.y, ll.y);
-      *reinterpret_cast<uint2*>(&h[(2 * rp + y) * PB + 4 * cg]) = hh;
-      *reinterpret_cast<uint2*>(&l[(2 * rp + y) * PB + 4 * cg]) = ll;
+      *reinterpret_cast<uint2*>(&h[(2 * rp + y) * PB + c]) = hh;
+      *reinterpret_cast<uint2*>(&l[(2 * rp + y) * PB + c]) = ll;
     }
   }
   template <int PB>
   __device__ __forceinline__ void put_hl(__bf16* h, __bf16* l) const {
-    const int rp = threadIdx.x & 31, cg = threadIdx.x >> 5;
+    const int tf = fresh_tid(), rp = tf & 31, cg = tf >> 5;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int c4 = 4 * (cg + G * j);
@@ -1846,13 +1873,13 @@ struct WnTile {
   __device__ __forceinline__ void fetch(const void* src) {
 #pragma unroll
     for (int p = 0; p < PER; ++p)
-      w[p] = *reinterpret_cast<const uint4*>(static_cast<const u16*>(src) + (threadIdx.x + p * NTH) * 8);
+      w[p] = *reinterpret_cast<const uint4*>(static_cast<const u16*>(src) + (fresh_tid() + p * NTH) * 8);
   }
   template <int PB>
   __device__ __forceinline__ void put_hl(__bf16* h, __bf16* l) const {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = threadIdx.x + p * NTH, f = e >> 6, ln = e & 63;
+      const int e = fresh_tid() + p * NTH, f = e >> 6, ln = e & 63;
       const int ct = f / (D / 32), j = f - ct * (D / 32);
       const int row = 16 * ct + (ln & 15), ch0 = 32 * j + 4 * (ln >> 4);
 #pragma unroll
@@ -1868,6 +1895,35 @@ struct WnTile {
   }
 };
 
+// Four consecutive rows of one column of an LDS tile of element type DT: fp32
+// in four registers, 16-bit elements packed in two.
+template <int DT>
+struct Col4 {
+  typedef typename InT<DT>::t E;
+  uint32_t w[DT == 0 ? 4 : 2];
+  __device__ __forceinline__ void load(const E* p, int pitch) {
+    if constexpr (DT == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(p[i * pitch]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) w[i] = p[2 * i * pitch] | (static_cast<uint32_t>(p[(2 * i + 1) * pitch]) << 16);
+    }
+  }
+  __device__ __forceinline__ float get(int i) const {
+    if constexpr (DT == 0) return __uint_as_float(w[i]);
+    else {
+      const uint32_t x = w[i >> 1];
+      const u16 b = static_cast<u16>((i & 1) ? (x >> 16) : (x & 0xFFFFu));
+      return (DT == 1) ? bf16_to_f32(b) : f16bits_to_f32(b);
+    }
+  }
+  __device__ __forceinline__ void opaque_() {
+#pragma unroll
+    for (int i = 0; i < (DT == 0 ? 4 : 2); ++i) asm volatile("" : "+v"(w[i]));
+  }
+};
+
 // ---------------------------------------------------------------------------
 // per chunk-head adjoint: one 512-thread workgroup per chunk-head, four
 // phases separated by workgroup barriers, every phase in the same thread
@@ -1880,51 +1936,37 @@ struct WnTile {
 //   3  dL = -(Yw W^T + Yu U^T)
 //   4  the score adjoints of the wave's row tile (row side) and key tile
 //      (column side); dg's reverse cumsum; dq, dk, dg, dbeta stored
+// Bound by the phases' latencies at one workgroup per CU (LDS) beside the 480
+// KiB it moves per chunk-head (d = 128, 16-bit inputs: 380 us of a 4 096
+// chunk-head call at the copy rate).  d = 128, 4 096 chunk-heads, 16-bit
+// inputs: 658 us with two waves per SIMD, a decay factor formed per operand
+// and tile pair and the operands read element by element from LDS in phase 4,
+// and two-byte column reads of q, k, v, g from memory; 561 us now.
 // ---------------------------------------------------------------------------
 template <int D, int DTQ, int DTG, int DO>
-__global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a) {
-  typedef BwdDims<D> BD;
-  constexpr int P = BD::P;
-  constexpr int PC = kC + 4;          // [64][64] pitch: 16-byte aligned rows, row fragments conflict-free
-  constexpr int NTH = kChunkThreads;
+__global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(BwdArgs a) {
+  constexpr int NTH = ChunkThreads<D>::value;
+  constexpr int NG = NTH / 256;      // waves per row tile (groups of column tiles)
   constexpr int HW = 64;             // value columns per pass of phase 1
   constexpr int NH = D / HW;
   // LDS of the largest phase: phase 1's bf16 planes, phase 2's planes plus
   // the dk, dG hand-off and the row tiles' sums of g, phase 3's planes,
-  // phase 4's dL, dAqk [64][PC] and q, k, G [64][P] plus beta
+  // phase 4's score cotangent and key / query fragments
   constexpr int ACC0 = (2 * kC + 4 * D) * (kC + 8) / 2;   // floats of phase 2's bf16 planes
-  constexpr int P4 = 2 * kC * PC + 3 * kC * P + kC + 17 * D + 40 * kC;   // floats of phase 4
-  // [4][D] row tiles' sums of g, from phase 1's epilogue to phase 4: past
-  // every buffer of phases 2 to 4
-  constexpr int GS0 = cmax(ACC0 + 2 * kC * D, P4);
-  constexpr int SMEM_FLOATS = cmax(cmax((6 * kC + 4 * D) * (HW + 8) / 2, GS0 + 4 * D), 8 * kC * (D + 8) / 2);
+  constexpr int GS0 = ACC0 + 2 * kC * D;                  // [4][D] row tiles' sums of g (phase 1's epilogue)
+  constexpr int NCT = D / 16;        // column tiles
+  constexpr int NPT = 10;            // 16 x 16 tiles (row tile R >= key tile s), at R (R + 1) / 2 + s
+  constexpr int FG = 68, FT = 4 * FG;   // row fragments: floats per lane group (padded) and per tile
+  constexpr int P4 = 2 * NPT * (FT + 256) + 3 * kC * D + 16 * D + D + NG * kC;   // floats of phase 4
+  constexpr int SMEM_FLOATS = cmax(cmax(cmax((6 * kC + 4 * D) * (HW + 8) / 2, GS0 + 4 * D), 8 * kC * (D + 8) / 2), P4);
   __shared__ __attribute__((aligned(16))) float sm[SMEM_FLOATS];
-  const int t = threadIdx.x;
   const int H = a.H;
   const int u = blockIdx.x / H, h = blockIdx.x - u * H;
   const ChunkRows cr = chunk_rows(a, u);
   const int64_t ch = static_cast<int64_t>(u) * H + h;
   auto in_idx = [&](int c, int d) { return ((cr.row0 + c) * H + h) * D + d; };
-  // loads from pad rows (c >= len) read row 0 and are zeroed where used, so
-  // no load sits inside a branch (whose end would wait for it)
-  auto ld_q = [&](int c, int d) {
-    const float x = ld1<DTQ>(a.q, in_idx(c < cr.len ? c : 0, d));
-    return (c < cr.len) ? x * a.scale : 0.f;
-  };
-  auto ld_k = [&](int c, int d) {
-    const float x = ld1<DTQ>(a.k, in_idx(c < cr.len ? c : 0, d));
-    return (c < cr.len) ? x : 0.f;
-  };
-  auto ld_v = [&](int c, int d) {
-    const float x = ld1<DTQ>(a.v, in_idx(c < cr.len ? c : 0, d));
-    return (c < cr.len) ? x : 0.f;
-  };
-  auto ld_b = [&](int c) {
-    const float x = ld1<DTG>(a.beta, (cr.row0 + (c < cr.len ? c : 0)) * H + h);
-    return (c < cr.len) ? x : 0.f;
-  };
-  // Every phase works in one mapping: wave wv owns row tile mt = wv / 2 and
-  // the NDT column tiles dt = (wv % 2) NDT + q of every [64][D] array (lane
+  // Every phase works in one mapping: wave wv owns row tile mt = wv / NG and
+  // the NDT column tiles dt = (wv % NG) NDT + q of every [64][D] array (lane
   // (r, gq) holds rows 16 mt + 4 gq + i, column 16 dt + r), so the gradients
   // of q, k and G accumulate in registers from phase 1 to phase 4 and each
   // is stored once.  Phases 1-3 run on the matrix cores as bf16 hi / lo
@@ -1933,56 +1975,26 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
   float* const gq_ = a.dq;
   float* const gk_ = a.dk;
   float* const gG_ = a.dg;
-  float pq[D / 32][4], pk[D / 32][4], pG[D / 32][4];   // partial dq, dk, dG at this thread's positions
-  constexpr int NDT = D / 32;          // column tiles per wave of a [64][D] product
-  const int wv = t >> 6, l = t & 63, r16 = l & 15, gq = l >> 4;
-  const int mt = wv >> 1, dg_ = wv & 1;
-  const int mts = __builtin_amdgcn_readfirstlane(mt);   // mt as a wave-uniform (scalar) value
+  constexpr int NDT = NCT / NG;        // column tiles per wave of a [64][D] product
+  float pq[NDT][4], pk[NDT][4], pG[NDT][4];   // partial dq, dk, dG at this thread's positions
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform, as mt and dg_
+  const int mt = wv / NG, dg_ = wv % NG;
+  // thread and lane indices are taken afresh in each phase (fresh_tid), so
+  // the addresses of one phase do not occupy registers in the others
 
   float dbrD[4], dzp[NDT];             // dbeta partials (rows 16 mt + 4 gq + i), dz partials
 #pragma unroll
   for (int i = 0; i < 4; ++i) dbrD[i] = 0.f;
 #pragma unroll
   for (int q = 0; q < NDT; ++q) dzp[q] = 0.f;
-  float dgc = 0.f;   // thread t < D: sum_n S[t][n] dS'[t][n]
   // G, k and q (times the scale; zero on pad rows) at this thread's positions
   // (rows 16 mt + 4 gq + i, columns 16 (dg_ NDT + q) + r16), read once in
   // phase 1's epilogue (G formed there from g): phase 2 shares the positions
   // and phase 4 takes its LDS copies of G, k, q from them
   // (q, k held as loaded: 16-bit inputs packed two to a register)
-  typedef typename std::conditional<DTQ == 0, f4, uint2>::type H4;
-  auto hload = [&](const void* src, int d) {   // rows 16 mt + 4 gq + i of column d (pad rows read row 0)
-    H4 hv;
-    if constexpr (DTQ == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = 16 * mt + 4 * gq + i;
-        hv[i] = static_cast<const float*>(src)[in_idx(c < cr.len ? c : 0, d)];
-      }
-    } else {
-      uint32_t b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = 16 * mt + 4 * gq + i;
-        b[i] = static_cast<const u16*>(src)[in_idx(c < cr.len ? c : 0, d)];
-      }
-      hv.x = b[0] | (b[1] << 16);
-      hv.y = b[2] | (b[3] << 16);
-    }
-    return hv;
-  };
-  auto hget = [&](const H4& hv, int i) {   // element i, zero on pad rows
-    float x;
-    if constexpr (DTQ == 0) x = hv[i];
-    else {
-      const uint32_t w = (i < 2) ? hv.x : hv.y;
-      const u16 bits = static_cast<u16>((i & 1) ? (w >> 16) : (w & 0xFFFFu));
-      x = (DTQ == 1) ? bf16_to_f32(bits) : f16bits_to_f32(bits);
-    }
-    return (16 * mt + 4 * gq + i < cr.len) ? x : 0.f;
-  };
   float gH[NDT][4], gLast[NDT];
-  H4 kH[NDT], qH[NDT];
+  float bH[4];                         // beta of rows 16 mt + 4 gq + i
+  Col4<DTQ> kH[NDT], qH[NDT], vH[NDT];
   constexpr int EF = BwdWs<DTQ != 0>::F;    // S_in, T, W
 
   // Phase 1's dk and dG terms reach phase 2 (same thread, same positions)
@@ -1997,20 +2009,28 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
   // lo hi, about 2^-16 of each product dropped); dW accumulates +dv~ S^T and
   // is negated where phase 2 takes it.
   f4 dW[NDT];
-  // dAqk = tril(do v~^T), two 16 x 16 tiles per wave (row tile mt, key tiles
-  // 2 (wv % 2) + q), from phase 1's do and v~ planes: K = the value channels
+  // dAqk = tril(do v~^T), NKT 16 x 16 tiles per wave (row tile mt, key tiles
+  // kt0 + q), from phase 1's do and v~ planes: K = the value channels
   // of each pass; key tiles above the row tile are skipped (masked in phase 3)
-  f4 dAa[2];
-  const int kt0 = 2 * (wv & 1);
-  const bool live0 = kt0 <= mts, live1 = kt0 + 1 <= mts;   // wave-uniform
+  constexpr int NKT = 4 / NG;
+  f4 dAa[NKT];
+  const int kt0 = __builtin_amdgcn_readfirstlane(NKT * dg_);
 #pragma unroll
-  for (int q = 0; q < 2; ++q) dAa[q] = f4{0.f, 0.f, 0.f, 0.f};
-  TTile<kC, NTH, EF> tT;     // phase 2's T, loaded during phase 1's last pass
-  // dv~ in row pairs: column block hp is phase 1's pass hp operand, and the
-  // whole tile phase 2's dv~^T (one read of dv~ serves both)
+  for (int q = 0; q < NKT; ++q) dAa[q] = f4{0.f, 0.f, 0.f, 0.f};
+  constexpr int TTH = 512;   // threads that hold T for its transposed store
+  TTile<kC, TTH, EF> tT;     // phase 2's T, loaded during phase 1's last pass
+  // dv~ in row pairs: phase 1's passes take their columns of it, phase 2 the
+  // whole tile as dv~^T (one read of dv~ serves both)
   TTile<D, NTH> tY;
-  static_assert(TTile<D, NTH>::PER == D / 64 && TTile<D, NTH>::G * 4 == 64, "one column block per pass");
+  static_assert(TTile<D, NTH>::PER == 1, "one block of columns");
+  // sum_n S[d][n] dS'[d][n] of the rows d this thread loads (a share of the
+  // columns each; 16 neighbouring threads share a row)
+  constexpr int NDG = Tile<D, HW, NTH>::PER;
+  float dgc[NDG];
+#pragma unroll
+  for (int p = 0; p < NDG; ++p) dgc[p] = 0.f;
   {
+    const int t = fresh_tid(), l = t & 63, r16 = l & 15, gq = l >> 4;
     f4 dY[NDT], dgq[NDT];
 #pragma unroll
     for (int q = 0; q < NDT; ++q)
@@ -2036,22 +2056,39 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
     auto fetch_pass = [&](int hp) {
       const int n0 = HW * hp;
       pV.fetch(a.VT + ch * kC * D, D, n0);
-      tY.fetch_block(a.DVT + ch * kC * D, D, 0, hp);
+      if (hp == 0) tY.fetch(a.DVT + ch * kC * D, D, 0);
       pS.fetch(ws_at<EF>(a.SI, ch * D * D), D, n0);
       pDS.fetch(a.DS + ch * D * D, D, n0);
       pDo.fetch(a.dout, cr.row0, cr.len, H, h, n0);
+    };
+    InTile<DTG, D, D, NTH> ig;
+    InTile<DTQ, D, D, NTH> iq, ik, iv;
+    auto fetch_in = [&]() {
+      ig.fetch(a.g, cr.row0, cr.len, H, h, 0);
+      iq.fetch(a.q, cr.row0, cr.len, H, h, 0);
+      ik.fetch(a.k, cr.row0, cr.len, H, h, 0);
+      iv.fetch(a.v, cr.row0, cr.len, H, h, 0);
     };
     fetch_pass(0);
 #pragma unroll
     for (int hp = 0; hp < NH; ++hp) {
       put_hl<PB>(pV, sVh, sVl);
-      tY.template put_rows_hl<PB>(hp, sUh, sUl);
+      tY.template put_rows_hl<PB, HW>(hp, sUh, sUl);
       put_hl<PB>(pS, sSh, sSl);
       put_hl<PB>(pDS, sDh, sDl);
       put_hl<PB>(pDo, sOh, sOl);
+#pragma unroll
+      for (int p = 0; p < NDG; ++p) {
+        const float4 x = pS.get(p), y = pDS.get(p);
+        dgc[p] += (x.x * y.x + x.y * y.y) + (x.z * y.z + x.w * y.w);
+        opaque(dgc[p]);
+      }
       __syncthreads();
       if (hp + 1 < NH) fetch_pass(hp + 1);
-      else tT.fetch(ws_at<EF>(a.TM, ch * kC * kC), kC, 0);   // phase 2's T
+      else {   // the epilogue's g, q, k, v (fp32 inputs: after the products, for registers) and phase 2's T
+        if constexpr (DTQ != 0) fetch_in();
+        if (t < TTH) tT.fetch(ws_at<EF>(a.TM, ch * kC * kC), kC, 0);
+      }
 #pragma unroll
       for (int kb = 0; kb < HW / 32; ++kb) {
         const int ka = (16 * mt + r16) * PB + 32 * kb + 8 * gq;
@@ -2067,46 +2104,55 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
           dgq[q] = mma3_bf16(dgq[q], oh, ol, sh, sl);
           dW[q] = mma3_bf16(dW[q], uh, ul, sh, sl);
         }
-        if (live0) {
 #pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            if (q == 1 && !live1) continue;
-            const int kv = (16 * (kt0 + q) + r16) * PB + 32 * kb + 8 * gq;
-            dAa[q] = mma3_bf16(dAa[q], oh, ol, *reinterpret_cast<const b8*>(&sVh[kv]),
-                               *reinterpret_cast<const b8*>(&sVl[kv]));
-          }
-        }
-      }
-      if (t < D) {
-#pragma unroll 2
-        for (int n8 = 0; n8 < HW; n8 += 8) {
-          const b8 sh = *reinterpret_cast<const b8*>(&sSh[t * PB + n8]), sl = *reinterpret_cast<const b8*>(&sSl[t * PB + n8]);
-          const b8 dh = *reinterpret_cast<const b8*>(&sDh[t * PB + n8]), dl = *reinterpret_cast<const b8*>(&sDl[t * PB + n8]);
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            dgc = fmaf(static_cast<float>(sh[e]) + static_cast<float>(sl[e]),
-                       static_cast<float>(dh[e]) + static_cast<float>(dl[e]), dgc);
+        for (int q = 0; q < NKT; ++q) {
+          if (kt0 + q > mt) continue;
+          const int kv = (16 * (kt0 + q) + r16) * PB + 32 * kb + 8 * gq;
+          dAa[q] = mma3_bf16(dAa[q], oh, ol, *reinterpret_cast<const b8*>(&sVh[kv]),
+                             *reinterpret_cast<const b8*>(&sVl[kv]));
         }
       }
       __syncthreads();
     }
+    // g, q, k and v of the chunk-head through LDS (over phase 1's planes) to
+    // this thread's positions: whole rows are read from memory and the lanes'
+    // column reads fall on distinct banks (pad rows are zero)
+    constexpr int PG = D + (DTG == 0 ? 4 : 8), PQ = D + (DTQ == 0 ? 4 : 8);
+    typedef typename InT<DTQ>::t EQ;
+    typedef typename InT<DTG>::t EG;
+    EG* const sGr = reinterpret_cast<EG*>(sm);
+    EQ* const sQr = reinterpret_cast<EQ*>(sm + (sizeof(EG) * kC * PG) / 4);
+    EQ* const sKr = sQr + kC * PQ;
+    EQ* const sVr = sKr + kC * PQ;
+    static_assert(sizeof(EG) * kC * PG + 3 * sizeof(EQ) * kC * PQ <= 4 * GS0, "g, q, k, v end below the sums of g");
+    if constexpr (DTQ == 0) fetch_in();
+    ig.template put_raw<PG>(sGr);
+    iq.template put_raw<PQ>(sQr);
+    ik.template put_raw<PQ>(sKr);
+    iv.template put_raw<PQ>(sVr);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = 16 * mt + 4 * gq + i;
+      const float x = ld1<DTG>(a.beta, (cr.row0 + (c < cr.len ? c : 0)) * H + h);
+      bH[i] = (c < cr.len) ? x : 0.f;
+    }
+    __syncthreads();
     // G_c = log2(e) sum_{c' <= c} g_c' at this thread's positions, from g:
     // the prefix over the lane's four rows, plus the lane groups above it in
     // the row tile (shuffles), plus the row tiles above (their sums through
-    // LDS, past phase 2's buffers).  G_{C-1} sums the four tile sums in the
-    // order the last row's prefix does, so the two agree bit for bit.
+    // LDS, past phase 2's buffers).
     float* const sGs = sm + GS0;
+    const int c0 = 16 * mt + 4 * gq;
 #pragma unroll
     for (int q = 0; q < NDT; ++q) {
       const int d = 16 * (dg_ * NDT + q) + r16;
+      Col4<DTG> gR;
+      gR.load(sGr + c0 * PG + d, PG);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = 16 * mt + 4 * gq + i;
-        const float x = ld1<DTG>(a.g, in_idx(c < cr.len ? c : 0, d));
-        gH[q][i] = (c < cr.len) ? x : 0.f;
-      }
-      qH[q] = hload(a.q, d);
-      kH[q] = hload(a.k, d);
+      for (int i = 0; i < 4; ++i) gH[q][i] = gR.get(i);
+      qH[q].load(sQr + c0 * PQ + d, PQ);
+      kH[q].load(sKr + c0 * PQ + d, PQ);
+      vH[q].load(sVr + c0 * PQ + d, PQ);
     }
 #pragma unroll
     for (int q = 0; q < NDT; ++q) {
@@ -2126,7 +2172,7 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
       float pre = 0.f, run = 0.f;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
-        if (m == mts) pre = run;
+        if (m == mt) pre = run;
         run += sGs[m * D + d];
       }
       gLast[q] = run * kLog2e;
@@ -2141,14 +2187,33 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
       for (int i = 0; i < 4; ++i) {
         const int c = 16 * mt + 4 * gq + i;
         const float gam = ex2(gH[q][i]), lam = ex2(gLast[q] - gH[q][i]);
-        const float dz = dY[q][i] * hget(kH[q], i) * lam;
+        const float dz = dY[q][i] * kH[q].get(i) * lam;
         dzp[q] += dz;
         pq[q][i] = dgq[q][i] * gam * a.scale;
         sAcc[c * D + d] = dY[q][i] * lam;
-        sAcc[(kC + c) * D + d] = dgq[q][i] * (hget(qH[q], i) * a.scale) * gam - dz;
+        sAcc[(kC + c) * D + d] = dgq[q][i] * (qH[q].get(i) * a.scale) * gam - dz;
       }
     }
   }
+  // A value carried to a later phase is formed where it is, not sunk into its
+  // use there with everything it depends on, and what each phase derives from
+  // G, q, k is not kept for the next (registers).
+  auto carry = [&](float (&x)[NDT][4]) {
+#pragma unroll
+    for (int q = 0; q < NDT; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) opaque(x[q][i]);
+  };
+  auto phase_end = [&]() {
+    carry(pq);
+    carry(gH);
+#pragma unroll
+    for (int q = 0; q < NDT; ++q) {
+      kH[q].opaque_();
+      qH[q].opaque_();
+    }
+  };
+  phase_end();
 
   // ---- phase 2: Yw = T^T dW, Yu = T^T dv~ (K = the chunk's 64 rows), as
   // bf16 hi / lo triples: T^T, (-dW)^T and dv~^T in LDS with the chunk row
@@ -2159,6 +2224,7 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
   typename std::conditional<EF == 0, Tile<kC, D, NTH>, WnTile<D, NTH>>::type tW3;
   Tile<kC, D, NTH> tU3;
   {
+    const int t = fresh_tid(), l = t & 63, r16 = l & 15, gq = l >> 4;
     constexpr int PB = kC + 8;
     static_assert((2 * kC + 4 * D) * PB / 2 <= ACC0, "phase 2 planes end below sAcc");
     __bf16* const sTh = reinterpret_cast<__bf16*>(sm);   // T^T [64][64]
@@ -2176,20 +2242,18 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
       *reinterpret_cast<uint2*>(&sXh[o]) = hh;
       *reinterpret_cast<uint2*>(&sXl[o]) = ll;
     }
-    tT.template put_hl<PB>(sTh, sTl);
+    if (t < TTH) tT.template put_hl<PB>(sTh, sTl);
     tY.template put_hl<PB>(sYh, sYl);
     __syncthreads();
-    H4 vH[NDT];   // the epilogue's v and beta, during the products
-    float bH[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) bH[i] = ld_b(16 * mt + 4 * gq + i);
-#pragma unroll
-    for (int q = 0; q < NDT; ++q) vH[q] = hload(a.v, 16 * (dg_ * NDT + q) + r16);
+    // phase 3's W and U, during the products
+    if constexpr (EF == 0) tW3.fetch(a.WM + ch * kC * D, D, 0);
+    else tW3.fetch(static_cast<const u16*>(a.FWN) + ch * kC * D);
+    tU3.fetch(a.UM + ch * kC * D, D, 0);
 #pragma unroll
     for (int q = 0; q < NDT; ++q)
 #pragma unroll
       for (int i = 0; i < 4; ++i) Yw[q][i] = Yu[q][i] = 0.f;
-    for (int kb = mts >> 1; kb < kC / 32; ++kb) {
+    for (int kb = mt >> 1; kb < kC / 32; ++kb) {
       const int ka = (16 * mt + r16) * PB + 32 * kb + 8 * gq;
       const b8 th = *reinterpret_cast<const b8*>(&sTh[ka]), tl = *reinterpret_cast<const b8*>(&sTl[ka]);
 #pragma unroll
@@ -2203,17 +2267,19 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
     }
     __syncthreads();
     // dG += Yw k beta gamma; dk += Yw gamma beta; dv = Yu beta; dbeta += Yw gamma k + Yu v
+    int cb = 16 * mt + 4 * gq;   // (addresses formed here, not held from the loads)
+    opaque(cb);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int c = 16 * mt + 4 * gq + i;
+      const int c = cb + i;
       const bool live = c < cr.len;
       const float bc = bH[i];
       float kv[NDT], vv[NDT], oG[NDT], ok[NDT];
 #pragma unroll
       for (int q = 0; q < NDT; ++q) {
         const int d = 16 * (dg_ * NDT + q) + r16;
-        kv[q] = hget(kH[q], i);
-        vv[q] = hget(vH[q], i);
+        kv[q] = kH[q].get(i);
+        vv[q] = vH[q].get(i);
         oG[q] = sAcc[(kC + c) * D + d];
         ok[q] = sAcc[c * D + d];
       }
@@ -2228,25 +2294,37 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
       }
     }
     __syncthreads();   // sAcc read before phase 3's operands overwrite it
+    carry(pk);
+    carry(pG);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) opaque(dbrD[i]);
+    phase_end();
   }
 
   // ---- phase 3: dL = strict(-(Yw W^T + Yu U^T)) [64][64] (dAqk came from
-  // phase 1), two 16 x 16 tiles per wave: row tile mt, key tiles 2 (wv % 2) + q,
+  // phase 1), NKT 16 x 16 tiles per wave: row tile mt, key tiles kt0 + q,
   // as bf16 hi / lo triples (operands row-major with the channel, the K index,
   // contiguous); key tiles above the row tile are masked to zero and skipped.
-  float* const sDL = sm;                 // phase 4's operands, written at the end of phase 3
-  float* const sDA = sDL + kC * PC;
-  // past phase 4's dL, dAqk, q, k, G, beta: [16][D] dz partials, then the
-  // per-column base of dg [D]
-  float* const sRed4 = sm + 2 * kC * PC + 3 * kC * P + kC;
-  float* const sBase = sRed4 + 16 * D;
-  // then the row partial sums of dbeta: [64][32] from phase 2 (written at the
-  // start of phase 3, past its planes), [64][8] from phase 4 (per column tile)
-  float* const sDbD = sBase + D;
-  float* const sDb4 = sDbD + kC * 32;
-  static_assert(P4 <= GS0 && GS0 + 4 * D <= SMEM_FLOATS, "phase 4 LDS, below the sums of g");
-  static_assert(8 * kC * (D + 8) / 2 <= 2 * kC * PC + 3 * kC * P + kC + 17 * D, "phase 3 planes end below sDbD");
+  // Phase 4's LDS, written at the end of phase 3.  Every fragment is 16 bytes
+  // per lane: lane (r, gq) holds K values 4 gq .. 4 gq + 3, one per K step of
+  // four v_mfma_f32_16x16x4f32 (the K order inside a tile is free as long as
+  // both operands share it).
+  float* const sFA = sm;                 // [NPT][FT]  dAqk tiles, rows as M (row r, keys 4 gq ..)
+  float* const sFL = sFA + NPT * FT;     //            dL
+  float* const sTA = sFL + NPT * FT;     // [NPT][64][4] their transposes, keys as M (key r, rows 4 gq ..)
+  float* const sTL = sTA + NPT * 256;
+  float* const sKD = sTL + NPT * 256;    // [4][NCT][64][4] k_i 2^(Ge - G_i)
+  float* const sQU = sKD + kC * D;       // q_c 2^(G_c - Ga)
+  float* const sKU = sQU + kC * D;       // beta_c k_c 2^(G_c - Ga)
+  float* const sGa = sKU + kC * D;       // [4][D] G of each row tile's first and last row
+  float* const sGe = sGa + 4 * D;
+  float* const sDz = sGe + 4 * D;        // [4][D] dz sums of each row tile
+  float* const sTile = sDz + 4 * D;      // [4][D] dG sums of each row tile
+  float* const sBase = sTile + 4 * D;    // [D] per-column base of dg
+  float* const sDb = sBase + D;          // [64][NG] dbeta's sums over each wave's columns
+  const int tm0 = mt * (mt + 1) / 2;   // tile (mt, 0)
   {
+    const int t = fresh_tid(), l = t & 63, r16 = l & 15, gq = l >> 4;
     constexpr int PB = D + 8;            // bf16 pitch: 16-byte aligned K blocks, rows 4 banks apart
     static_assert(8 * kC * PB / 2 <= SMEM_FLOATS, "phase 3 LDS");
     __bf16* const sAh = reinterpret_cast<__bf16*>(sm);   // Yw
@@ -2262,27 +2340,22 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
       acc_put_hl<PB>(Yw[q], 16 * mt, 16 * (dg_ * NDT + q), sAh, sAl);
       acc_put_hl<PB>(Yu[q], 16 * mt, 16 * (dg_ * NDT + q), sBh, sBl);
     }
-    if constexpr (EF == 0) tW3.fetch(a.WM + ch * kC * D, D, 0);
-    else tW3.fetch(static_cast<const u16*>(a.FWN) + ch * kC * D);
-    tU3.fetch(a.UM + ch * kC * D, D, 0);
     if constexpr (EF == 0) put_hl<PB>(tW3, sWh, sWl);
     else tW3.template put_hl<PB>(sWh, sWl);
     put_hl<PB>(tU3, sUh, sUl);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sDbD[(16 * mt + 4 * gq + i) * 32 + 16 * dg_ + r16] = dbrD[i];
     __syncthreads();
-    f4 dLa[2];
+    f4 dLa[NKT];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) dLa[q] = f4{0.f, 0.f, 0.f, 0.f};
-    if (live0) {
+    for (int q = 0; q < NKT; ++q) dLa[q] = f4{0.f, 0.f, 0.f, 0.f};
+    if (kt0 <= mt) {
 #pragma unroll 2
       for (int kb = 0; kb < D / 32; ++kb) {
         const int ka = (16 * mt + r16) * PB + 32 * kb + 8 * gq;
         const b8 ywh = *reinterpret_cast<const b8*>(&sAh[ka]), ywl = *reinterpret_cast<const b8*>(&sAl[ka]);
         const b8 yuh = *reinterpret_cast<const b8*>(&sBh[ka]), yul = *reinterpret_cast<const b8*>(&sBl[ka]);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          if (q == 1 && !live1) continue;
+        for (int q = 0; q < NKT; ++q) {
+          if (kt0 + q > mt) continue;
           const int kbb = (16 * (kt0 + q) + r16) * PB + 32 * kb + 8 * gq;
           dLa[q] = mma3_bf16(dLa[q], ywh, ywl, *reinterpret_cast<const b8*>(&sWh[kbb]),
                              *reinterpret_cast<const b8*>(&sWl[kbb]));
@@ -2291,214 +2364,236 @@ __global__ __launch_bounds__(kChunkThreads) void kda_bwd_chunk_kernel(BwdArgs a)
         }
       }
     }
-    __syncthreads();   // every read of the planes done before sDL, sDA overwrite them
-    // phase 4's masked operands
+    __syncthreads();   // every read of the planes done before phase 4's operands overwrite them
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < NKT; ++q) {
+      if (kt0 + q > mt) continue;
+      const int ti = tm0 + kt0 + q;
+      const bool diag = kt0 + q == mt;
+      f4 vA, vL;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int c = 16 * mt + 4 * gq + i, ii = 16 * (2 * dg_ + q) + r16;
-        sDL[c * PC + ii] = (ii < c) ? -dLa[q][i] : 0.f;
-        sDA[c * PC + ii] = (ii <= c) ? dAa[q][i] : 0.f;
+        vA[i] = (!diag || r16 <= 4 * gq + i) ? dAa[q][i] : 0.f;
+        vL[i] = (!diag || r16 < 4 * gq + i) ? -dLa[q][i] : 0.f;
+        const int o = ti * FT + (r16 >> 2) * FG + (4 * gq + i) * 4 + (r16 & 3);
+        sFA[o] = vA[i];
+        sFL[o] = vL[i];
       }
-    // dz column partials (slot 4 mt + gq) for the per-column base of dg
-#pragma unroll
-    for (int q = 0; q < NDT; ++q) sRed4[(4 * mt + gq) * D + 16 * (dg_ * NDT + q) + r16] = dzp[q];
-    __syncthreads();
+      *reinterpret_cast<f4*>(&sTA[ti * 256 + 4 * l]) = vA;
+      *reinterpret_cast<f4*>(&sTL[ti * 256 + 4 * l]) = vL;
+    }
   }
 
-  // ---- phase 4: score adjoints.  With dA = sDA, dL = sDL (masked):
+  // ---- phase 4: score adjoints.  With dA, dL masked:
   //   row side  rA[c] = sum_i dA[c][i] k_i 2^(G_c - G_i),  rK likewise with dL;
   //   col side  cS[i] = sum_c (dA[c][i] q_c + dL[c][i] beta_c k_c) 2^(G_c - G_i);
   //   dq += rA; dk += rK beta + cS; dG += rA q + rK k beta - cS k; dbeta_c += sum_d rK k_c
-  // (q carries the scale).  Off-diagonal tile pairs (row tile R > key tile s)
-  // factor the decay at the row tile's first row a, 2^(G_c - G_a) 2^(G_a - G_i),
-  // both <= 1, and run on the matrix cores: (16 x 16 block) x (k_i 2^(G_a - G_i))
-  // for the row side, (block)^T x (q_c 2^(G_c - G_a)) for the column side.
-  // Diagonal tiles are anchored the same way (their key factors >= 1, bounded
-  // by the tile's decay) unless the tile decays past 2^-kDiagAnchorLog2 in a
-  // column of the wave; those take 2^-|G_c - G_i| per element.  Wave (mt, half)
-  // forms, for each of its column tiles, the row side of row tile mt (key
-  // tiles s <= mt) and the column side of key tile mt (row tiles R >= mt), so
-  // the results land on the positions whose partial sums it holds.
-  constexpr int NCT = D / 16;
+  // (q carries the scale).  The decay of a pair in row tile R, key tile s <= R
+  // is 2^(G_c - Ga_R) 2^(Ga_R - Ge_s) 2^(Ge_s - G_i), Ga and Ge the G of a row
+  // tile's first and last row: the outer factors (<= 1) belong to one row or
+  // one key each, so they are formed once per element and shared through LDS
+  // by every tile pair, and the middle one, constant over the pair for a
+  // channel, is applied to the pair's accumulator column (it is <= 1 off the
+  // diagonal, and up to the tile's decay on it; a diagonal tile that decays by
+  // more than 2^-kDiagAnchorLog2 in one of the wave's columns takes
+  // 2^-|G_c - G_i| per element instead).  Wave (mt, half) forms, for each of
+  // its column tiles, the row side of row tile mt (key tiles s <= mt) and the
+  // column side of key tile mt (row tiles R >= mt): five tile pairs for every
+  // wave, and the results land on the positions whose partial sums it holds.
+  // The fp32 matrix cores' floor is half of it (80 v_mfma_f32_16x16x4f32 per
+  // wave at d = 128, 10 k of 21 k cycles for the SIMD's four waves); both
+  // operands are one 16-byte read for four of them.
   {
-    float* sQ = sDA + kC * PC;       // q * scale
-    float* sK = sQ + kC * P;
-    float* sG = sK + kC * P;
-    float* sB = sG + kC * P;
-#pragma unroll
-    for (int q = 0; q < NDT; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int o = (16 * mt + 4 * gq + i) * P + 16 * (dg_ * NDT + q) + r16;
-        sQ[o] = hget(qH[q], i) * a.scale;
-        sK[o] = hget(kH[q], i);
-        sG[o] = gH[q][i];
-      }
-    if (t < kC) sB[t] = ld_b(t);
-    if (t < D) {   // dg[c] = base + sum_{c' >= c} dG[c']: the G_C terms and the dz terms
-      const float* sGs = sm + GS0;   // G_{C-1} of column t, summed as in phase 1's epilogue
-      float acc = dgc * ex2((((sGs[t] + sGs[D + t]) + sGs[2 * D + t]) + sGs[3 * D + t]) * kLog2e);
-      for (int r = 0; r < 16; ++r) acc += sRed4[r * D + t];
-      sBase[t] = acc;
-    }
-    __syncthreads();
-    float* const sTile = sRed4;      // [4][D] dG column sums of each row tile (sRed4 is read above)
-    const int a0 = 16 * mt;
-    float sfx[NDT][4], abv[NDT];
+    const int t = fresh_tid(), l = t & 63, r16 = l & 15, gq = l >> 4;
+    float ga[NDT], ge[NDT];   // Ga, Ge of row tile mt
+    unsigned far = 0;         // column tiles q whose diagonal tile goes per element (wave-uniform)
 #pragma unroll
     for (int q = 0; q < NDT; ++q) {
-      const int d = 16 * (dg_ * NDT + q) + r16;
-      const float ga = sG[a0 * P + d];
-      f4 accA = {0.f, 0.f, 0.f, 0.f}, accK = {0.f, 0.f, 0.f, 0.f};
-      // row side: key tiles below the row tile
-      for (int sk = 0; sk < mts; ++sk) {
+      const int ct = dg_ * NDT + q, d = 16 * ct + r16;
+      ga[q] = __shfl(gH[q][0], r16, 64);
+      ge[q] = __shfl(gH[q][3], 48 + r16, 64);
+      if (__any(ga[q] - ge[q] > kDiagAnchorLog2)) far |= 1u << q;
+      f4 kd, qu, ku;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int i = 16 * sk + 4 * k + gq;
-          const float kb = sK[i * P + d] * ex2(ga - sG[i * P + d]);   // k_i 2^(G_a - G_i)
-          accA = mfma4(sDA[(a0 + r16) * PC + 16 * sk + 4 * k + gq], kb, accA);
-          accK = mfma4(sDL[(a0 + r16) * PC + 16 * sk + 4 * k + gq], kb, accK);
-        }
+      for (int i = 0; i < 4; ++i) {
+        const float kk = kH[q].get(i), up = ex2(gH[q][i] - ga[q]);
+        kd[i] = kk * ex2(ge[q] - gH[q][i]);
+        qu[i] = qH[q].get(i) * a.scale * up;
+        ku[i] = kk * bH[i] * up;
       }
-      // column side: row tiles above the key tile, the furthest first
-      float colS[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int R = 3; R > mts; --R) {
-        const int aR = 16 * R;
-        const float gR = sG[aR * P + d];
-        f4 cS = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int c = aR + 4 * k + gq;
-          const float fr = ex2(sG[c * P + d] - gR);   // q_c 2^(G_c - G_R), beta_c k_c 2^(G_c - G_R)
-          cS = mfma4(sDA[c * PC + a0 + r16], sQ[c * P + d] * fr, cS);
-          cS = mfma4(sDL[c * PC + a0 + r16], sK[c * P + d] * sB[c] * fr, cS);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) colS[e] += cS[e] * ex2(gR - sG[(a0 + 4 * gq + e) * P + d]);
+      const int o = ((mt * NCT + ct) * 64 + l) * 4;
+      *reinterpret_cast<f4*>(&sKD[o]) = kd;
+      *reinterpret_cast<f4*>(&sQU[o]) = qu;
+      *reinterpret_cast<f4*>(&sKU[o]) = ku;
+      float dz = dzp[q];
+      dz += __shfl_xor(dz, 16, 64);
+      dz += __shfl_xor(dz, 32, 64);
+      if (gq == 0) {
+        sGa[mt * D + d] = ga[q];
+        sGe[mt * D + d] = ge[q];
+        sDz[mt * D + d] = dz;
       }
-      float gc[4], rA[4], rK[4], cS[4];
+    }
+    __syncthreads();
+    // dg[c] = base + sum_{c' >= c} dG[c']: the G_{C-1} terms and the dz terms
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        gc[e] = sG[(a0 + 4 * gq + e) * P + d];
-        rA[e] = rK[e] = cS[e] = 0.f;
-      }
-      // The diagonal tile on the matrix cores, anchored at its first row a
-      // like the off-diagonal ones: row side (block) x (k_y 2^(G_a - G_y)),
-      // column side (block)^T x (q_c 2^(G_c - G_a)), times 2^(G_c - G_a) and
-      // 2^(G_a - G_i) afterwards.  Key factors here are >= 1, up to the
-      // tile's decay in the column; the masked cotangents zero every pair
-      // whose factor would exceed 1 overall.  A tile that decays by more
-      // than 2^-kDiagAnchorLog2 in one of the wave's columns (the factors
-      // would leave fp32 headroom for the cotangents) takes the per-element
-      // form below.
-      if (!__any(ga - sG[(a0 + 15) * P + d] > kDiagAnchorLog2)) {
-        f4 cd = {0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < NDG; ++p) {
+      float x = dgc[p];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int y = a0 + 4 * k + gq;
-          const float fr = ex2(sG[y * P + d] - ga);
-          const float kb = sK[y * P + d] * ex2(ga - sG[y * P + d]);   // k_y 2^(G_a - G_y)
-          accA = mfma4(sDA[(a0 + r16) * PC + y], kb, accA);
-          accK = mfma4(sDL[(a0 + r16) * PC + y], kb, accK);
-          cd = mfma4(sDA[y * PC + a0 + r16], sQ[y * P + d] * fr, cd);
-          cd = mfma4(sDL[y * PC + a0 + r16], sK[y * P + d] * sB[y] * fr, cd);
-        }
+      for (int off = 8; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+      const int d = (t + p * NTH) >> 4;
+      if ((t & 15) == 0)
+        sBase[d] = x * ex2(sGe[3 * D + d]) + ((sDz[d] + sDz[D + d]) + (sDz[2 * D + d] + sDz[3 * D + d]));
+    }
+    phase_end();
+    float sfx[NDT][4], abv[NDT];
+    // one column tile at a time, which keeps everything in registers
 #pragma unroll
-        for (int e = 0; e < 4; ++e) cS[e] = cd[e] * ex2(ga - gc[e]);
-      } else {
-        // With G non-increasing (g <= 0), the pair (c, a0 + y) of the row
-        // side (y <= x) decays by 2^(G_c - G_y) and the pair (a0 + y, c) of
-        // the column side (y >= x) by 2^(G_y - G_c): both are 2^-|G_c - G_y|,
-        // and the masked cotangents zero the side a given y does not belong to.
-        // Row y's G, k, q, beta are read once for the lane's four rows c.
-#pragma unroll 1
-        for (int y4 = 0; y4 < 16; y4 += 4) {
-          f4 rowA[4], rowL[4];   // dA[c][a0 + y4 .. + 3], dL likewise, for the lane's rows c
+    for (int q0 = 0; q0 < NDT; ++q0) {
+      __builtin_amdgcn_sched_barrier(0);
+      f4 rA[NDT], rK[NDT], cS[NDT];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int c = a0 + 4 * gq + e;
-            rowA[e] = *reinterpret_cast<const f4*>(&sDA[c * PC + a0 + y4]);
-            rowL[e] = *reinterpret_cast<const f4*>(&sDL[c * PC + a0 + y4]);
+      for (int q = q0; q < q0 + 1; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rA[q][i] = rK[q][i] = cS[q][i] = 0.f;
+      // row side
+      for (int s = 0; s <= mt; ++s) {
+        const f4 fa = *reinterpret_cast<const f4*>(&sFA[(tm0 + s) * FT + gq * FG + r16 * 4]);
+        const f4 fl = *reinterpret_cast<const f4*>(&sFL[(tm0 + s) * FT + gq * FG + r16 * 4]);
+#pragma unroll
+        for (int q = q0; q < q0 + 1; ++q) {
+          if (s == mt && (far >> q & 1)) continue;
+          const int ct = dg_ * NDT + q;
+          const f4 kd = *reinterpret_cast<const f4*>(&sKD[((s * NCT + ct) * 64 + l) * 4]);
+          const float m = ex2(ga[q] - sGe[s * D + 16 * ct + r16]);
+          f4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            x = mfma4(fa[k], kd[k], x);
+            y = mfma4(fl[k], kd[k], y);
           }
 #pragma unroll
-          for (int yy = 0; yy < 4; ++yy) {
-            const int y = y4 + yy;
-            const float gy = sG[(a0 + y) * P + d], ky = sK[(a0 + y) * P + d];
-            const float qy = sQ[(a0 + y) * P + d], by = sB[a0 + y];
+          for (int i = 0; i < 4; ++i) {
+            rA[q][i] = fmaf(m, x[i], rA[q][i]);
+            rK[q][i] = fmaf(m, y[i], rK[q][i]);
+          }
+        }
+      }
+      // column side
+      for (int R = mt; R < 4; ++R) {
+        const int ti = R * (R + 1) / 2 + mt;
+        const f4 ta = *reinterpret_cast<const f4*>(&sTA[ti * 256 + 4 * l]);
+        const f4 tl = *reinterpret_cast<const f4*>(&sTL[ti * 256 + 4 * l]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int c = a0 + 4 * gq + e;
-              const float ev = ex2(-fabsf(gc[e] - gy));
-              const float kr = ky * ev;
-              rA[e] = fmaf(rowA[e][yy], kr, rA[e]);
-              rK[e] = fmaf(rowL[e][yy], kr, rK[e]);
-              cS[e] = fmaf(sDA[(a0 + y) * PC + c], qy * ev, cS[e]);
-              cS[e] = fmaf(sDL[(a0 + y) * PC + c], by * kr, cS[e]);
+        for (int q = q0; q < q0 + 1; ++q) {
+          if (R == mt && (far >> q & 1)) continue;
+          const int ct = dg_ * NDT + q, o = ((R * NCT + ct) * 64 + l) * 4;
+          const f4 qu = *reinterpret_cast<const f4*>(&sQU[o]), ku = *reinterpret_cast<const f4*>(&sKU[o]);
+          const float m = ex2(sGa[R * D + 16 * ct + r16] - ge[q]);
+          f4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            x = mfma4(ta[k], qu[k], x);
+            y = mfma4(tl[k], ku[k], y);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) cS[q][i] = fmaf(m, x[i] + y[i], cS[q][i]);
+        }
+      }
+#pragma unroll
+      for (int q = q0; q < q0 + 1; ++q) {
+        const int d = 16 * (dg_ * NDT + q) + r16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float up = ex2(gH[q][i] - ga[q]);
+          rA[q][i] *= up;
+          rK[q][i] *= up;
+          cS[q][i] *= ex2(ge[q] - gH[q][i]);
+        }
+        if (far >> q & 1) {
+          // With G non-increasing (g <= 0), the pair (c, y) of the row side
+          // (y <= c) decays by 2^(G_c - G_y) and the pair (y, c) of the column
+          // side (y >= c) by 2^(G_y - G_c): both are 2^-|G_c - G_y|, and the
+          // masked cotangents zero the side a given y does not belong to.  Row
+          // y's G, k, q, beta come from the lane of its column that holds them.
+#pragma unroll
+          for (int yy = 0; yy < 4; ++yy) {
+            const float qs = qH[q].get(yy) * a.scale, kk = kH[q].get(yy);
+#pragma unroll 1
+            for (int y4 = 0; y4 < 4; ++y4) {
+              const int src = 16 * y4 + r16, y = 4 * y4 + yy;
+              const float gy = __shfl(gH[q][yy], src, 64), ky = __shfl(kk, src, 64);
+              const float qy = __shfl(qs, src, 64), by = __shfl(bH[yy], src, 64);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const int c = 4 * gq + e;
+                const float ev = ex2(-fabsf(gH[q][e] - gy)), kr = ky * ev;
+                const int of = (tm0 + mt) * FT + y4 * FG + c * 4 + yy;
+                const int ot = (tm0 + mt) * 256 + (y4 * 16 + c) * 4 + yy;
+                rA[q][e] = fmaf(sFA[of], kr, rA[q][e]);
+                rK[q][e] = fmaf(sFL[of], kr, rK[q][e]);
+                cS[q][e] = fmaf(sTA[ot], qy * ev, cS[q][e]);
+                cS[q][e] = fmaf(sTL[ot], by * kr, cS[q][e]);
+              }
             }
           }
         }
-      }
-      float gn[4], dbq[4];   // this tile's dG (zero on pad rows), dbeta terms
+        float gn[4];   // this tile's dG (zero on pad rows)
+        int cb = 16 * mt + 4 * gq;   // (addresses formed here, not held from the loads)
+        opaque(cb);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = a0 + 4 * gq + e;
-        const float kc = sK[c * P + d], qc = sQ[c * P + d], bc = sB[c];
-        const float f = ex2(gc[e] - ga);   // accA, accK: every tile pair but a per-element diagonal
-        rA[e] = fmaf(accA[e], f, rA[e]);
-        rK[e] = fmaf(accK[e], f, rK[e]);
-        if (mts < 3) cS[e] += colS[e];
-        dbq[e] = rK[e] * kc;
-        gn[e] = (c < cr.len) ? pG[q][e] + rA[e] * qc + rK[e] * kc * bc - cS[e] * kc : 0.f;
-        if (c < cr.len) {
-          const int64_t o = in_idx(c, d);
-          gq_[o] = pq[q][e] + rA[e] * a.scale;
-          gk_[o] = pk[q][e] + rK[e] * bc + cS[e];
+        for (int e = 0; e < 4; ++e) {
+          const int c = cb + e;
+          const float kc = kH[q].get(e), qc = qH[q].get(e) * a.scale, bc = bH[e];
+          dbrD[e] = fmaf(rK[q][e], kc, dbrD[e]);
+          gn[e] = (c < cr.len) ? pG[q][e] + rA[q][e] * qc + rK[q][e] * kc * bc - cS[q][e] * kc : 0.f;
+          if (c < cr.len) {
+            const int64_t o = in_idx(c, d);
+            gq_[o] = pq[q][e] + rA[q][e] * a.scale;
+            gk_[o] = pk[q][e] + rK[q][e] * bc + cS[q][e];
+          }
         }
-      }
-      // reverse cumsum down the column: within the lane's four rows, then
-      // over the row groups gq' > gq of the tile (lanes 16 gq' + r16); the
-      // tiles below come after the barrier
-      sfx[q][3] = gn[3];
-      sfx[q][2] = gn[2] + sfx[q][3];
-      sfx[q][1] = gn[1] + sfx[q][2];
-      sfx[q][0] = gn[0] + sfx[q][1];
-      const float x1 = __shfl_down(sfx[q][0], 16, 64), x2 = __shfl_down(sfx[q][0], 32, 64);
-      const float x3 = __shfl_down(sfx[q][0], 48, 64);
-      abv[q] = (gq < 3 ? x1 : 0.f) + (gq < 2 ? x2 : 0.f) + (gq < 1 ? x3 : 0.f);
-      if (gq == 0) sTile[mt * D + d] = sfx[q][0] + abv[q];   // the tile's column sum
-      // dbeta partials: sum over the 16 columns of the tile
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = dbq[e];
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (r16 == 0) sDb4[(a0 + 4 * gq + e) * 8 + dg_ * NDT + q] = v;
+        // reverse cumsum down the column: within the lane's four rows, then
+        // over the row groups gq' > gq of the tile (lanes 16 gq' + r16); the
+        // tiles below come after the barrier
+        sfx[q][3] = gn[3];
+        sfx[q][2] = gn[2] + sfx[q][3];
+        sfx[q][1] = gn[1] + sfx[q][2];
+        sfx[q][0] = gn[0] + sfx[q][1];
+        const float x1 = __shfl_down(sfx[q][0], 16, 64), x2 = __shfl_down(sfx[q][0], 32, 64);
+        const float x3 = __shfl_down(sfx[q][0], 48, 64);
+        abv[q] = (gq < 3 ? x1 : 0.f) + (gq < 2 ? x2 : 0.f) + (gq < 1 ? x3 : 0.f);
+        if (gq == 0) sTile[mt * D + d] = sfx[q][0] + abv[q];   // the tile's column sum
       }
     }
-    __syncthreads();   // phase 4's LDS reads done; every tile's column sums written
+    // dbeta: phase 2's and this phase's terms, summed over the wave's columns
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float v = dbrD[e];
+#pragma unroll
+      for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (r16 == 0) sDb[(16 * mt + 4 * gq + e) * NG + dg_] = v;
+    }
+    __syncthreads();   // every tile's column sums and dbeta's row sums written
 #pragma unroll
     for (int q = 0; q < NDT; ++q) {
       const int d = 16 * (dg_ * NDT + q) + r16;
       float carry = 0.f;   // the tiles below, the furthest first
-      for (int R = 3; R > mts; --R) carry += sTile[R * D + d];
+      for (int R = 3; R > mt; --R) carry += sTile[R * D + d];
       const float base = sBase[d] + carry + abv[q];
+      int cb = 16 * mt + 4 * gq;
+      opaque(cb);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int c = a0 + 4 * gq + e;
+        const int c = cb + e;
         if (c < cr.len) gG_[in_idx(c, d)] = base + sfx[q][e];
       }
     }
-  }
-
-  // ---- outputs: dbeta (its row partial sums in LDS before phase 4's last barrier)
-  {
     if (t < kC && t < cr.len) {
-      float acc = 0.f;
-      for (int j = 0; j < NCT; ++j) acc += sDb4[t * 8 + j];
-      for (int j = 0; j < 32; ++j) acc += sDbD[t * 32 + j];
-      a.dbeta[(cr.row0 + t) * H + h] = acc;
+      float x = sDb[t * NG];
+#pragma unroll
+      for (int j = 1; j < NG; ++j) x += sDb[t * NG + j];
+      a.dbeta[(cr.row0 + t) * H + h] = x;
     }
   }
 }
@@ -2523,7 +2618,7 @@ hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((kda_bwd_rscan_kernel<D, DO, false>), dim3(scan_grid), dim3(ScanThreads<D>::value), 0, s, a);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((kda_bwd_chunk_kernel<D, DTQ, DTG, DO>), dim3(chunk_heads), dim3(kChunkThreads), 0, s, a);
+  hipLaunchKernelGGL((kda_bwd_chunk_kernel<D, DTQ, DTG, DO>), dim3(chunk_heads), dim3(ChunkThreads<D>::value), 0, s, a);
   return hipGetLastError();
 }
 
