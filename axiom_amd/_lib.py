@@ -75,6 +75,16 @@ _SIGNATURES = {
     "kda_abi_version": (_i, []),
 }
 
+# Entry points of this binding's own, outside the C ABI of the header: the two
+# backward calls whose outputs may be rounded to the primals' 16-bit types by
+# the kernels that form them (axiom_amd/csrc/kda_internal.h)
+_PRIVATE = {
+    "axiom_chunk_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                             _vp, _vp, _vp, _vp, _vp, _vp,
+                             _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _i, _vp, _sz]),
+    "axiom_prologue_bwd": (_i, [_vp] * 22 + [_i, _i, _i, _i, _i, _i, _i, _vp, _sz]),
+}
+
 _lib = None
 
 
@@ -93,7 +103,7 @@ def lib() -> ctypes.CDLL:
                 f"axiom_amd: {LIB_PATH.name} is not built (run `python -m axiom_amd.build`); "
                 "the KDA path has no fallback implementation")
         L = ctypes.CDLL(str(LIB_PATH))
-        for name, (res, args) in _SIGNATURES.items():
+        for name, (res, args) in {**_SIGNATURES, **_PRIVATE}.items():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args

@@ -605,6 +605,26 @@ BwdLayout bwd_layout(int B, int T, int H, int d) {
   return L;
 }
 
+void bwd_workspace(kda::BwdArgs& a, const BwdLayout& L, unsigned char* ws) {
+  a.QG = reinterpret_cast<float*>(ws + L.QG);
+  a.KL = reinterpret_cast<float*>(ws + L.KL);
+  a.GCV = reinterpret_cast<float*>(ws + L.GCV);
+  a.AQ = reinterpret_cast<float*>(ws + L.AQ);
+  a.TM = reinterpret_cast<float*>(ws + L.TM);
+  a.WM = reinterpret_cast<float*>(ws + L.WM);
+  a.UM = reinterpret_cast<float*>(ws + L.UM);
+  a.SI = reinterpret_cast<float*>(ws + L.SI);
+  a.VT = reinterpret_cast<float*>(ws + L.VT);
+  a.DS = reinterpret_cast<float*>(ws + L.DS);
+  a.DVT = reinterpret_cast<float*>(ws + L.DVT);
+  a.FL = ws + L.FL;
+  a.FA = ws + L.FA;
+  a.FQ = ws + L.FQ;
+  a.FW = ws + L.FW;
+  a.FWN = ws + L.FWN;
+  a.FLT = ws + L.FLT;
+}
+
 int ut_check(const void* a, const void* b, const void* x, int H, int C, int N, int dtype) {
   if (!a || !b || !x) return fail(KDA_ERR_INVALID_ARGUMENT, "null pointer");
   if (H < 1 || N < 1) return fail(KDA_ERR_INVALID_ARGUMENT, "H=%d, N=%d must be >= 1", H, N);
@@ -865,6 +885,16 @@ int kda_chunk_bwd(hipStream_t stream, const void* q, const void* k, const void* 
                   float* dq, float* dk, float* dv, float* dg, float* dbeta, float* dh0,
                   int B, int T, int H, int dk_dim, int dv_dim, int chunk, float scale,
                   int in_dtype, int dout_dtype, void* workspace, size_t workspace_bytes) {
+  return axiom_chunk_bwd(stream, q, k, v, g, beta, h0, dout, dht, dq, dk, dv, dg, dbeta, dh0, B, T, H, dk_dim, dv_dim,
+                          chunk, scale, in_dtype, dout_dtype, KDA_DTYPE_F32, KDA_DTYPE_F32, workspace, workspace_bytes);
+}
+
+int axiom_chunk_bwd(hipStream_t stream, const void* q, const void* k, const void* v, const void* g,
+                     const void* beta, const float* h0, const void* dout, const float* dht,
+                     void* dq, void* dk, void* dv, void* dg, void* dbeta, float* dh0,
+                     int B, int T, int H, int dk_dim, int dv_dim, int chunk, float scale,
+                     int in_dtype, int dout_dtype, int qkv_grad_dtype, int gate_grad_dtype,
+                     void* workspace, size_t workspace_bytes) {
   g_err[0] = 0;
   if (B < 1) return fail(KDA_ERR_INVALID_ARGUMENT, "B=%d must be >= 1", B);
   if (T < 0) return fail(KDA_ERR_INVALID_ARGUMENT, "T=%d must be >= 0", T);
@@ -879,6 +909,12 @@ int kda_chunk_bwd(hipStream_t stream, const void* q, const void* k, const void* 
     return fail(KDA_ERR_INVALID_ARGUMENT, "in_dtype=%d is not a kda_dtype_t", in_dtype);
   if (dout_dtype != KDA_DTYPE_F32 && dout_dtype != KDA_DTYPE_BF16)
     return fail(KDA_ERR_INVALID_ARGUMENT, "dout_dtype=%d: dout is F32 or BF16", dout_dtype);
+  const int qkv_dtype = in_dtype == KDA_DTYPE_BF16_F32GATES ? KDA_DTYPE_BF16 : in_dtype;
+  const int gate_dtype = in_dtype == KDA_DTYPE_BF16_F32GATES ? KDA_DTYPE_F32 : in_dtype;
+  if (qkv_grad_dtype != KDA_DTYPE_F32 && qkv_grad_dtype != qkv_dtype)
+    return fail(KDA_ERR_INVALID_ARGUMENT, "qkv_grad_dtype=%d: F32 or the dtype of q, k, v", qkv_grad_dtype);
+  if (gate_grad_dtype != KDA_DTYPE_F32 && gate_grad_dtype != gate_dtype)
+    return fail(KDA_ERR_INVALID_ARGUMENT, "gate_grad_dtype=%d: F32 or the dtype of g, beta", gate_grad_dtype);
   if (!std::isfinite(scale)) return fail(KDA_ERR_INVALID_ARGUMENT, "scale must be finite");
   const int64_t elems = static_cast<int64_t>(B) * T * H * dk_dim;
   if (elems >= (1LL << 40)) return fail(KDA_ERR_INVALID_ARGUMENT, "problem too large");
@@ -898,29 +934,14 @@ int kda_chunk_bwd(hipStream_t stream, const void* q, const void* k, const void* 
     }
     return KDA_OK;
   }
-  unsigned char* ws = static_cast<unsigned char*>(workspace);
   kda::BwdArgs a{};
   a.B = B; a.T = T; a.H = H; a.NT = static_cast<int>(NT);
   a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta;
   a.h0 = h0; a.dout = dout; a.dht = dht; a.scale = scale;
   a.dq = dq; a.dk = dk; a.dv = dv; a.dg = dg; a.dbeta = dbeta; a.dh0 = dh0;
-  a.QG = reinterpret_cast<float*>(ws + L.QG);
-  a.KL = reinterpret_cast<float*>(ws + L.KL);
-  a.GCV = reinterpret_cast<float*>(ws + L.GCV);
-  a.AQ = reinterpret_cast<float*>(ws + L.AQ);
-  a.TM = reinterpret_cast<float*>(ws + L.TM);
-  a.WM = reinterpret_cast<float*>(ws + L.WM);
-  a.UM = reinterpret_cast<float*>(ws + L.UM);
-  a.SI = reinterpret_cast<float*>(ws + L.SI);
-  a.VT = reinterpret_cast<float*>(ws + L.VT);
-  a.DS = reinterpret_cast<float*>(ws + L.DS);
-  a.DVT = reinterpret_cast<float*>(ws + L.DVT);
-  a.FL = ws + L.FL;
-  a.FA = ws + L.FA;
-  a.FQ = ws + L.FQ;
-  a.FW = ws + L.FW;
-  a.FWN = ws + L.FWN;
-  a.FLT = ws + L.FLT;
+  a.qkv_out = qkv_grad_dtype;   // F32, BF16, F16: the kernels' element types
+  a.g_out = gate_grad_dtype;
+  bwd_workspace(a, L, static_cast<unsigned char*>(workspace));
   const hipError_t e = kda::launch_bwd(a, dk_dim, in_dtype, dout_dtype, stream);
   if (e != hipSuccess) return hip_fail(e, "backward kernel launch");
   return KDA_OK;
@@ -978,6 +999,31 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   float* dbeta = reinterpret_cast<float*>(ws);
   ws += align_up(th * 4);
   const size_t rest = workspace_bytes - static_cast<size_t>(ws - static_cast<unsigned char*>(workspace));
+  // The kernels take the seam's operands as they are (log alpha and the mean
+  // of beta32 in the prep and chunk kernels, bf16 / dalpha / dbeta32 outputs
+  // from the chunk kernel) when every pointer allows their 16-byte (dq, dk,
+  // dv: 4-byte) accesses; a pass before and one after the dense backward
+  // cost 42 and 126 us at B2 T8192 H12 d128.  Other pointers keep those two
+  // passes, whose element-wise forms take any alignment.
+  const uintptr_t a16 = reinterpret_cast<uintptr_t>(alpha) | reinterpret_cast<uintptr_t>(beta32) |
+                        reinterpret_cast<uintptr_t>(dbeta32);
+  const uintptr_t a4 = reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) |
+                       reinterpret_cast<uintptr_t>(dv) | reinterpret_cast<uintptr_t>(dalpha);
+  const int64_t nt = (T + kC - 1) / kC;
+  if (T > 0 && (a16 & 15) == 0 && (a4 & 3) == 0 && static_cast<int64_t>(B) * nt * H <= 0x7FFFFFFFLL &&
+      th * dk_dim < (1ULL << 40)) {
+    kda::BwdArgs a{};
+    a.B = B; a.T = T; a.H = H; a.NT = static_cast<int>(nt);
+    a.q = q; a.k = k; a.v = v; a.g = alpha; a.beta = beta32;
+    a.h0 = S_in; a.dout = d_o; a.dht = dS; a.scale = 1.0f;
+    a.dq = dq; a.dk = dk; a.dv = dv; a.dg = dalpha; a.dbeta = dbeta32; a.dh0 = dS_in;
+    a.qkv_out = KDA_DTYPE_BF16;
+    a.g_out = KDA_DTYPE_F32;
+    bwd_workspace(a, bwd_layout(B, T, H, dk_dim), ws);
+    const hipError_t e = kda::launch_bwd(a, dk_dim, kda::kInAlphaGates, 0, stream);
+    if (e != hipSuccess) return hip_fail(e, "cc_scan backward launch");
+    return KDA_OK;
+  }
   kda::AdaptArgs aa{};
   aa.alpha = alpha; aa.beta32 = beta32; aa.g_out = g32; aa.beta_out = b32;
   aa.n_tok_heads = static_cast<int64_t>(th);
@@ -1098,18 +1144,32 @@ int kda_prologue_bwd(hipStream_t stream, const void* qp, const void* kp, const v
                      float* dqp, float* dkp, float* dvp, float* dwq, float* dwk, float* dwv,
                      float* dbq, float* dbk, float* dbv,
                      int B, int T, int H, int d, int K, int in_dtype, void* workspace, size_t workspace_bytes) {
+  return axiom_prologue_bwd(stream, qp, kp, vp, wq, wk, wv, bq_in, bk_in, bv_in, dq, dk, dv, dqp, dkp, dvp, dwq, dwk,
+                             dwv, dbq, dbk, dbv, B, T, H, d, K, in_dtype, KDA_DTYPE_F32, workspace, workspace_bytes);
+}
+
+int axiom_prologue_bwd(hipStream_t stream, const void* qp, const void* kp, const void* vp,
+                        const float* wq, const float* wk, const float* wv,
+                        const float* bq_in, const float* bk_in, const float* bv_in,
+                        const float* dq, const float* dk, const float* dv,
+                        void* dqp, void* dkp, void* dvp, float* dwq, float* dwk, float* dwv,
+                        float* dbq, float* dbk, float* dbv,
+                        int B, int T, int H, int d, int K, int in_dtype, int dx_dtype,
+                        void* workspace, size_t workspace_bytes) {
   g_err[0] = 0;
   if (B < 1 || T < 0 || H < 1) return fail(KDA_ERR_INVALID_ARGUMENT, "B=%d, T=%d, H=%d out of range", B, T, H);
   if (!dim_ok(d)) return fail(KDA_ERR_UNSUPPORTED, "d=%d: this build runs d in {64, 128}", d);
   if (K < 1 || K > 8) return fail(KDA_ERR_UNSUPPORTED, "K=%d: conv kernels of 1..8 taps", K);
   if (in_dtype != KDA_DTYPE_F32 && in_dtype != KDA_DTYPE_BF16)
     return fail(KDA_ERR_INVALID_ARGUMENT, "in_dtype=%d: projections are F32 or BF16", in_dtype);
+  if (dx_dtype != KDA_DTYPE_F32 && dx_dtype != in_dtype)
+    return fail(KDA_ERR_INVALID_ARGUMENT, "dx_dtype=%d: F32 or the projections' dtype", dx_dtype);
   if (!wq || !wk || !wv || !dwq || !dwk || !dwv) return fail(KDA_ERR_INVALID_ARGUMENT, "null conv taps or dw");
   if (T > 0 && (!qp || !kp || !vp || !dq || !dk || !dv || !dqp || !dkp || !dvp))
     return fail(KDA_ERR_INVALID_ARGUMENT, "null pointer");
   if (int rc = require_aligned(four_elems(in_dtype) / 2, "qp, kp, vp (two elements)", {qp, kp, vp})) return rc;
-  if (int rc = require_aligned(8, "dq, dk, dv, dqp, dkp, dvp (two elements)", {dq, dk, dv, dqp, dkp, dvp}))
-    return rc;
+  if (int rc = require_aligned(8, "dq, dk, dv (two elements)", {dq, dk, dv})) return rc;
+  if (int rc = require_aligned(four_elems(dx_dtype) / 2, "dqp, dkp, dvp (two elements)", {dqp, dkp, dvp})) return rc;
   if (static_cast<int64_t>(B) * T * H * 3 / 4 > 0x7FFFFFFFLL) return fail(KDA_ERR_INVALID_ARGUMENT, "too large");
   const size_t need = kda_prologue_bwd_workspace(B, T, H, d, K);
   if (!workspace || workspace_bytes < need)
@@ -1124,7 +1184,8 @@ int kda_prologue_bwd(hipStream_t stream, const void* qp, const void* kp, const v
   a.db[0] = K > 1 ? dbq : nullptr; a.db[1] = K > 1 ? dbk : nullptr; a.db[2] = K > 1 ? dbv : nullptr;
   a.B = B; a.T = T; a.H = H; a.K = K; a.G = (T + 63) / 64;
   a.part = static_cast<float*>(workspace);
-  const hipError_t e = kda::launch_prologue_bwd(a, d, in_dtype == KDA_DTYPE_F32 ? 0 : 1, stream);
+  const hipError_t e = kda::launch_prologue_bwd(a, d, in_dtype == KDA_DTYPE_F32 ? 0 : 1,
+                                                dx_dtype == KDA_DTYPE_F32 ? 0 : 1, stream);
   if (e != hipSuccess) return hip_fail(e, "prologue backward launch");
   return KDA_OK;
 }

@@ -319,16 +319,23 @@ struct InTile {
       }
     }
   }
-  // the elements as they are, rows of PITCH elements
-  template <int PITCH>
-  __device__ __forceinline__ void put_raw(typename InT<DT>::t* dst) const {
+  // the elements as they are (LOG: as in put), rows of PITCH elements
+  template <int PITCH, bool LOG = false>
+  __device__ __forceinline__ void put_raw(typename InT<DT>::t* dst, int len = kC) const {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
       const int e = fresh_tid() + p * NTH;
       if (N % NTH == 0 || e < N) {
         const int r = e / V, c8 = e - r * V;
         u32x4* o = reinterpret_cast<u32x4*>(dst + r * PITCH + 8 * c8);
-        auto vec = [](const uint4& x) { return u32x4{x.x, x.y, x.z, x.w}; };
+        auto vec = [&](const uint4& x) {
+          u32x4 y = {x.x, x.y, x.z, x.w};
+          if constexpr (LOG) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = (r < len) ? __float_as_uint(logf(__uint_as_float(y[i]))) : 0u;
+          }
+          return y;
+        };
         if constexpr (DT == 0) {
           o[0] = vec(w[2 * p]);
           o[1] = vec(w[2 * p + 1]);
@@ -338,8 +345,9 @@ struct InTile {
       }
     }
   }
-  template <int PITCH>
-  __device__ __forceinline__ void put(float* dst, float mul) const {
+  // LOG: the elements are decay factors alpha; their logarithm (0 in the rows from len on)
+  template <int PITCH, bool LOG = false>
+  __device__ __forceinline__ void put(float* dst, float mul, int len = kC) const {
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
       const int e = fresh_tid() + p * NTH;
@@ -356,11 +364,39 @@ struct InTile {
           for (int q = 0; q < 4; ++q) { x[q] = lo[q]; x[4 + q] = hi[q]; }
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) dst[r * PITCH + 8 * c8 + q] = x[q] * mul;
+        for (int q = 0; q < 8; ++q) {
+          if constexpr (LOG) dst[r * PITCH + 8 * c8 + q] = (r < len) ? logf(x[q]) : 0.f;
+          else dst[r * PITCH + 8 * c8 + q] = x[q] * mul;
+        }
       }
     }
   }
 };
+
+// Gate type (beside the element types 0 fp32, 1 bf16, 2 fp16) of the cc_scan
+// seam: g holds the decay factors alpha in fp32 (the log decay is their
+// logarithm) and beta the [token-head][32] columns beta32 whose mean it is.
+constexpr int kAlphaGates = 3;
+
+// beta of one token-head (the seam's 32 columns summed in column order, as
+// the forward does)
+template <int DTG>
+__device__ __forceinline__ float ld_beta(const void* p, int64_t th) {
+  if constexpr (DTG == kAlphaGates) {
+    const f4* b = reinterpret_cast<const f4*>(static_cast<const float*>(p) + th * 32);
+    f4 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = b[j];
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += v[j][e];
+    return s * (1.0f / 32.0f);
+  } else {
+    return ld1<DTG>(p, th);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // prep: G, gamma*q, lambda*k, gamma_C, Aqk, T, W, U of one chunk-head
@@ -381,6 +417,8 @@ __device__ __forceinline__ int fa_frag(int it, int kb) { return (it < 2) ? 2 * i
 template <int D, int DTQ, int DTG>
 __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a) {
   constexpr int EF = BwdWs<DTQ != 0>::F;   // gamma q, lambda k, Aqk, T, W, U
+  constexpr bool ALPHA = DTG == kAlphaGates;
+  constexpr int GT = ALPHA ? 0 : DTG;  // element type of g
   constexpr int HD = 64;              // channels per half
   constexpr int NHALF = D / HD;
   // [64][HD] pitch: row fragments conflict-free (rows 4 banks apart), rows
@@ -405,11 +443,11 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
   // (both tiles' loads issued before either is stored)
   auto stage_k_g = [&](int c0) {
     InTile<DTQ, D, HD, NTH> ik;
-    InTile<DTG, D, HD, NTH> ig;
+    InTile<GT, D, HD, NTH> ig;
     ik.fetch(a.k, cr.row0, cr.len, H, h, c0);
     ig.fetch(a.g, cr.row0, cr.len, H, h, c0);
     ik.template put<P>(sK, 1.f);
-    ig.template put<P>(sG, 1.f);
+    ig.template put<P, ALPHA>(sG, 1.f, cr.len);
   };
   // every thread: channel t % HD, rows 8 s .. 8 s + 7 (s = t / HD): the
   // prefix over its rows, then the sums of the segments above it (through
@@ -454,14 +492,14 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
   for (int pi = 0; pi < 2; ++pi) accA[pi] = accL[pi] = f4{0.f, 0.f, 0.f, 0.f};
   // the next half's q, k, g and beta, loaded during this half's scores
   InTile<DTQ, D, HD, NTH> nq, nk;
-  InTile<DTG, D, HD, NTH> ng;
+  InTile<GT, D, HD, NTH> ng;
   float nb = 0.f;
   auto fetch_half = [&](int c0) {
     nq.fetch(a.q, cr.row0, cr.len, H, h, c0);
     nk.fetch(a.k, cr.row0, cr.len, H, h, c0);
     ng.fetch(a.g, cr.row0, cr.len, H, h, c0);
     const int tb = t & (kC - 1);
-    nb = ld1<DTG>(a.beta, (cr.row0 + (tb < cr.len ? tb : 0)) * H + h);
+    nb = ld_beta<DTG>(a.beta, (cr.row0 + (tb < cr.len ? tb : 0)) * H + h);
   };
   fetch_half(0);
   for (int hf = 0; hf < NHALF; ++hf) {
@@ -469,7 +507,7 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
     if (hf > 0) __syncthreads();      // the previous half's reads are done
     nq.template put<P>(sQ, a.scale);
     nk.template put<P>(sK, 1.f);
-    ng.template put<P>(sG, 1.f);
+    ng.template put<P, ALPHA>(sG, 1.f, cr.len);
     if (hf == 0 && t < kC) sB[t] = (t < cr.len) ? nb : 0.f;
     __syncthreads();
     cumsum_g();
@@ -1946,6 +1984,8 @@ struct Col4 {
 template <int D, int DTQ, int DTG, int DO>
 __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(BwdArgs a) {
   constexpr int NTH = ChunkThreads<D>::value;
+  constexpr bool ALPHA = DTG == kAlphaGates;
+  constexpr int GT = ALPHA ? 0 : DTG;  // element type of g
   constexpr int NG = NTH / 256;      // waves per row tile (groups of column tiles)
   constexpr int HW = 64;             // value columns per pass of phase 1
   constexpr int NH = D / HW;
@@ -1972,9 +2012,35 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
   // is stored once.  Phases 1-3 run on the matrix cores as bf16 hi / lo
   // triples.  Pad rows (c >= len) are never stored (their dG is zero: every
   // term carries a factor q_c or k_c).
-  float* const gq_ = a.dq;
-  float* const gk_ = a.dk;
-  float* const gG_ = a.dg;
+  // Output types: fp32, or the primal's 16 bits, rounded here (each rounding
+  // pass over fp32 gradients in memory was 37 us a tensor at 2^25 elements)
+  const int qot = DTQ == 0 ? 0 : ALPHA ? 1 : a.qkv_out;
+  const int got = (DTQ == 0 || GT == 0) ? 0 : a.g_out;
+  // rows c0 .. c0 + 3 (those below len) of column d, the lane's column of 16
+  // consecutive ones; 16-bit: lanes r and r ^ 1 swap one value of each row
+  // pair, so each lane stores packed column pairs of two rows
+  auto put_rows = [&](void* dst, int ot, int c0, int d, const float (&x)[4]) {
+    if (ot == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (c0 + i < cr.len) static_cast<float*>(dst)[in_idx(c0 + i, d)] = x[i];
+    } else {
+      const bool odd = (d & 1) != 0;
+      const float x0 = __shfl_xor(odd ? x[0] : x[1], 1, 64), x1 = __shfl_xor(odd ? x[2] : x[3], 1, 64);
+      const float lo[2] = {odd ? x0 : x[0], odd ? x1 : x[2]}, hi[2] = {odd ? x[1] : x0, odd ? x[3] : x1};
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int c = c0 + 2 * j + (odd ? 1 : 0);
+        uint32_t w;
+        if (ot == 1) w = pack_bf16x2(lo[j], hi[j]);
+        else {
+          typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+          w = __builtin_bit_cast(uint32_t, h2{static_cast<_Float16>(lo[j]), static_cast<_Float16>(hi[j])});
+        }
+        if (c < cr.len) *reinterpret_cast<uint32_t*>(static_cast<u16*>(dst) + in_idx(c, d & ~1)) = w;
+      }
+    }
+  };
   constexpr int NDT = NCT / NG;        // column tiles per wave of a [64][D] product
   float pq[NDT][4], pk[NDT][4], pG[NDT][4];   // partial dq, dk, dG at this thread's positions
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform, as mt and dg_
@@ -2018,7 +2084,7 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
 #pragma unroll
   for (int q = 0; q < NKT; ++q) dAa[q] = f4{0.f, 0.f, 0.f, 0.f};
   constexpr int TTH = 512;   // threads that hold T for its transposed store
-  TTile<kC, TTH, EF> tT;     // phase 2's T, loaded during phase 1's last pass
+  TTile<kC, TTH, EF> tT;     // phase 2's T, loaded during phase 1's epilogue
   // dv~ in row pairs: phase 1's passes take their columns of it, phase 2 the
   // whole tile as dv~^T (one read of dv~ serves both)
   TTile<D, NTH> tY;
@@ -2061,7 +2127,7 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
       pDS.fetch(a.DS + ch * D * D, D, n0);
       pDo.fetch(a.dout, cr.row0, cr.len, H, h, n0);
     };
-    InTile<DTG, D, D, NTH> ig;
+    InTile<GT, D, D, NTH> ig;
     InTile<DTQ, D, D, NTH> iq, ik, iv;
     auto fetch_in = [&]() {
       ig.fetch(a.g, cr.row0, cr.len, H, h, 0);
@@ -2085,24 +2151,31 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
       }
       __syncthreads();
       if (hp + 1 < NH) fetch_pass(hp + 1);
-      else {   // the epilogue's g, q, k, v (fp32 inputs: after the products, for registers) and phase 2's T
-        if constexpr (DTQ != 0) fetch_in();
-        if (t < TTH) tT.fetch(ws_at<EF>(a.TM, ch * kC * kC), kC, 0);
-      }
+      else if constexpr (DTQ != 0) fetch_in();   // the epilogue's g, q, k, v (fp32 inputs: after the products)
 #pragma unroll
       for (int kb = 0; kb < HW / 32; ++kb) {
         const int ka = (16 * mt + r16) * PB + 32 * kb + 8 * gq;
-        const b8 vh = *reinterpret_cast<const b8*>(&sVh[ka]), vl = *reinterpret_cast<const b8*>(&sVl[ka]);
-        const b8 oh = *reinterpret_cast<const b8*>(&sOh[ka]), ol = *reinterpret_cast<const b8*>(&sOl[ka]);
-        const b8 uh = *reinterpret_cast<const b8*>(&sUh[ka]), ul = *reinterpret_cast<const b8*>(&sUl[ka]);
+        // (operands in two groups, which bounds the fragments in registers)
+        {
+          const b8 vh = *reinterpret_cast<const b8*>(&sVh[ka]), vl = *reinterpret_cast<const b8*>(&sVl[ka]);
 #pragma unroll
-        for (int q = 0; q < NDT; ++q) {
-          const int kbb = (16 * (dg_ * NDT + q) + r16) * PB + 32 * kb + 8 * gq;
-          const b8 sh = *reinterpret_cast<const b8*>(&sSh[kbb]), sl = *reinterpret_cast<const b8*>(&sSl[kbb]);
-          const b8 dh = *reinterpret_cast<const b8*>(&sDh[kbb]), dl = *reinterpret_cast<const b8*>(&sDl[kbb]);
-          dY[q] = mma3_bf16(dY[q], vh, vl, dh, dl);
-          dgq[q] = mma3_bf16(dgq[q], oh, ol, sh, sl);
-          dW[q] = mma3_bf16(dW[q], uh, ul, sh, sl);
+          for (int q = 0; q < NDT; ++q) {
+            const int kbb = (16 * (dg_ * NDT + q) + r16) * PB + 32 * kb + 8 * gq;
+            dY[q] = mma3_bf16(dY[q], vh, vl, *reinterpret_cast<const b8*>(&sDh[kbb]),
+                              *reinterpret_cast<const b8*>(&sDl[kbb]));
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const b8 oh = *reinterpret_cast<const b8*>(&sOh[ka]), ol = *reinterpret_cast<const b8*>(&sOl[ka]);
+        {
+          const b8 uh = *reinterpret_cast<const b8*>(&sUh[ka]), ul = *reinterpret_cast<const b8*>(&sUl[ka]);
+#pragma unroll
+          for (int q = 0; q < NDT; ++q) {
+            const int kbb = (16 * (dg_ * NDT + q) + r16) * PB + 32 * kb + 8 * gq;
+            const b8 sh = *reinterpret_cast<const b8*>(&sSh[kbb]), sl = *reinterpret_cast<const b8*>(&sSl[kbb]);
+            dgq[q] = mma3_bf16(dgq[q], oh, ol, sh, sl);
+            dW[q] = mma3_bf16(dW[q], uh, ul, sh, sl);
+          }
         }
 #pragma unroll
         for (int q = 0; q < NKT; ++q) {
@@ -2117,36 +2190,39 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
     // g, q, k and v of the chunk-head through LDS (over phase 1's planes) to
     // this thread's positions: whole rows are read from memory and the lanes'
     // column reads fall on distinct banks (pad rows are zero)
-    constexpr int PG = D + (DTG == 0 ? 4 : 8), PQ = D + (DTQ == 0 ? 4 : 8);
+    constexpr int PG = D + (GT == 0 ? 4 : 8), PQ = D + (DTQ == 0 ? 4 : 8);
     typedef typename InT<DTQ>::t EQ;
-    typedef typename InT<DTG>::t EG;
+    typedef typename InT<GT>::t EG;
     EG* const sGr = reinterpret_cast<EG*>(sm);
     EQ* const sQr = reinterpret_cast<EQ*>(sm + (sizeof(EG) * kC * PG) / 4);
     EQ* const sKr = sQr + kC * PQ;
     EQ* const sVr = sKr + kC * PQ;
     static_assert(sizeof(EG) * kC * PG + 3 * sizeof(EQ) * kC * PQ <= 4 * GS0, "g, q, k, v end below the sums of g");
     if constexpr (DTQ == 0) fetch_in();
-    ig.template put_raw<PG>(sGr);
+    ig.template put_raw<PG, ALPHA>(sGr, cr.len);
     iq.template put_raw<PQ>(sQr);
     ik.template put_raw<PQ>(sKr);
     iv.template put_raw<PQ>(sVr);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = 16 * mt + 4 * gq + i;
-      const float x = ld1<DTG>(a.beta, (cr.row0 + (c < cr.len ? c : 0)) * H + h);
-      bH[i] = (c < cr.len) ? x : 0.f;
+    float* const sBt = sm + GS0 - kC;
+    static_assert(sizeof(EG) * kC * PG + 3 * sizeof(EQ) * kC * PQ <= 4 * (GS0 - kC), "beta past g, q, k, v");
+    if (t < kC) {
+      const float x = ld_beta<DTG>(a.beta, (cr.row0 + (t < cr.len ? t : 0)) * H + h);
+      sBt[t] = (t < cr.len) ? x : 0.f;
     }
     __syncthreads();
     // G_c = log2(e) sum_{c' <= c} g_c' at this thread's positions, from g:
     // the prefix over the lane's four rows, plus the lane groups above it in
     // the row tile (shuffles), plus the row tiles above (their sums through
     // LDS, past phase 2's buffers).
+    if (t < TTH) tT.fetch(ws_at<EF>(a.TM, ch * kC * kC), kC, 0);
     float* const sGs = sm + GS0;
     const int c0 = 16 * mt + 4 * gq;
 #pragma unroll
+    for (int i = 0; i < 4; ++i) bH[i] = sBt[c0 + i];
+#pragma unroll
     for (int q = 0; q < NDT; ++q) {
       const int d = 16 * (dg_ * NDT + q) + r16;
-      Col4<DTG> gR;
+      Col4<GT> gR;
       gR.load(sGr + c0 * PG + d, PG);
 #pragma unroll
       for (int i = 0; i < 4; ++i) gH[q][i] = gR.get(i);
@@ -2270,28 +2346,19 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
     int cb = 16 * mt + 4 * gq;   // (addresses formed here, not held from the loads)
     opaque(cb);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = cb + i;
-      const bool live = c < cr.len;
-      const float bc = bH[i];
-      float kv[NDT], vv[NDT], oG[NDT], ok[NDT];
+    for (int q = 0; q < NDT; ++q) {
+      const int d = 16 * (dg_ * NDT + q) + r16;
+      float gv[4];
 #pragma unroll
-      for (int q = 0; q < NDT; ++q) {
-        const int d = 16 * (dg_ * NDT + q) + r16;
-        kv[q] = kH[q].get(i);
-        vv[q] = vH[q].get(i);
-        oG[q] = sAcc[(kC + c) * D + d];
-        ok[q] = sAcc[c * D + d];
+      for (int i = 0; i < 4; ++i) {
+        const int c = cb + i;
+        const float bc = bH[i], gam = ex2(gH[q][i]), kv = kH[q].get(i);
+        dbrD[i] += Yw[q][i] * gam * kv + Yu[q][i] * vH[q].get(i);
+        pG[q][i] = sAcc[(kC + c) * D + d] + Yw[q][i] * kv * bc * gam;
+        pk[q][i] = sAcc[c * D + d] + Yw[q][i] * gam * bc;
+        gv[i] = Yu[q][i] * bc;
       }
-#pragma unroll
-      for (int q = 0; q < NDT; ++q) {
-        const int d = 16 * (dg_ * NDT + q) + r16;
-        const float gam = ex2(gH[q][i]);
-        dbrD[i] += Yw[q][i] * gam * kv[q] + Yu[q][i] * vv[q];
-        pG[q][i] = oG[q] + Yw[q][i] * kv[q] * bc * gam;
-        pk[q][i] = ok[q] + Yw[q][i] * gam * bc;
-        if (live) a.dv[in_idx(c, d)] = Yu[q][i] * bc;
-      }
+      put_rows(a.dv, qot, cb, d, gv);
     }
     __syncthreads();   // sAcc read before phase 3's operands overwrite it
     carry(pk);
@@ -2538,7 +2605,7 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
             }
           }
         }
-        float gn[4];   // this tile's dG (zero on pad rows)
+        float gn[4], oq[4], ok[4];   // this tile's dG (zero on pad rows), dq, dk
         int cb = 16 * mt + 4 * gq;   // (addresses formed here, not held from the loads)
         opaque(cb);
 #pragma unroll
@@ -2547,12 +2614,11 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
           const float kc = kH[q].get(e), qc = qH[q].get(e) * a.scale, bc = bH[e];
           dbrD[e] = fmaf(rK[q][e], kc, dbrD[e]);
           gn[e] = (c < cr.len) ? pG[q][e] + rA[q][e] * qc + rK[q][e] * kc * bc - cS[q][e] * kc : 0.f;
-          if (c < cr.len) {
-            const int64_t o = in_idx(c, d);
-            gq_[o] = pq[q][e] + rA[q][e] * a.scale;
-            gk_[o] = pk[q][e] + rK[q][e] * bc + cS[q][e];
-          }
+          oq[e] = pq[q][e] + rA[q][e] * a.scale;
+          ok[e] = pk[q][e] + rK[q][e] * bc + cS[q][e];
         }
+        put_rows(a.dq, qot, cb, d, oq);
+        put_rows(a.dk, qot, cb, d, ok);
         // reverse cumsum down the column: within the lane's four rows, then
         // over the row groups gq' > gq of the tile (lanes 16 gq' + r16); the
         // tiles below come after the barrier
@@ -2574,6 +2640,16 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
       for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
       if (r16 == 0) sDb[(16 * mt + 4 * gq + e) * NG + dg_] = v;
     }
+    float al[NDT][4];   // the seam's alpha at this thread's positions
+    if constexpr (ALPHA) {
+      int cb = 16 * mt + 4 * gq;
+      opaque(cb);
+#pragma unroll
+      for (int q = 0; q < NDT; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          al[q][e] = static_cast<const float*>(a.g)[in_idx(cb + e < cr.len ? cb + e : 0, 16 * (dg_ * NDT + q) + r16)];
+    }
     __syncthreads();   // every tile's column sums and dbeta's row sums written
 #pragma unroll
     for (int q = 0; q < NDT; ++q) {
@@ -2583,17 +2659,32 @@ __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(B
       const float base = sBase[d] + carry + abv[q];
       int cb = 16 * mt + 4 * gq;
       opaque(cb);
+      float gn[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int c = cb + e;
-        if (c < cr.len) gG_[in_idx(c, d)] = base + sfx[q][e];
+        gn[e] = base + sfx[q][e];
+        if constexpr (ALPHA) gn[e] /= al[q][e];   // dalpha = d(log alpha) / alpha
       }
+      put_rows(a.dg, got, cb, d, gn);
     }
-    if (t < kC && t < cr.len) {
+    if constexpr (ALPHA) {   // each of the 32 columns gets a 32nd
+      constexpr int V = 8;   // 16-byte pieces per row
+      if (t < kC * V && t / V < cr.len) {
+        const int row = t / V;
+        float x = sDb[row * NG];
+#pragma unroll
+        for (int j = 1; j < NG; ++j) x += sDb[row * NG + j];
+        x *= 1.0f / 32.0f;
+        *reinterpret_cast<f4*>(static_cast<float*>(a.dbeta) + ((cr.row0 + row) * H + h) * 32 + 4 * (t % V)) = f4{x, x, x, x};
+      }
+    } else if (t < kC && t < cr.len) {
       float x = sDb[t * NG];
 #pragma unroll
       for (int j = 1; j < NG; ++j) x += sDb[t * NG + j];
-      a.dbeta[(cr.row0 + t) * H + h] = x;
+      const int64_t o = (cr.row0 + t) * H + h;
+      if (got == 0) static_cast<float*>(a.dbeta)[o] = x;
+      else if (got == 1) static_cast<u16*>(a.dbeta)[o] = cvt_bf16(x);
+      else static_cast<_Float16*>(a.dbeta)[o] = static_cast<_Float16>(x);
     }
   }
 }
@@ -2649,6 +2740,8 @@ hipError_t launch_copy_or_zero(float* dst, const float* src, int64_t n, hipStrea
 }
 
 hipError_t launch_bwd(const BwdArgs& a, int d, int in_dtype, int do_dtype, hipStream_t s) {
+  if (in_dtype == kInAlphaGates)   // do is fp32
+    return d == 128 ? launch_bwd_t<128, 1, kAlphaGates, 0>(a, s) : launch_bwd_t<64, 1, kAlphaGates, 0>(a, s);
   if (d == 128) return do_dtype == 0 ? launch_bwd_dt<128, 0>(a, in_dtype, s) : launch_bwd_dt<128, 1>(a, in_dtype, s);
   return do_dtype == 0 ? launch_bwd_dt<64, 0>(a, in_dtype, s) : launch_bwd_dt<64, 1>(a, in_dtype, s);
 }

@@ -118,11 +118,12 @@ struct BwdArgs {
   const void* dout;     // cotangent of o, [B,T,H,dv] (fp32 or bf16)
   const float* dht;     // cotangent of the final state, [B,H,dk,dv] or null
   float scale;
-  float* dq;            // [B,T,H,dk]
-  float* dk;
-  float* dv;            // [B,T,H,dv]
-  float* dg;            // [B,T,H,dk]
-  float* dbeta;         // [B,T,H]
+  void* dq;             // [B,T,H,dk] of element type qkv_out
+  void* dk;
+  void* dv;             // [B,T,H,dv]
+  void* dg;             // [B,T,H,dk] of element type g_out
+  void* dbeta;          // [B,T,H]
+  int qkv_out, g_out;   // 0 fp32, 1 bf16, 2 fp16 (16-bit only where the input is of that type)
   float* dh0;           // [B,H,dk,dv] or null
   float* QG;            // [ch][C][dk] gamma * q (scaled)
   float* KL;            // [ch][C][dk] lambda * k
@@ -189,7 +190,7 @@ struct PrologueBwdArgs {
   const float* w[3];       // [K, H*d]
   const float* bin[3];     // [B, K-1, H*d] or null (zeros)
   const float* dy[3];      // dq, dk, dv [B,T,H*d] fp32
-  float* dx[3];            // [B,T,H*d] fp32
+  void* dx[3];             // [B,T,H*d] fp32, or bf16 with bf16 projections
   float* dw[3];            // [K, H*d] fp32
   float* db[3];            // [B, K-1, H*d] fp32 or null (not wanted)
   float* part;             // workspace: [3][B * G][K][H*d] fp32, dw partial sums (G groups of 64 rows)
@@ -207,12 +208,16 @@ struct EpilogueBwdArgs {
 };
 
 hipError_t launch_prologue(const PrologueArgs& a, int d, int in_dt, int out_dt, hipStream_t s);
-hipError_t launch_prologue_bwd(const PrologueBwdArgs& a, int d, int in_dt, hipStream_t s);
+hipError_t launch_prologue_bwd(const PrologueBwdArgs& a, int d, int in_dt, int dx_dt, hipStream_t s);
 hipError_t launch_epilogue_bwd(const EpilogueBwdArgs& a, int d, int o_dt, int g_dt, int dy_dt, int dg_dt,
                                hipStream_t s);
 // only the conv buffer update of launch_prologue (the last K-1 inputs)
 hipError_t launch_prologue_buffers(const PrologueArgs& a, int d, int in_dt, hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs& a, int d, int o_dt, int g_dt, int y_dt, hipStream_t s);
+// in_dtype: a kda_dtype_t, or kInAlphaGates (the cc_scan seam: bf16 q, k, v,
+// fp32 do; g = alpha, beta = beta32 [token-head][32], dg = dalpha, dbeta =
+// dbeta32, bf16 dq, dk, dv)
+constexpr int kInAlphaGates = 16;
 hipError_t launch_bwd(const BwdArgs& a, int d, int in_dtype, int do_dtype, hipStream_t s);
 hipError_t launch_ut(const UtArgs& a, int dtype, bool transpose, bool with_da, hipStream_t s);
 // dst[0..n) = src (or 0 when src is null), by a kernel (no memset/memcpy node)
@@ -275,3 +280,22 @@ struct CcFinishArgs {
 hipError_t launch_cc_finish(const CcFinishArgs& a, hipStream_t s);
 
 }  // namespace kda
+
+// Entry points of the package's own binding (axiom_amd/_lib.py), outside the C
+// ABI: kda_chunk_bwd and kda_prologue_bwd with the outputs' types chosen by
+// the caller.  dq, dk, dv in qkv_grad_dtype (KDA_DTYPE_F32 or the dtype of q,
+// k, v), dg and dbeta in gate_grad_dtype (F32 or the dtype of g, beta); dqp,
+// dkp, dvp in dx_dtype (F32 or in_dtype).  A 16-bit gradient is the fp32 one
+// rounded to nearest even by the kernel that forms it.
+extern "C" {
+__attribute__((visibility("default"))) int axiom_chunk_bwd(
+    hipStream_t stream, const void* q, const void* k, const void* v, const void* g, const void* beta, const float* h0,
+    const void* dout, const float* dht, void* dq, void* dk, void* dv, void* dg, void* dbeta, float* dh0, int B, int T,
+    int H, int dk_dim, int dv_dim, int chunk, float scale, int in_dtype, int dout_dtype, int qkv_grad_dtype,
+    int gate_grad_dtype, void* workspace, size_t workspace_bytes);
+__attribute__((visibility("default"))) int axiom_prologue_bwd(
+    hipStream_t stream, const void* qp, const void* kp, const void* vp, const float* wq, const float* wk,
+    const float* wv, const float* bq_in, const float* bk_in, const float* bv_in, const float* dq, const float* dk,
+    const float* dv, void* dqp, void* dkp, void* dvp, float* dwq, float* dwk, float* dwv, float* dbq, float* dbk,
+    float* dbv, int B, int T, int H, int d, int K, int in_dtype, int dx_dtype, void* workspace, size_t workspace_bytes);
+}

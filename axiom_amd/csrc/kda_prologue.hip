@@ -373,7 +373,7 @@ __device__ __forceinline__ void ld_row(const void* row, unsigned lo, float (&o)[
   }
 }
 
-template <int DI, int D, int KW>
+template <int DI, int DX, int D, int KW>
 __global__ __launch_bounds__(64 * kRowsPerBlock) void kda_prologue_bwd_kernel(PrologueBwdArgs a) {
   constexpr int RW = 16;
   constexpr int HW = KW - 1;      // halo rows (da after the block; x before it)
@@ -496,7 +496,7 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void kda_prologue_bwd_kernel(Pr
       for (int q = 0; q < PL; ++q) dd[r][q] *= fv[r][q];
   }
   // dx
-  float* xo = pick3(a.dx, tensor) + rowbase;
+  void* xo = pick3(a.dx, tensor);
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
     if (t0 + r >= a.T) break;
@@ -507,9 +507,16 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void kda_prologue_bwd_kernel(Pr
 #pragma unroll
       for (int i = 0; i < KW; ++i) acc[q] = fmaf(wt[i][q], dd[r + i][q], acc[q]);
     }
-    float* p = xo + static_cast<int64_t>(t0 + r) * HD + lo;
-    if constexpr (PL == 2) *reinterpret_cast<float2*>(p) = make_float2(acc[0], acc[1]);
-    else p[0] = acc[0];
+    const int64_t o = rowbase + static_cast<int64_t>(t0 + r) * HD + lo;
+    if constexpr (DX == 0) {
+      float* p = static_cast<float*>(xo) + o;
+      if constexpr (PL == 2) *reinterpret_cast<float2*>(p) = make_float2(acc[0], acc[1]);
+      else p[0] = acc[0];
+    } else {   // rounded here: no pass over fp32 gradients afterwards
+      u16* p = static_cast<u16*>(xo) + o;
+      if constexpr (PL == 2) *reinterpret_cast<unsigned*>(p) = pack_bf16x2(acc[0], acc[1]);
+      else p[0] = cvt_bf16(acc[0]);
+    }
   }
   // the incoming buffer: sequence row -m (m = 1 .. K-1) is its row K-1-m and
   // reaches the outputs 0 .. KW-1-m through taps m .. KW-1
@@ -602,11 +609,13 @@ __global__ __launch_bounds__(64 * kDwWaves) void kda_prologue_bwd_dw_kernel(Prol
 }
 
 template <int D, int KW>
-hipError_t launch_prologue_bwd_k(const PrologueBwdArgs& a, int in_dt, hipStream_t s) {
+hipError_t launch_prologue_bwd_k(const PrologueBwdArgs& a, int in_dt, int dx_dt, hipStream_t s) {
   if (a.T > 0) {
     const int grid = 3 * a.B * a.H * a.G;
-    if (in_dt == 0) hipLaunchKernelGGL((kda_prologue_bwd_kernel<0, D, KW>), dim3(grid), dim3(64 * kRowsPerBlock), 0, s, a);
-    else hipLaunchKernelGGL((kda_prologue_bwd_kernel<1, D, KW>), dim3(grid), dim3(64 * kRowsPerBlock), 0, s, a);
+    const dim3 blk(64 * kRowsPerBlock);
+    if (in_dt == 0) hipLaunchKernelGGL((kda_prologue_bwd_kernel<0, 0, D, KW>), dim3(grid), blk, 0, s, a);
+    else if (dx_dt == 0) hipLaunchKernelGGL((kda_prologue_bwd_kernel<1, 0, D, KW>), dim3(grid), blk, 0, s, a);
+    else hipLaunchKernelGGL((kda_prologue_bwd_kernel<1, 1, D, KW>), dim3(grid), blk, 0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -697,9 +706,10 @@ hipError_t launch_epilogue(const EpilogueArgs& a, int d, int o_dt, int g_dt, int
 
 namespace kda {
 
-hipError_t launch_prologue_bwd(const PrologueBwdArgs& a, int d, int in_dt, hipStream_t s) {
-  if (d == 128) return a.K <= 4 ? launch_prologue_bwd_k<128, 4>(a, in_dt, s) : launch_prologue_bwd_k<128, 8>(a, in_dt, s);
-  return a.K <= 4 ? launch_prologue_bwd_k<64, 4>(a, in_dt, s) : launch_prologue_bwd_k<64, 8>(a, in_dt, s);
+hipError_t launch_prologue_bwd(const PrologueBwdArgs& a, int d, int in_dt, int dx_dt, hipStream_t s) {
+  if (d == 128)
+    return a.K <= 4 ? launch_prologue_bwd_k<128, 4>(a, in_dt, dx_dt, s) : launch_prologue_bwd_k<128, 8>(a, in_dt, dx_dt, s);
+  return a.K <= 4 ? launch_prologue_bwd_k<64, 4>(a, in_dt, dx_dt, s) : launch_prologue_bwd_k<64, 8>(a, in_dt, dx_dt, s);
 }
 
 hipError_t launch_epilogue_bwd(const EpilogueBwdArgs& a, int d, int o_dt, int g_dt, int dy_dt, int dg_dt,

@@ -202,6 +202,14 @@ def kda_chunk_bwd(q, k, v, g, beta, do, dht=None, initial_state=None, scale: flo
     ``dg`` is the cotangent of the log decay ``g``.  The backward rule of the
     reference's ``cc_scan`` (``net/kernels/kda_cc_fused_persist.py:1707``).
     """
+    return _chunk_bwd(q, k, v, g, beta, do, dht, initial_state, scale, chunk_size, need_dh0, workspace,
+                      torch.float32, torch.float32)
+
+
+def _chunk_bwd(q, k, v, g, beta, do, dht, initial_state, scale, chunk_size, need_dh0, workspace,
+               qkv_dtype, gate_dtype):
+    """:func:`kda_chunk_bwd` with dq, dk, dv in ``qkv_dtype`` and dg, dbeta in
+    ``gate_dtype`` (fp32, or the primal's dtype: rounded by the kernel that forms them)."""
     what = "kda_chunk_bwd"
     if q.dim() != 4 or k.shape != q.shape or g.shape != q.shape:
         raise ValueError(f"{what}: q, k, g must share a [B,T,H,dk] shape")
@@ -238,18 +246,17 @@ def kda_chunk_bwd(q, k, v, g, beta, do, dht=None, initial_state=None, scale: flo
         raise ValueError(f"{what}: unsupported configuration")
     if workspace is None or workspace.numel() * workspace.element_size() < ws_bytes:
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    f32 = torch.float32
-    dq = torch.empty((B, T, H, dk), dtype=f32, device=dev)
-    dk_ = torch.empty((B, T, H, dk), dtype=f32, device=dev)
-    dv_ = torch.empty((B, T, H, dv), dtype=f32, device=dev)
-    dg = torch.empty((B, T, H, dk), dtype=f32, device=dev)
-    dbeta = torch.empty((B, T, H), dtype=f32, device=dev)
-    dh0 = torch.empty((B, H, dk, dv), dtype=f32, device=dev) if need_dh0 else None
-    rc = L.kda_chunk_bwd(_stream(dev), _ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta),
+    dq = torch.empty((B, T, H, dk), dtype=qkv_dtype, device=dev)
+    dk_ = torch.empty((B, T, H, dk), dtype=qkv_dtype, device=dev)
+    dv_ = torch.empty((B, T, H, dv), dtype=qkv_dtype, device=dev)
+    dg = torch.empty((B, T, H, dk), dtype=gate_dtype, device=dev)
+    dbeta = torch.empty((B, T, H), dtype=gate_dtype, device=dev)
+    dh0 = torch.empty((B, H, dk, dv), dtype=torch.float32, device=dev) if need_dh0 else None
+    rc = L.axiom_chunk_bwd(_stream(dev), _ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta),
                          _ptr(initial_state), _ptr(do), _ptr(dht),
                          _ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dg), _ptr(dbeta), _ptr(dh0),
                          B, T, H, dk, dv, CHUNK, float(scale), in_code, _OUT_CODES[do.dtype],
-                         _ptr(workspace), ws_bytes)
+                         _IN_CODES[qkv_dtype], _IN_CODES[gate_dtype], _ptr(workspace), ws_bytes)
     _lib.check(rc, what)
     return dq, dk_, dv_, dg, dbeta, dh0
 
@@ -273,10 +280,9 @@ class _KDAChunk(torch.autograd.Function):
         if do.dtype not in _OUT_CODES:
             do = do.float()
         dht = None if dht is None else dht.float().contiguous()
-        dq, dk, dv, dg, dbeta, dh0 = kda_chunk_bwd(q, k, v, g, beta, do, dht=dht, initial_state=h0,
-                                                   scale=ctx.scale, need_dh0=ctx.needs_input_grad[5])
-        return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype),
-                dh0, None)
+        grads = _chunk_bwd(q, k, v, g, beta, do, dht, h0, ctx.scale, CHUNK, ctx.needs_input_grad[5], None,
+                           q.dtype, g.dtype)
+        return (*grads, None)
 
 
 def kda_chunk(q, k, v, g, beta, initial_state=None, scale: float = 1.0):
@@ -570,6 +576,11 @@ def kda_prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state=None, worksp
     gradients (None when ``conv_state`` is None or K == 1).  A row whose
     swish output is all zeros gets a zero L2-norm gradient.
     """
+    return _prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state, workspace, torch.float32)
+
+
+def _prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state, workspace, dx_dtype):
+    """:func:`kda_prologue_bwd` with dqp, dkp, dvp in ``dx_dtype`` (fp32 or the projections' dtype)."""
     what = "kda_prologue_bwd"
     if qp.dim() != 3 or kp.shape != qp.shape or vp.shape != qp.shape:
         raise ValueError(f"{what}: qp, kp, vp must share a [B,T,H*d] shape")
@@ -604,16 +615,16 @@ def kda_prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state=None, worksp
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     f32 = torch.float32
-    dx = tuple(torch.empty((B, T, HD), dtype=f32, device=dev) for _ in range(3))
+    dx = tuple(torch.empty((B, T, HD), dtype=dx_dtype, device=dev) for _ in range(3))
     dw = tuple(torch.empty((K, HD), dtype=f32, device=dev) for _ in range(3))
     want_db = conv_state is not None and K > 1
     db = tuple(torch.empty((B, K - 1, HD), dtype=f32, device=dev) for _ in range(3)) if want_db \
         else (None, None, None)
     bin_ = conv_state if conv_state is not None else (None, None, None)
-    rc = L.kda_prologue_bwd(_stream(dev), _ptr(qp), _ptr(kp), _ptr(vp), _ptr(wq), _ptr(wk), _ptr(wv),
+    rc = L.axiom_prologue_bwd(_stream(dev), _ptr(qp), _ptr(kp), _ptr(vp), _ptr(wq), _ptr(wk), _ptr(wv),
                             *(_ptr(b) for b in bin_), _ptr(dq), _ptr(dk), _ptr(dv),
                             *(_ptr(t) for t in dx), *(_ptr(t) for t in dw), *(_ptr(t) for t in db),
-                            B, T, H, d, K, _UT_CODES[qp.dtype], _ptr(workspace), need)
+                            B, T, H, d, K, _UT_CODES[qp.dtype], _UT_CODES[dx_dtype], _ptr(workspace), need)
     _lib.check(rc, what)
     return dx, dw, (db if want_db else None)
 
@@ -678,12 +689,11 @@ class _KDALayer(torch.autograd.Function):
                                   out_dtype=qp.dtype)
         do, dgate = kda_epilogue_bwd(o, gate, dy, eps=ctx.eps)
         dht = None if dht is None else dht.float().contiguous()
-        dq, dk, dv, dg, dbeta, dh0 = kda_chunk_bwd(q, k, v, g, beta, do, dht=dht, initial_state=h0,
-                                                   scale=ctx.scale, need_dh0=ctx.needs_input_grad[12])
-        dx, dw, db = kda_prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state=conv_state)
+        dq, dk, dv, dg, dbeta, dh0 = _chunk_bwd(q, k, v, g, beta, do, dht, h0, ctx.scale, CHUNK,
+                                                ctx.needs_input_grad[12], None, torch.float32, g.dtype)
+        dx, dw, db = _prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state, None, qp.dtype)
         db = db if db is not None else (None, None, None)
-        return (dx[0].to(qp.dtype), dx[1].to(kp.dtype), dx[2].to(vp.dtype), dg.to(g.dtype),
-                dbeta.to(beta.dtype), dgate, dw[0], dw[1], dw[2], db[0], db[1], db[2], dh0, None, None)
+        return (dx[0], dx[1], dx[2], dg, dbeta, dgate, dw[0], dw[1], dw[2], db[0], db[1], db[2], dh0, None, None)
 
 
 def kda_layer(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state=None, initial_state=None,
