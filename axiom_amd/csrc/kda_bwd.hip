@@ -4,8 +4,8 @@
 // with respect to q, k, v, g (the log decay), beta and h0, following the
 // reference's analytic adjoint per chunk (net/kernels/kda_cc_fused_bwd.py:30-55,
 // code :139-228) scanned in reverse over the chunks
-// (net/kernels/kda_cc_fused_persist.py:794-842, reference_bwd_scan).  Four
-// launches:
+// (net/kernels/kda_cc_fused_persist.py:794-842, reference_bwd_scan).  Three
+// launches, the two scans in one:
 //   kda_bwd_prep_kernel   one workgroup per chunk-head: in-chunk log2 cumsum G,
 //                         gamma*q, lambda*k, gamma_C, Aqk, T = (I+L)^-1, W, U;
 //   forward state scan    one workgroup per (chain, 32 value columns): every
@@ -19,16 +19,15 @@
 //                         score adjoints, the cumsum adjoint) and the outputs.
 // Two precisions of the workspace, chosen by the input dtype:
 //  * fp32 inputs: every workspace array fp32 row-major per chunk-head
-//    ch = (b * NT + n) * H + h; scans kda_bwd_fscan_kernel and
-//    kda_bwd_rscan_kernel (16 waves, operands split into bf16 hi/lo planes
-//    in LDS each chunk step).
+//    ch = (b * NT + n) * H + h; scans fscan_block and rscan_block
+//    (16 waves, operands split into bf16 hi/lo planes in LDS each chunk step).
 //  * 16-bit inputs (bf16, fp16): the forward-side arrays gamma q, lambda k,
 //    Aqk, T, W and the stored state S are fp16 (BwdWs<true>: the operand
 //    width the forward's own kernels give them), and the
 //    prep kernel writes the scans' operands directly as MFMA lane fragments
 //    (FL, FA, FQ, FW, FWN, FLT); G, gamma_C, U, v~ and the cotangents dS', dv~
-//    stay fp32.  Scans kda_bwd_fscan16_kernel and kda_bwd_rscan16_kernel in
-//    the column-owner form: two compute waves (one 16-column tile each of the
+//    stay fp32.  Scans fscan16_block and rscan16_block in the column-owner
+//    form: two compute waves (one 16-column tile each of the
 //    32-column slice, the state slice in their accumulators) and four
 //    producer waves that load two chunks ahead into registers, fill a
 //    double-buffered LDS chunk, and store the compute waves' staged outputs
@@ -232,8 +231,8 @@ constexpr float kDiagAnchorLog2 = 32.f;
 // of a chain on one XCD (workgroup x runs on XCD x % 8), so the operands all
 // of them read come from that XCD's L2.  Grid: ceil(chains / 8) * 8 * NS.
 template <int NS>
-__device__ __forceinline__ bool scan_slot(int nchains, int& chain, int& split) {
-  const int x = blockIdx.x, xcd = x & 7, kk = x >> 3;
+__device__ __forceinline__ bool scan_slot(int x, int nchains, int& chain, int& split) {
+  const int xcd = x & 7, kk = x >> 3;
   const int slot = kk / NS;
   split = kk - slot * NS;
   chain = slot * 8 + xcd;
@@ -876,24 +875,32 @@ struct TTile {
 // stored; S rounded as it is stored, v~ rounded for the product and stored
 // in fp32), so each product is one fp16 MFMA per K block, the forward
 // kernels' operand precision.
+template <int D>
+struct alignas(16) FscanLds {
+  static constexpr int PW = D + 8;     // bf16 pitch of rows whose K index is a channel
+  static constexpr int PK = kC + 8;    // bf16 pitch of rows whose K index is a chunk row
+  __bf16 Wh[kC * PW], Wl[kC * PW];     // W [64][D]
+  __bf16 Kh[D * PK], Kl[D * PK];       // (lambda k)^T [D][64]
+  __bf16 Sh[32 * PW], Sl[32 * PW];     // S^T [32][D]
+  __bf16 Vh[32 * PK], Vl[32 * PK];     // v~^T [32][64]
+  float U[kC * kPB], GC[D];
+};
+
 template <int D, bool WS16>
-__global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_fscan_kernel(BwdArgs a) {
+__device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLds<D>& L) {
   constexpr int EF = BwdWs<WS16>::F;   // W, lambda k in; S_in out
   constexpr int NTH = ScanThreads<D>::value;
   constexpr int NS = D / 32;
   constexpr int NST = (D / 8) / (NTH / 64);   // state tiles per wave (D / 8 tiles of the 32-column slice)
   static_assert(NST >= 1, "at least one state tile per wave");
-  constexpr int PW = D + 8;     // bf16 pitch of rows whose K index is a channel
-  constexpr int PK = kC + 8;    // bf16 pitch of rows whose K index is a chunk row
-  __shared__ __attribute__((aligned(16))) __bf16 sWh[kC * PW], sWl[kC * PW];    // W [64][D]
-  __shared__ __attribute__((aligned(16))) __bf16 sKh[D * PK], sKl[D * PK];      // (lambda k)^T [D][64]
-  __shared__ __attribute__((aligned(16))) __bf16 sSh[32 * PW], sSl[32 * PW];    // S^T [32][D]
-  __shared__ __attribute__((aligned(16))) __bf16 sVh[32 * PK], sVl[32 * PK];    // v~^T [32][64]
-  __shared__ float sU[kC * kPB], sGC[D];
+  constexpr int PW = FscanLds<D>::PW, PK = FscanLds<D>::PK;
+  __bf16 *const sWh = L.Wh, *const sWl = L.Wl, *const sKh = L.Kh, *const sKl = L.Kl;
+  __bf16 *const sSh = L.Sh, *const sSl = L.Sl, *const sVh = L.Vh, *const sVl = L.Vl;
+  float *const sU = L.U, *const sGC = L.GC;
   const int t = threadIdx.x, wv = t >> 6, l = t & 63, r = l & 15, gq = l >> 4;
   const int H = a.H;
   int chain, split;
-  if (!scan_slot<NS>(a.B * H, chain, split)) return;   // uniform per workgroup
+  if (!scan_slot<NS>(block, a.B * H, chain, split)) return;   // uniform per workgroup
   const int b = chain / H, h = chain - b * H;
   const int c0 = 32 * split;
   const int mt = wv >> 1, ct = wv & 1;                  // this wave's v~ tile (waves 0-7: 8 tiles)
@@ -1071,27 +1078,37 @@ __global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_fscan_kernel(Bw
 //   C  dS <- dS - W^T dv~; every wave stages lambda k, Aqk^T, do^T,
 //      (gamma q)^T and gamma_C of the next chunk (read in its A and B) and
 //      loads the one after.
+template <int D>
+struct alignas(16) RscanLds {
+  static constexpr int PW = D + 8;     // bf16 pitch of rows whose K index is a channel
+  static constexpr int PK = kC + 8;    // bf16 pitch of rows whose K index is a chunk row
+  __bf16 Lh[kC * PW], Ll[kC * PW];     // lambda k [64][D]
+  __bf16 Ah[kC * PK], Al[kC * PK];     // Aqk^T [64][64]
+  __bf16 Qh[D * PK], Ql[D * PK];       // (gamma q)^T [D][64]
+  __bf16 Wh[D * PK], Wl[D * PK];       // W^T [D][64]
+  __bf16 Sh[32 * PW], Sl[32 * PW];     // dS^T [32][D]
+  __bf16 Oh[32 * PK], Ol[32 * PK];     // do^T [32][64]
+  __bf16 Vh[32 * PK], Vl[32 * PK];     // (-dv~)^T [32][64]
+  float GC[D];
+};
+
 template <int D, int DO, bool WS16>
-__global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_rscan_kernel(BwdArgs a) {
+__device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLds<D>& L) {
   constexpr int EF = BwdWs<WS16>::F;    // lambda k, Aqk, gamma q, W in
   constexpr int NTH = ScanThreads<D>::value;
   constexpr int NS = D / 32;
   constexpr int NST = (D / 8) / (NTH / 64);
   static_assert(NST >= 1, "at least one state tile per wave");
-  constexpr int PW = D + 8;     // bf16 pitch of rows whose K index is a channel
-  constexpr int PK = kC + 8;    // bf16 pitch of rows whose K index is a chunk row
-  __shared__ __attribute__((aligned(16))) __bf16 sLh[kC * PW], sLl[kC * PW];   // lambda k [64][D]
-  __shared__ __attribute__((aligned(16))) __bf16 sAh[kC * PK], sAl[kC * PK];   // Aqk^T [64][64]
-  __shared__ __attribute__((aligned(16))) __bf16 sQh[D * PK], sQl[D * PK];     // (gamma q)^T [D][64]
-  __shared__ __attribute__((aligned(16))) __bf16 sWh[D * PK], sWl[D * PK];     // W^T [D][64]
-  __shared__ __attribute__((aligned(16))) __bf16 sSh[32 * PW], sSl[32 * PW];   // dS^T [32][D]
-  __shared__ __attribute__((aligned(16))) __bf16 sOh[32 * PK], sOl[32 * PK];   // do^T [32][64]
-  __shared__ __attribute__((aligned(16))) __bf16 sVh[32 * PK], sVl[32 * PK];   // (-dv~)^T [32][64]
-  __shared__ float sGC[D];
+  constexpr int PW = RscanLds<D>::PW, PK = RscanLds<D>::PK;
+  __bf16 *const sLh = L.Lh, *const sLl = L.Ll, *const sAh = L.Ah, *const sAl = L.Al;
+  __bf16 *const sQh = L.Qh, *const sQl = L.Ql, *const sWh = L.Wh, *const sWl = L.Wl;
+  __bf16 *const sSh = L.Sh, *const sSl = L.Sl, *const sOh = L.Oh, *const sOl = L.Ol;
+  __bf16 *const sVh = L.Vh, *const sVl = L.Vl;
+  float* const sGC = L.GC;
   const int t = threadIdx.x, wv = t >> 6, l = t & 63, r = l & 15, gq = l >> 4;
   const int H = a.H;
   int chain, split;
-  if (!scan_slot<NS>(a.B * H, chain, split)) return;   // uniform per workgroup
+  if (!scan_slot<NS>(block, a.B * H, chain, split)) return;   // uniform per workgroup
   const int b = chain / H, h = chain - b * H;
   const int c0 = 32 * split;
   const int mt = wv >> 1, ct = wv & 1;                  // this wave's dv~ tile (waves 0-7: 8 tiles)
@@ -1605,13 +1622,19 @@ __device__ __forceinline__ void rs_chain(const BwdArgs& a, unsigned char (*buf)[
   }
 }
 
+template <int D>
+struct alignas(16) Rscan16Lds {
+  unsigned char buf[2][RsLayout<D>::BYTES];
+  unsigned char stg[2][RsLayout<D>::STG];
+};
+
 template <int D, int DO>
-__global__ __launch_bounds__(64 * (2 + kRsProducers), 1) void kda_bwd_rscan16_kernel(BwdArgs a) {
+__device__ __forceinline__ void rscan16_block(const BwdArgs& a, int block, Rscan16Lds<D>& L) {
   constexpr int NS = D / 32;
-  __shared__ __attribute__((aligned(16))) unsigned char buf[2][RsLayout<D>::BYTES];
-  __shared__ __attribute__((aligned(16))) unsigned char stg[2][RsLayout<D>::STG];
+  auto& buf = L.buf;
+  auto& stg = L.stg;
   int chain, split;
-  if (!scan_slot<NS>(a.B * a.H, chain, split)) return;   // uniform per workgroup
+  if (!scan_slot<NS>(block, a.B * a.H, chain, split)) return;   // uniform per workgroup
   const int b = chain / a.H, h = chain - b * a.H;
   const int c0 = 32 * split;
   const int wave = threadIdx.x >> 6;
@@ -1860,12 +1883,18 @@ __device__ __forceinline__ void fs_chain(const BwdArgs& a, unsigned char (*buf)[
 }
 
 template <int D>
-__global__ __launch_bounds__(64 * (2 + kFsProducers), 1) void kda_bwd_fscan16_kernel(BwdArgs a) {
+struct alignas(16) Fscan16Lds {
+  unsigned char buf[2][FsLayout<D>::BYTES];
+  unsigned char stg[2][FsLayout<D>::STG];
+};
+
+template <int D>
+__device__ __forceinline__ void fscan16_block(const BwdArgs& a, int block, Fscan16Lds<D>& L) {
   constexpr int NS = D / 32;
-  __shared__ __attribute__((aligned(16))) unsigned char buf[2][FsLayout<D>::BYTES];
-  __shared__ __attribute__((aligned(16))) unsigned char stg[2][FsLayout<D>::STG];
+  auto& buf = L.buf;
+  auto& stg = L.stg;
   int chain, split;
-  if (!scan_slot<NS>(a.B * a.H, chain, split)) return;   // uniform per workgroup
+  if (!scan_slot<NS>(block, a.B * a.H, chain, split)) return;   // uniform per workgroup
   const int b = chain / a.H, h = chain - b * a.H;
   const int c0 = 32 * split;
   switch (threadIdx.x >> 6) {
@@ -1876,6 +1905,36 @@ __global__ __launch_bounds__(64 * (2 + kFsProducers), 1) void kda_bwd_fscan16_ke
     case 4: fs_producer<D, 2>(a, buf, stg, b, h, split); break;
     default: fs_producer<D, 3>(a, buf, stg, b, h, split); break;
   }
+}
+
+// ---------------------------------------------------------------------------
+// Both scans in one launch: neither reads what the other writes (the forward
+// scan gives S and v~ to the chunk kernel, the reverse scan dS' and dv~), and
+// each is a serial chain on its own workgroups, so a call whose chains leave
+// CUs idle runs them side by side.  The reverse scan's workgroups, the longer
+// ones, come first: with more workgroups than CUs the forward ones fill in as
+// CUs free up.  Whole backward against the two scans one after the other
+// (d = 128, 16-bit inputs): 24 chains of 128 chunks 1 137 -> 974 us, 48 of 64
+// 935 -> 896, 64 of 64 1 120 -> 1 117; fp32, 16 of 16 176 -> 138; the same bits.
+// ---------------------------------------------------------------------------
+static_assert(kRsProducers == kFsProducers, "one workgroup size");
+
+template <int D, int DO>
+__global__ __launch_bounds__(64 * (2 + kRsProducers), 1) void kda_bwd_scans16_kernel(BwdArgs a, int nblk) {
+  constexpr size_t N = sizeof(Rscan16Lds<D>) > sizeof(Fscan16Lds<D>) ? sizeof(Rscan16Lds<D>) : sizeof(Fscan16Lds<D>);
+  __shared__ __attribute__((aligned(16))) unsigned char sm[N];
+  const int x = blockIdx.x;
+  if (x < nblk) rscan16_block<D, DO>(a, x, *reinterpret_cast<Rscan16Lds<D>*>(sm));
+  else fscan16_block<D>(a, x - nblk, *reinterpret_cast<Fscan16Lds<D>*>(sm));
+}
+
+template <int D, int DO>
+__global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_scans_kernel(BwdArgs a, int nblk) {
+  constexpr size_t N = sizeof(RscanLds<D>) > sizeof(FscanLds<D>) ? sizeof(RscanLds<D>) : sizeof(FscanLds<D>);
+  __shared__ __attribute__((aligned(16))) unsigned char sm[N];
+  const int x = blockIdx.x;
+  if (x < nblk) rscan_block<D, DO, false>(a, x, *reinterpret_cast<RscanLds<D>*>(sm));
+  else fscan_block<D, false>(a, x - nblk, *reinterpret_cast<FscanLds<D>*>(sm));
 }
 
 // A 16 x 16 accumulator tile (lane (r, gq): rows 4 gq + i, column r) into
@@ -2696,17 +2755,11 @@ hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((kda_bwd_prep_kernel<D, DTQ, DTG>), dim3(chunk_heads), dim3(kPrepThreads), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int scan_grid = (chains + 7) / 8 * 8 * (D / 32);
+  const int scan_grid = (chains + 7) / 8 * 8 * (D / 32);   // workgroups of either scan
   if constexpr (DTQ != 0)
-    hipLaunchKernelGGL((kda_bwd_fscan16_kernel<D>), dim3(scan_grid), dim3(64 * (2 + kFsProducers)), 0, s, a);
+    hipLaunchKernelGGL((kda_bwd_scans16_kernel<D, DO>), dim3(2 * scan_grid), dim3(64 * (2 + kRsProducers)), 0, s, a, scan_grid);
   else
-    hipLaunchKernelGGL((kda_bwd_fscan_kernel<D, false>), dim3(scan_grid), dim3(ScanThreads<D>::value), 0, s, a);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if constexpr (DTQ != 0)
-    hipLaunchKernelGGL((kda_bwd_rscan16_kernel<D, DO>), dim3(scan_grid), dim3(64 * (2 + kRsProducers)), 0, s, a);
-  else
-    hipLaunchKernelGGL((kda_bwd_rscan_kernel<D, DO, false>), dim3(scan_grid), dim3(ScanThreads<D>::value), 0, s, a);
+    hipLaunchKernelGGL((kda_bwd_scans_kernel<D, DO>), dim3(2 * scan_grid), dim3(ScanThreads<D>::value), 0, s, a, scan_grid);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((kda_bwd_chunk_kernel<D, DTQ, DTG, DO>), dim3(chunk_heads), dim3(ChunkThreads<D>::value), 0, s, a);
