@@ -412,73 +412,60 @@ __device__ __forceinline__ int fa_frag(int it, int kb) { return (it < 2) ? 2 * i
 // The chunk's channels are taken in halves of 64 (d = 128) so the shared
 // memory fits two workgroups per CU: the scores accumulate over the halves in
 // registers, T = (I+L)^-1 is built once, and W, U are formed per half of
-// their columns (the last half's k and G still staged, the other reloaded).
+// their columns.
+//
+// Per half, thread (channel d = t % 64, rows 8 s .. 8 s + 7, s = t / 64) owns a
+// column segment of q, k, g: it forms G there, and from G everything with a
+// decay in it, once per element: the scores' operands q 2^(G - Ga), k 2^(G -
+// Ga), k 2^(Ge - G) (Ga, Ge: G of the row tile's first and last row; into LDS,
+// over the raw rows), gamma q, lambda k (stored as the scans' fragments) and
+// gamma k (kept in registers for W).  The scores read their operands 16 bytes
+// at a time, four channels per lane for four v_mfma_f32_16x16x4f32, and a tile
+// pair costs one factor 2^(Ga_R - Ge_s) per channel.
+// Bound by its phases' latencies beside its traffic (200 KiB per chunk-head at
+// d = 128, 16-bit inputs: 160 us of 4 096 chunk-heads at the copy rate).  4 096
+// chunk-heads, 16-bit inputs: 267 us with each decay factor formed per operand
+// and tile pair, element-wise LDS reads and the first half's k, g staged again
+// for W; 212 now; 3 072 with the seam's gates 227 -> 167; 256 in fp32 29 -> 24.
 template <int D, int DTQ, int DTG>
 __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a) {
-  constexpr int EF = BwdWs<DTQ != 0>::F;   // gamma q, lambda k, Aqk, T, W, U
+  constexpr int EF = BwdWs<DTQ != 0>::F;   // gamma q, lambda k, Aqk, T, W
   constexpr bool ALPHA = DTG == kAlphaGates;
   constexpr int GT = ALPHA ? 0 : DTG;  // element type of g
   constexpr int HD = 64;              // channels per half
   constexpr int NHALF = D / HD;
-  // [64][HD] pitch: row fragments conflict-free (rows 4 banks apart), rows
-  // 16-byte aligned for the diagonal tiles' vector reads
+  // [64][64] pitch: rows 4 banks apart and 16-byte aligned
   constexpr int P = HD + 4;
-  constexpr int PC = kC + 1;
-  static_assert(kC * PC <= kC * P, "T shares sQ's buffer");
-  __shared__ __attribute__((aligned(16))) float sQ[kC * P], sK[kC * P], sG[kC * P];   // one channel half; sQ then holds T
-  __shared__ float sL[kC * PC];       // L, then one half of beta*v
-  __shared__ float sTmp[768];         // the triangular inversion's scratch
+  __shared__ __attribute__((aligned(16))) float sQ[kC * P];   // q, then q 2^(G - Ga); T after the scores
+  __shared__ __attribute__((aligned(16))) float sK[kC * P];   // k, then k 2^(G - Ga); (beta gamma k)^T for W
+  __shared__ __attribute__((aligned(16))) float sG[kC * P];   // g, then k 2^(Ge - G); v for U
+  __shared__ __attribute__((aligned(16))) float sL[kC * P];   // L; (beta v)^T for U
+  __shared__ __attribute__((aligned(16))) float sGa[4 * HD], sGe[4 * HD];
+  __shared__ float sTmp[768];         // segment sums; the triangular inversion's scratch
   __shared__ float sB[kC];
+  __shared__ int sFar[NHALF];         // a diagonal tile of the half decays past the anchor's range
   constexpr int NTH = kPrepThreads;
+  static_assert(NTH == 8 * HD && kC == 64, "eight 8-row segments per channel");
   const int t = threadIdx.x;
-  const int wv = t >> 6, l = t & 63, r16 = l & 15, gq = l >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63, r16 = l & 15, gq = l >> 4;
   const int H = a.H;
   const int u = blockIdx.x / H, h = blockIdx.x - u * H;
   const ChunkRows cr = chunk_rows(a, u);
   const int64_t ch = static_cast<int64_t>(u) * H + h;
   float* const sT = sQ;
-
-  // k and the in-chunk inclusive cumsum of g (log2 units) of channel half c0
-  // (both tiles' loads issued before either is stored)
-  auto stage_k_g = [&](int c0) {
-    InTile<DTQ, D, HD, NTH> ik;
-    InTile<GT, D, HD, NTH> ig;
-    ik.fetch(a.k, cr.row0, cr.len, H, h, c0);
-    ig.fetch(a.g, cr.row0, cr.len, H, h, c0);
-    ik.template put<P>(sK, 1.f);
-    ig.template put<P, ALPHA>(sG, 1.f, cr.len);
-  };
-  // every thread: channel t % HD, rows 8 s .. 8 s + 7 (s = t / HD): the
-  // prefix over its rows, then the sums of the segments above it (through
-  // sTmp, which the triangular inversion alone uses otherwise); ends with a
-  // barrier before which sG must not be read
-  static_assert(NTH == 8 * HD && kC == 64, "eight 8-row segments per channel");
-  auto cumsum_g = [&]() {
-    const int d = t & (HD - 1), s8 = t / HD;
-    float x[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = sG[(8 * s8 + j) * P + d];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) x[j] += x[j - 1];
-    sTmp[s8 * HD + d] = x[7];
-    __syncthreads();
-    float pre = 0.f;
-    for (int k = 0; k < s8; ++k) pre += sTmp[k * HD + d];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sG[(8 * s8 + j) * P + d] = (x[j] + pre) * kLog2e;
-  };
+  const int d0 = t & (HD - 1), s8 = wv, tile = wv >> 1;   // this thread's column segment (in row tile `tile`)
 
   // scores: Aqk (c >= i) to the workspace, L = beta_c Akk (c > i) to LDS,
   // accumulated over the channel halves on the matrix cores, one 16 x 16 tile
   // pair per wave: waves 0..5 the off-diagonal pairs (row tile R > key tile
-  // s), waves 6 and 7 two diagonal tiles each.  The decay is factored at the
-  // row tile's first row a, 2^(G_c - G_i) = 2^(G_c - G_a) 2^(G_a - G_i), and
-  // applied to each operand element as it is read: both factors <= 1 off the
-  // diagonal; on it the key factor is >= 1, up to the tile's decay, and pairs
-  // where the product would exceed 1 are masked.  A diagonal tile that decays
-  // by more than 2^-kDiagAnchorLog2 in a channel of the half takes
-  // 2^(G_c - G_i) per element for that half instead (lane (r, gq) forming its
-  // own four outputs, rows 4 gq + e, key r).
+  // s), waves 6 and 7 two diagonal tiles each.  The decay of a pair is
+  // 2^(G_c - Ga_R) 2^(Ga_R - Ge_s) 2^(Ge_s - G_i); the outer factors are <= 1
+  // and in the operands, the middle one is <= 1 off the diagonal and, on it,
+  // >= 1, up to the tile's decay (pairs whose product would exceed 1 are
+  // masked).  A diagonal tile that decays by more than 2^-kDiagAnchorLog2 in a
+  // channel of the half takes 2^(G_c - G_i) per element for that half instead
+  // (lane (r, gq) forming its own four outputs, rows 4 gq + e, key r), before
+  // the operands replace q, k, G.
   const int R_off = (wv < 1) ? 1 : (wv < 3) ? 2 : 3;
   const int sk_off = wv - R_off * (R_off - 1) / 2;
   const int NPAIR = (wv < 6) ? 1 : 2;   // wave-uniform
@@ -489,18 +476,20 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
   f4 accA[2], accL[2];
 #pragma unroll
   for (int pi = 0; pi < 2; ++pi) accA[pi] = accL[pi] = f4{0.f, 0.f, 0.f, 0.f};
+  float kg[NHALF][8];                 // gamma k of this thread's segment
   // the next half's q, k, g and beta, loaded during this half's scores
   InTile<DTQ, D, HD, NTH> nq, nk;
   InTile<GT, D, HD, NTH> ng;
-  float nb = 0.f;
   auto fetch_half = [&](int c0) {
     nq.fetch(a.q, cr.row0, cr.len, H, h, c0);
     nk.fetch(a.k, cr.row0, cr.len, H, h, c0);
     ng.fetch(a.g, cr.row0, cr.len, H, h, c0);
-    const int tb = t & (kC - 1);
-    nb = ld_beta<DTG>(a.beta, (cr.row0 + (tb < cr.len ? tb : 0)) * H + h);
   };
   fetch_half(0);
+  float nb = 0.f;
+  if (t < NHALF) sFar[t] = 0;
+  if (t < kC) nb = ld_beta<DTG>(a.beta, (cr.row0 + (t < cr.len ? t : 0)) * H + h);
+#pragma unroll
   for (int hf = 0; hf < NHALF; ++hf) {
     const int c0 = HD * hf;
     if (hf > 0) __syncthreads();      // the previous half's reads are done
@@ -509,47 +498,124 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
     ng.template put<P, ALPHA>(sG, 1.f, cr.len);
     if (hf == 0 && t < kC) sB[t] = (t < cr.len) ? nb : 0.f;
     __syncthreads();
-    cumsum_g();
+    // G of the segment (log2 units): its prefix, plus the sums of the segments above
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = sG[(8 * s8 + j) * P + d0];
+    const float first = x[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) x[j] += x[j - 1];
+    sTmp[s8 * HD + d0] = x[7];
+    if ((s8 & 1) == 0) sGa[tile * HD + d0] = first;   // (g of the tile's first row, made G below)
     __syncthreads();
+    float pre = 0.f, all = 0.f, mid = 0.f, end = 0.f;   // sums above the segment, of the chunk, up to the tile, through it
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      if (m == s8) pre = all;
+      if (m == 2 * tile) mid = all;
+      all += sTmp[m * HD + d0];
+      if (m == 2 * tile + 1) end = all;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = (x[j] + pre) * kLog2e;
+    const float ga = (mid + sGa[tile * HD + d0]) * kLog2e;
+    const float ge = (s8 & 1) ? x[7] : end * kLog2e;
+    const float gz = (s8 == 7) ? x[7] : all * kLog2e;
+    if (__any(ga - ge > kDiagAnchorLog2) && l == 0) sFar[hf] = 1;
+    __syncthreads();                  // (also: sGa's first rows are read)
+    if ((s8 & 1) == 0) sGa[tile * HD + d0] = ga;
+    else sGe[tile * HD + d0] = ge;
+    unsigned far = 0;   // diagonal tiles of this wave done per element (bit pi)
+    if (sFar[hf] != 0) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sG[(8 * s8 + j) * P + d0] = x[j];
+      __syncthreads();
+      if (wv >= 6) {
+#pragma unroll
+        for (int pi = 0; pi < 2; ++pi) {
+          const int a0 = 16 * (2 * (wv - 6) + pi), i = a0 + r16;
+          if (!__any(sG[a0 * P + l] - sG[(a0 + 15) * P + l] > kDiagAnchorLog2)) continue;
+          far |= 1u << pi;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int c = a0 + 4 * gq + e;
+            if (r16 > 4 * gq + e) continue;   // above the diagonal (masked below)
+            float sA = 0.f, sL4 = 0.f;
+#pragma unroll 2
+            for (int d4 = 0; d4 < HD; d4 += 4) {
+              const f4 kI = *reinterpret_cast<const f4*>(&sK[i * P + d4]), gI = *reinterpret_cast<const f4*>(&sG[i * P + d4]);
+              const f4 gC = *reinterpret_cast<const f4*>(&sG[c * P + d4]), qC = *reinterpret_cast<const f4*>(&sQ[c * P + d4]);
+              const f4 kC4 = *reinterpret_cast<const f4*>(&sK[c * P + d4]);
+#pragma unroll
+              for (int y = 0; y < 4; ++y) {
+                const float ki = kI[y] * ex2(gC[y] - gI[y]);
+                sA = fmaf(qC[y], ki, sA);
+                sL4 = fmaf(kC4[y], ki, sL4);
+              }
+            }
+            accA[pi][e] += sA;
+            accL[pi][e] += sL4;
+          }
+        }
+      }
+      __syncthreads();
+    }
     {
+      // the segment's operands over q, k, g in LDS; gamma q, lambda k stored
+      const float fa = ex2(ga), fe = ex2(gz - ge);
+      h4 vq[2], vl[2];
+      f4 wq[2], wl[2];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int o = (8 * s8 + j) * P + d0;
+        const float up = ex2(x[j] - ga), q = sQ[o] * up, k = sK[o], ku = k * up, kd = k * ex2(ge - x[j]);
+        sQ[o] = q;
+        sK[o] = ku;
+        sG[o] = kd;
+        kg[hf][j] = ku * fa;
+        wq[j >> 2][j & 3] = q * fa;
+        wl[j >> 2][j & 3] = kd * fe;
+        vq[j >> 2][j & 3] = static_cast<_Float16>(wq[j >> 2][j & 3]);
+        vl[j >> 2][j & 3] = static_cast<_Float16>(wl[j >> 2][j & 3]);
+      }
       if constexpr (EF == 0) {
-        // gamma q and lambda k, row-major
-        const int64_t base = ch * kC * D + c0;
-        constexpr int V4 = HD / 4;      // float4 groups per row
-        for (int e = t; e < kC * V4; e += NTH) {
-          const int c = e / V4, d = 4 * (e - c * V4);
-          const float4 gl = *reinterpret_cast<const float4*>(&sG[c * P + d]);
-          const float4 gz = *reinterpret_cast<const float4*>(&sG[(kC - 1) * P + d]);
-          const float4 qv = *reinterpret_cast<const float4*>(&sQ[c * P + d]);
-          const float4 kv = *reinterpret_cast<const float4*>(&sK[c * P + d]);
-          const float4 qg = make_float4(ex2(gl.x) * qv.x, ex2(gl.y) * qv.y, ex2(gl.z) * qv.z, ex2(gl.w) * qv.w);
-          const float4 kl = make_float4(ex2(gz.x - gl.x) * kv.x, ex2(gz.y - gl.y) * kv.y, ex2(gz.z - gl.z) * kv.z,
-                                        ex2(gz.w - gl.w) * kv.w);
-          ws_st4<EF>(a.QG, base + c * D + d, qg);
-          ws_st4<EF>(a.KL, base + c * D + d, kl);
+        // row-major
+        const int64_t base = (ch * kC + 8 * s8) * D + c0 + d0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          a.QG[base + j * D] = wq[j >> 2][j & 3];
+          a.KL[base + j * D] = wl[j >> 2][j & 3];
         }
       } else {
-        // the reverse scan's A fragments of this half's channels, one lane
-        // fragment per thread each (the slot order of kda_internal.h)
-        static_assert(NTH == 512 && HD == 64, "one (gamma q)^T and one lambda k lane fragment per thread");
-        const int ln = t & 63, rr = ln & 15, g4 = ln >> 4, hi = (t >> 6) & 1, tt = t >> 7;
-        h8 vq, vl, vt;
+        // (gamma q)^T and (lambda k)^T fragments (the slot order of
+        // kda_internal.h): channel tile dt, K step s8 / 4, half (s8 % 4) / 2,
+        // row groups 2 (s8 % 2) and the next
+        const int64_t f = ((ch * (D / 16) + (c0 + d0) / 16) * 2 + (s8 >> 2)) * 64 + (d0 & 15) + 32 * (s8 & 1);
+        const int hh = 4 * ((s8 >> 1) & 1);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          // (gamma q)^T and (lambda k)^T: channel tile tt of the half, K step hi over the rows
-          const int c = 32 * hi + 4 * g4 + (e & 3) + 16 * (e >> 2), dq = 16 * tt + rr;
-          vq[e] = static_cast<_Float16>(ex2(sG[c * P + dq]) * sQ[c * P + dq]);
-          vt[e] = static_cast<_Float16>(ex2(sG[(kC - 1) * P + dq] - sG[c * P + dq]) * sK[c * P + dq]);
-          // lambda k: row tile tt, K step hi over the half's channels
-          const int row = 16 * tt + rr, dl = 32 * hi + 4 * g4 + (e & 3) + 16 * (e >> 2);
-          vl[e] = static_cast<_Float16>(ex2(sG[(kC - 1) * P + dl] - sG[row * P + dl]) * sK[row * P + dl]);
+        for (int g2 = 0; g2 < 2; ++g2) {
+          *reinterpret_cast<h4*>(static_cast<_Float16*>(a.FQ) + (f + 16 * g2) * 8 + hh) = vq[g2];
+          *reinterpret_cast<h4*>(static_cast<_Float16*>(a.FLT) + (f + 16 * g2) * 8 + hh) = vl[g2];
         }
-        const int dt = (c0 >> 4) + tt, j = (c0 >> 5) + hi;
-        *reinterpret_cast<h8*>(static_cast<_Float16*>(a.FQ) + (((ch * (D / 16) + dt) * 2 + hi) * 64 + ln) * 8) = vq;
-        *reinterpret_cast<h8*>(static_cast<_Float16*>(a.FLT) + (((ch * (D / 16) + dt) * 2 + hi) * 64 + ln) * 8) = vt;
-        *reinterpret_cast<h8*>(static_cast<_Float16*>(a.FL) + (((ch * 4 + tt) * (D / 32) + j) * 64 + ln) * 8) = vl;
       }
-      if (t < HD) a.GCV[ch * D + c0 + t] = ex2(sG[(kC - 1) * P + t]);
+      if (s8 == 7) a.GCV[ch * D + c0 + d0] = ex2(gz);
+    }
+    __syncthreads();
+    if constexpr (EF != 0) {
+      // lambda k fragments (rows as M): row tile tt, K step hi over the half's
+      // channels, one lane fragment per thread
+      static_assert(NTH == 512 && HD == 64, "one lambda k lane fragment per thread");
+      const int hi = wv & 1, tt = wv >> 1, row = 16 * tt + r16;
+      h8 v;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int dl = 32 * hi + 4 * gq + 16 * p;
+        const f4 kd = *reinterpret_cast<const f4*>(&sG[row * P + dl]);
+        const f4 ge4 = *reinterpret_cast<const f4*>(&sGe[tt * HD + dl]), gz4 = *reinterpret_cast<const f4*>(&sGe[3 * HD + dl]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * p + e] = static_cast<_Float16>(kd[e] * ex2(gz4[e] - ge4[e]));
+      }
+      *reinterpret_cast<h8*>(static_cast<_Float16*>(a.FL) + (((ch * 4 + tt) * (D / 32) + (c0 >> 5) + hi) * 64 + l) * 8) = v;
     }
     if (hf + 1 < NHALF) fetch_half(c0 + HD);
 #pragma unroll
@@ -557,54 +623,27 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
       if (pi >= NPAIR) break;
       int R, sk;
       pair_rs(pi, R, sk);
-      const int a0 = 16 * R, i = 16 * sk + r16;
-      // a diagonal tile decaying past the anchor's range in a channel of the half
-      bool far = false;
-      if (R == sk) {
+      if (R == sk && (far >> pi & 1)) continue;
+      const int ro = (16 * R + r16) * P + 4 * gq, ko = (16 * sk + r16) * P + 4 * gq;
 #pragma unroll
-        for (int k = 0; k < HD / 4; ++k) {
-          const int d = 4 * k + gq;
-          far |= sG[a0 * P + d] - sG[(a0 + 15) * P + d] > kDiagAnchorLog2;
-        }
-      }
-      if (!__any(far)) {
-#pragma unroll 8
-        for (int k = 0; k < HD / 4; ++k) {
-          const int d = 4 * k + gq;
-          const float ga = sG[a0 * P + d];
-          const float fa = ex2(sG[(a0 + r16) * P + d] - ga);
-          const float bk = sK[i * P + d] * ex2(ga - sG[i * P + d]);
-          accA[pi] = mfma4(sQ[(a0 + r16) * P + d] * fa, bk, accA[pi]);
-          accL[pi] = mfma4(sK[(a0 + r16) * P + d] * fa, bk, accL[pi]);
-        }
-      } else {
+      for (int j = 0; j < HD / 16; ++j) {
+        const f4 qu = *reinterpret_cast<const f4*>(&sQ[ro + 16 * j]), ku = *reinterpret_cast<const f4*>(&sK[ro + 16 * j]);
+        f4 kd = *reinterpret_cast<const f4*>(&sG[ko + 16 * j]);
+        const f4 ga4 = *reinterpret_cast<const f4*>(&sGa[R * HD + 16 * j + 4 * gq]);
+        const f4 ge4 = *reinterpret_cast<const f4*>(&sGe[sk * HD + 16 * j + 4 * gq]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kd[e] *= ex2(ga4[e] - ge4[e]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int c = a0 + 4 * gq + e;
-          if (r16 > 4 * gq + e) continue;   // above the diagonal (masked below)
-          float sA = 0.f, sL4 = 0.f;
-#pragma unroll 2
-          for (int d4 = 0; d4 < HD; d4 += 4) {
-            const float4 kI = *reinterpret_cast<const float4*>(&sK[i * P + d4]);
-            const float4 gI = *reinterpret_cast<const float4*>(&sG[i * P + d4]);
-            const float4 gC = *reinterpret_cast<const float4*>(&sG[c * P + d4]);
-            const float4 qC = *reinterpret_cast<const float4*>(&sQ[c * P + d4]);
-            const float4 kC4 = *reinterpret_cast<const float4*>(&sK[c * P + d4]);
-            const float ki[4] = {kI.x * ex2(gC.x - gI.x), kI.y * ex2(gC.y - gI.y), kI.z * ex2(gC.z - gI.z),
-                                 kI.w * ex2(gC.w - gI.w)};
-            const float qc[4] = {qC.x, qC.y, qC.z, qC.w}, kc[4] = {kC4.x, kC4.y, kC4.z, kC4.w};
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              sA = fmaf(qc[x], ki[x], sA);
-              sL4 = fmaf(kc[x], ki[x], sL4);
-            }
-          }
-          accA[pi][e] += sA;
-          accL[pi][e] += sL4;
+          accA[pi] = mfma4(qu[e], kd[e], accA[pi]);
+          accL[pi] = mfma4(ku[e], kd[e], accL[pi]);
         }
       }
     }
   }
+  // the first W/U pass's v half, loaded until the scores are out of LDS
+  InTile<DTQ, D, HD, NTH> iv;
+  iv.fetch(a.v, cr.row0, cr.len, H, h, 0);
   const int64_t aq0 = ch * kC * kC;
 #pragma unroll
   for (int pi = 0; pi < 2; ++pi) {
@@ -619,22 +658,21 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
       const bool diag = R == sk;
       vA[e] = (!diag || r16 <= 4 * gq + e) ? accA[pi][e] : 0.f;   // Aqk: i <= c
       if constexpr (EF == 0) ws_st<EF>(a.AQ, aq0 + c * kC + i, vA[e]);
-      sL[c * PC + i] = (!diag || r16 < 4 * gq + e) ? accL[pi][e] * sB[c] : 0.f;   // L: i < c
+      sL[c * P + i] = (!diag || r16 < 4 * gq + e) ? accL[pi][e] * sB[c] : 0.f;   // L: i < c
     }
     if constexpr (EF != 0)   // Aqk^T fragment (key tile sk, K step R / 2), half R % 2
       *reinterpret_cast<uint2*>(static_cast<u16*>(a.FA) + ((ch * 6 + fa_frag(sk, R >> 1)) * 64 + l) * 8 +
                                 4 * (R & 1)) = pack_f16x4(vA);
   }
-  // blocks above the diagonal: zero
-  for (int e = t; e < 6 * 256; e += NTH) {
-    const int blk = e >> 8, rc = (e >> 4) & 15, ri = e & 15;
-    const int R = (blk < 3) ? 0 : (blk < 5) ? 1 : 2;             // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
-    const int sk = (blk < 3) ? blk + 1 : (blk < 5) ? blk - 1 : 3;
-    const int c = 16 * R + rc, i = 16 * sk + ri;
-    if constexpr (EF == 0) ws_st<EF>(a.AQ, aq0 + c * kC + i, 0.f);
-    sL[c * PC + i] = 0.f;
-  }
-  if constexpr (EF != 0) {
+  if constexpr (EF == 0) {
+    // blocks above the diagonal: zero
+    for (int e = t; e < 6 * 256; e += NTH) {
+      const int blk = e >> 8, rc = (e >> 4) & 15, ri = e & 15;
+      const int R = (blk < 3) ? 0 : (blk < 5) ? 1 : 2;             // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
+      const int sk = (blk < 3) ? blk + 1 : (blk < 5) ? blk - 1 : 3;
+      ws_st<EF>(a.AQ, aq0 + (16 * R + rc) * kC + 16 * sk + ri, 0.f);
+    }
+  } else {
     // the zero halves of the stored Aqk^T fragments: key tile 1 against row
     // tile 0, key tile 3 against row tile 2
     if (t < 128)
@@ -644,58 +682,68 @@ __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a
   }
   __syncthreads();
 
-  // T = (I + L)^-1 (into sQ's buffer: q is no longer read); the first W/U
-  // pass's v half is loaded during the inversion
-  InTile<DTQ, D, HD, NTH> iv;
-  iv.fetch(a.v, cr.row0, cr.len, H, h, HD * (NHALF - 1));
-  invert_unit_lower64<PC, NTH>(sL, sT, sTmp);
+  // W = T (beta gamma k), U = T (beta v) on the matrix cores, per half of
+  // their columns, the right sides transposed in LDS so both operands are
+  // 16-byte reads of four K values; wave wv owns row tile wv / 2 and column
+  // tiles (wv % 2) HD/32 + q of the half.  The first half's beta gamma k and v
+  // go to LDS here, T = (I + L)^-1 goes into sQ's buffer.
+  float bs[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) bs[j] = sB[8 * s8 + j];
+  auto put_col = [&](float* dst, const float (&y)[8]) {   // beta times the segment, transposed
+    float* o = dst + d0 * P + 8 * s8;
+    *reinterpret_cast<f4*>(o) = f4{bs[0] * y[0], bs[1] * y[1], bs[2] * y[2], bs[3] * y[3]};
+    *reinterpret_cast<f4*>(o + 4) = f4{bs[4] * y[4], bs[5] * y[5], bs[6] * y[6], bs[7] * y[7]};
+  };
+  put_col(sK, kg[0]);
+  iv.template put<P>(sG, 1.f);
+  if constexpr (NHALF > 1) iv.fetch(a.v, cr.row0, cr.len, H, h, HD);   // the next half's, during the inversion
+  invert_unit_lower64<P, NTH>(sL, sT, sTmp);
   {
     static_assert(kC * kC == 8 * NTH, "eight entries of T per thread");
     const int c = t >> 3, i0 = 8 * (t & 7);
-    const float* row = sT + c * PC + i0;
+    const f4 lo = *reinterpret_cast<const f4*>(sT + c * P + i0), hi = *reinterpret_cast<const f4*>(sT + c * P + i0 + 4);
     const int64_t o = ch * kC * kC + c * kC + i0;
-    ws_st4<EF>(a.TM, o, make_float4(row[0], row[1], row[2], row[3]));
-    ws_st4<EF>(a.TM, o + 4, make_float4(row[4], row[5], row[6], row[7]));
+    ws_st4<EF>(a.TM, o, make_float4(lo[0], lo[1], lo[2], lo[3]));
+    ws_st4<EF>(a.TM, o + 4, make_float4(hi[0], hi[1], hi[2], hi[3]));
   }
-  // W = T (beta gamma k), U = T (beta v) on the matrix cores, per half of
-  // their columns (the last half first: its k and G are still staged); wave
-  // wv owns row tile wv / 2 and column tiles (wv % 2) HD/32 + q of the half
-  float* const sV = sL;               // beta * v of the half, pitch PC
-  for (int pass = 0; pass < NHALF; ++pass) {
-    const int c0 = HD * (NHALF - 1 - pass);
-    if (pass > 0) {
-      __syncthreads();                // the previous pass's products are done
-      iv.fetch(a.v, cr.row0, cr.len, H, h, c0);   // in flight during the k, g staging
-      stage_k_g(c0);
-      __syncthreads();
-      cumsum_g();
+#pragma unroll
+  for (int hf = 0; hf < NHALF; ++hf) {
+    const int c0 = HD * hf;
+    if (hf > 0) {
+      __syncthreads();                // the previous half's products are done
+      put_col(sK, kg[hf]);
     }
-    iv.template put<PC>(sV, 1.f);
+    float y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[j] = sG[(8 * s8 + j) * P + d0];
+    put_col(sL, y);
     __syncthreads();
-    for (int e = t; e < kC * HD; e += NTH) {
-      const int c = e / HD, d = e - c * HD;
-      sK[c * P + d] *= sB[c] * ex2(sG[c * P + d]);
-      sV[c * PC + d] *= sB[c];
-    }
-    __syncthreads();
+    if (hf + 1 < NHALF) iv.template put<P>(sG, 1.f);
     constexpr int NDT = HD / 32;
     const int mt = wv >> 1, dg = wv & 1;
-    const int mts = __builtin_amdgcn_readfirstlane(mt);
     f4 accW[NDT], accU[NDT];
 #pragma unroll
     for (int q = 0; q < NDT; ++q)
 #pragma unroll
       for (int e = 0; e < 4; ++e) accW[q][e] = accU[q][e] = 0.f;
-    // T[c][i] is zero for i > c: row tile mt needs K steps i < 16 (mt + 1) only
-#pragma unroll 4
-    for (int k = 0; k < 4 * (mts + 1); ++k) {
-      const float at = sT[(16 * mt + r16) * PC + 4 * k + gq];
+    // T[c][i] is zero for i > c: row tile mt needs the K blocks up to its own
+    for (int j = 0; j <= mt; ++j) {
+      const f4 at = *reinterpret_cast<const f4*>(&sT[(16 * mt + r16) * P + 16 * j + 4 * gq]);
+      f4 bk[NDT], bv[NDT];
 #pragma unroll
       for (int q = 0; q < NDT; ++q) {
-        const int col = 16 * (dg * NDT + q) + r16;
-        accW[q] = mfma4(at, sK[(4 * k + gq) * P + col], accW[q]);
-        accU[q] = mfma4(at, sV[(4 * k + gq) * PC + col], accU[q]);
+        const int o = (16 * (dg * NDT + q) + r16) * P + 16 * j + 4 * gq;
+        bk[q] = *reinterpret_cast<const f4*>(&sK[o]);
+        bv[q] = *reinterpret_cast<const f4*>(&sL[o]);
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int q = 0; q < NDT; ++q) {
+          accW[q] = mfma4(at[e], bk[q][e], accW[q]);
+          accU[q] = mfma4(at[e], bv[q][e], accU[q]);
+        }
     }
     const int64_t wu0 = ch * kC * D + c0;
 #pragma unroll
