@@ -44,7 +44,7 @@
 //  * kda_overlap_kernel (16-bit inputs, <= 24 chains) -- one segment's
 //    state-slice workgroups and the next segment's intra work in one launch.
 //  * kda_state_kernel (exact mode, fp32 inputs) -- one workgroup per (chain,
-//    32-column dv slice) with fp32 operands.
+//    32- or 16-column dv slice) with fp32 operands.
 
 #include <type_traits>
 
@@ -1183,220 +1183,222 @@ void kda_intra_kernel(IntraArgs a) {
 }
 
 // ----------------------------------------------------------------------------
-// State step: one chunk of one chain for a 32-column value slice
+// State kernel, exact mode (fp32 operands): one workgroup per (chain, slice of
+// ET 16-column value tiles), eight waves.  Chain wave W (0 .. 3) owns row tile
+// W of v~ and channel tiles W DTW .. of S and runs the recurrence,
+//   v~ = U - W S,  S <- gamma_C S + (lambda k)^T v~;
+// output wave W forms row tile W of o = (gamma q) S + Aqk v~ one chunk behind,
+// from the S^T and v~^T the chain waves leave in LDS (two buffers each), so the
+// serial step holds only the recurrence's products and the outputs' fill the
+// matrix cores while it waits on LDS and barriers.  Two barriers per chunk.
+// The fp32 MFMAs bound it (per SIMD and chunk 112 ET at d = 128, 32 cycles
+// each), so a call whose two-tile slices leave half the CUs idle runs one-tile
+// slices on twice the CUs; past that they only add reads and barriers.
+// Four waves doing all of it on two-tile slices: 24.3 us (B1 T512 H4 d64) and
+// 77 us (B2 T1024 H8 d128) of state launch; one-tile slices 16.2 and 51, the
+// output waves too 15.4 and 49.6.  Where slices stay two-tile the output waves
+// gain 1 to 8 % of the call (B8 T2048 H32 d64 575 -> 533 us).
 // ----------------------------------------------------------------------------
-template <int DK, bool EXACT>
-struct StateFrags {
-  typedef typename Prec<EXACT>::v8 v8;
-  typedef typename Prec<EXACT>::v4 v4;
-  static constexpr int NJ = DK / 32;
-  static constexpr int DTW = DK / 64;
-  v8 W[NJ], Q[NJ], A[2], L[DTW][2];
-  v4 U[2];
-  f4 gc[DTW];
+template <int DK, int ET>
+struct ExactChainFrags {
+  f8 W[DK / 32], L[DK / 64][2];
+  f4 U[ET], gc[DK / 64];
+};
+template <int DK>
+struct ExactOutFrags {
+  f8 Q[DK / 32], A[2];
 };
 
-template <int DK, int DV, bool EXACT>
-struct StateSmem {
-  typedef typename Prec<EXACT>::st st;
+template <int DK, int ET>
+struct ExactSmem {
   static constexpr int PK = DK + 8;
   static constexpr int PC = kC + 8;
-  st St[32 * PK];   // S^T slice: [value col][channel]
-  st Vt[32 * PC];   // v~^T: [value col][row]
+  float St[2][16 * ET * PK];   // S^T slice: [value col][channel]
+  float Vt[2][16 * ET * PC];   // v~^T: [value col][row]
 };
 
-template <int DK, int DV, bool EXACT, int W>
-__device__ __forceinline__ void load_frags(StateFrags<DK, EXACT>& f, const StateArgs& a,
-                                           int64_t chead, int split, int l, int gq) {
-  typedef typename Prec<EXACT>::st st;
-  typedef typename Prec<EXACT>::v8 v8;
-  typedef typename Prec<EXACT>::v4 v4;
-  constexpr int NJ = DK / 32;
-  constexpr int DTW = DK / 64;
-  const st* iW = static_cast<const st*>(a.W);
-  const st* iQ = static_cast<const st*>(a.GQ);
-  const st* iA = static_cast<const st*>(a.AQ);
-  const st* iL = static_cast<const st*>(a.LK);
-  const st* iU = static_cast<const st*>(a.U);
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    f.W[j] = *reinterpret_cast<const v8*>(iW + (chead * (kC / 16) * NJ + (W * NJ + j)) * 512 + l * 8);
-    f.Q[j] = *reinterpret_cast<const v8*>(iQ + (chead * (kC / 16) * NJ + (W * NJ + j)) * 512 + l * 8);
-  }
-  constexpr int NA = (W < 2) ? 1 : 2;  // Aqk row tile W has no keys past tile W
-#pragma unroll
-  for (int jj = 0; jj < NA; ++jj)
-    f.A[jj] = *reinterpret_cast<const v8*>(iA + (chead * (kC / 16) * 2 + (W * 2 + jj)) * 512 + l * 8);
-#pragma unroll
-  for (int et = 0; et < 2; ++et)
-    f.U[et] = *reinterpret_cast<const v4*>(
-        iU + (chead * (kC / 16) * (DV / 16) + (W * (DV / 16) + 2 * split + et)) * 256 + l * 4);
-#pragma unroll
-  for (int t = 0; t < DTW; ++t) {
-    const int dt = W * DTW + t;
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-      f.L[t][jj] = *reinterpret_cast<const v8*>(iL + (chead * (DK / 16) * 2 + (dt * 2 + jj)) * 512 + l * 8);
-    f.gc[t] = *reinterpret_cast<const f4*>(a.GC + chead * DK + 16 * dt + 4 * gq);
-  }
+// B fragment of a 32-wide K step from an S^T or v~^T row
+__device__ __forceinline__ f8 exact_bfrag(const float* row) {
+  const f4 s0 = *reinterpret_cast<const f4*>(row), s1 = *reinterpret_cast<const f4*>(row + 16);
+  return f8{s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
 }
 
-template <int DK, int DV, bool EXACT, int OUT_DT, int W>
-__device__ __forceinline__ void state_step(f4 (&S)[DK / 64][2], const StateFrags<DK, EXACT>& f,
-                                           StateSmem<DK, DV, EXACT>& sm, const StateArgs& a,
-                                           int64_t row0, int len, int h, int split,
-                                           int r, int gq) {
-  typedef typename Prec<EXACT>::st st;
-  typedef typename Prec<EXACT>::v8 v8;
-  typedef typename Prec<EXACT>::v4 v4;
+template <int DK, int DV, int ET, int W>
+__device__ __forceinline__ void exact_chain(const StateArgs& a, ExactSmem<DK, ET>& sm, const ChainRef& c, int h,
+                                            int split) {
   constexpr int NJ = DK / 32;
   constexpr int DTW = DK / 64;
-  constexpr int PK = DK + 8;
-  constexpr int PC = kC + 8;
-  const int H = a.geom.H;
-
-  // 1. S^T slice -> LDS (operand precision)
-#pragma unroll
-  for (int t = 0; t < DTW; ++t)
-#pragma unroll
-    for (int et = 0; et < 2; ++et)
-      *reinterpret_cast<v4*>(&sm.St[(16 * et + r) * PK + 16 * (W * DTW + t) + 4 * gq]) = cvt4<EXACT>(S[t][et]);
-  lds_barrier();
-
-  // 2. P = W S, O = (gamma q) S, v~ = U - P
-  f4 O[2];
-#pragma unroll
-  for (int et = 0; et < 2; ++et) {
-    f4 P = {0, 0, 0, 0};
-    O[et] = f4{0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      v8 Sf;
-      const st* row = &sm.St[(16 * et + r) * PK + 32 * j + 4 * gq];
-      const v4 s0 = *reinterpret_cast<const v4*>(row);
-      const v4 s1 = *reinterpret_cast<const v4*>(row + 16);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { Sf[i] = s0[i]; Sf[4 + i] = s1[i]; }
-      P = mma32(P, f.W[j], Sf);
-      O[et] = mma32(O[et], f.Q[j], Sf);
-    }
-    f4 vt;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) vt[i] = static_cast<float>(f.U[et][i]) - P[i];
-    *reinterpret_cast<v4*>(&sm.Vt[(16 * et + r) * PC + 16 * W + 4 * gq]) = cvt4<EXACT>(vt);
-  }
-  lds_barrier();
-
-  // 3. O += Aqk v~ ; 4. S <- gamma_C S + (lambda k)^T v~
-  constexpr int NA = (W < 2) ? 1 : 2;
-#pragma unroll
-  for (int et = 0; et < 2; ++et) {
-    v8 Vf[2];
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const st* row = &sm.Vt[(16 * et + r) * PC + 32 * jj + 4 * gq];
-      const v4 s0 = *reinterpret_cast<const v4*>(row);
-      const v4 s1 = *reinterpret_cast<const v4*>(row + 16);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { Vf[jj][i] = s0[i]; Vf[jj][4 + i] = s1[i]; }
-    }
-#pragma unroll
-    for (int jj = 0; jj < NA; ++jj) O[et] = mma32(O[et], f.A[jj], Vf[jj]);
-#pragma unroll
-    for (int t = 0; t < DTW; ++t) {
-      f4 s = S[t][et] * f.gc[t];
-      s = mma32(s, f.L[t][0], Vf[0]);
-      s = mma32(s, f.L[t][1], Vf[1]);
-      S[t][et] = s;
-    }
-  }
-  // o stores last: nothing in this step reuses their source registers, so the
-  // caller's next prefetch is younger than every pending store
-#pragma unroll
-  for (int et = 0; et < 2; ++et)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int cr = 16 * W + 4 * gq + i;
-      if (cr < len) {
-        const int64_t oi = ((row0 + cr) * H + h) * (int64_t)DV + 32 * split + 16 * et + r;
-        if constexpr (OUT_DT == 0) static_cast<float*>(a.o)[oi] = O[et][i];
-        else static_cast<u16*>(a.o)[oi] = f32_to_bf16_bits(O[et][i]);
-      }
-    }
-  // (the next step's first barrier orders St/Vt reuse)
-}
-
-template <int DK, int DV, bool EXACT, int OUT_DT, int W>
-__device__ __forceinline__ void state_chain(const StateArgs& a, StateSmem<DK, DV, EXACT>& sm,
-                                            int seq, int h, int split) {
-  constexpr int DTW = DK / 64;
+  constexpr int PK = ExactSmem<DK, ET>::PK, PC = ExactSmem<DK, ET>::PC;
   const Geom& G = a.geom;
   const int H = G.H;
   const int l = threadIdx.x & 63, r = l & 15, gq = l >> 4;
-  const ChainRef c = chain_ref(G, seq);
-  if (!c.active) return;
-  const int nchunks = c.nchunks, seq_len = c.seq_len;
-  const int64_t tok0 = c.tok0;
-
-  f4 S[DTW][2];
+  const int nchunks = c.nchunks;
+  f4 S[DTW][ET];
   const int64_t sbase = (static_cast<int64_t>(c.seq) * H + h) * DK * DV;
   const float* const s_in = c.from_h0 ? a.h0 : a.ht;
 #pragma unroll
   for (int t = 0; t < DTW; ++t)
 #pragma unroll
-    for (int et = 0; et < 2; ++et)
+    for (int et = 0; et < ET; ++et)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int d = 16 * (W * DTW + t) + 4 * gq + i;
-        const int e = 32 * split + 16 * et + r;
+        const int e = 16 * (ET * split + et) + r;
         S[t][et][i] = (s_in != nullptr) ? s_in[sbase + static_cast<int64_t>(d) * DV + e] : 0.f;
       }
-
-  auto chead_of = [&](int n) { return static_cast<int64_t>(chain_unit(G, c, n)) * H + h; };
-  auto step = [&](const StateFrags<DK, EXACT>& f, int n) {
-    const int64_t row0 = tok0 + static_cast<int64_t>(n) * kC;
-    const int len = min(kC, seq_len - n * kC);
-    state_step<DK, DV, EXACT, OUT_DT, W>(S, f, sm, a, row0, len, h, split, r, gq);
+  auto load = [&](ExactChainFrags<DK, ET>& f, int n) {
+    const int64_t ch = static_cast<int64_t>(chain_unit(G, c, min(n, nchunks - 1))) * H + h;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      f.W[j] = *reinterpret_cast<const f8*>(static_cast<const float*>(a.W) + (ch * 4 * NJ + W * NJ + j) * 512 + l * 8);
+#pragma unroll
+    for (int et = 0; et < ET; ++et)
+      f.U[et] = *reinterpret_cast<const f4*>(static_cast<const float*>(a.U) +
+                                             (ch * 4 * (DV / 16) + W * (DV / 16) + ET * split + et) * 256 + l * 4);
+#pragma unroll
+    for (int t = 0; t < DTW; ++t) {
+      const int dt = W * DTW + t;
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj)
+        f.L[t][jj] = *reinterpret_cast<const f8*>(static_cast<const float*>(a.LK) + (ch * (DK / 16) * 2 + dt * 2 + jj) * 512 + l * 8);
+      f.gc[t] = *reinterpret_cast<const f4*>(a.GC + ch * DK + 16 * dt + 4 * gq);
+    }
   };
-  // Three fragment sets in fixed registers.  The loads for chunk n+3 are issued
-  // right after step n (and its o stores), so they are younger than every
-  // store the next steps must retire before reusing registers: vmcnt retires
-  // in order on this architecture, and a prefetch issued before the stores
-  // would have to complete before them.
-  StateFrags<DK, EXACT> f0, f1, f2;
-  if (nchunks > 0) load_frags<DK, DV, EXACT, W>(f0, a, chead_of(0), split, l, gq);
-  if (nchunks > 1) load_frags<DK, DV, EXACT, W>(f1, a, chead_of(1), split, l, gq);
-  if (nchunks > 2) load_frags<DK, DV, EXACT, W>(f2, a, chead_of(2), split, l, gq);
-  for (int n = 0; n < nchunks; n += 3) {
+  auto step = [&](const ExactChainFrags<DK, ET>& f, int n) {
+    float* const St = sm.St[n & 1];
+    float* const Vt = sm.Vt[n & 1];
+#pragma unroll
+    for (int t = 0; t < DTW; ++t)
+#pragma unroll
+      for (int et = 0; et < ET; ++et)
+        *reinterpret_cast<f4*>(&St[(16 * et + r) * PK + 16 * (W * DTW + t) + 4 * gq]) = S[t][et];
+    lds_barrier();   // S of chunk n written
+    f4 P[ET];
+#pragma unroll
+    for (int et = 0; et < ET; ++et) P[et] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int et = 0; et < ET; ++et)
+        P[et] = mma32(P[et], f.W[j], exact_bfrag(&St[(16 * et + r) * PK + 32 * j + 4 * gq]));
+#pragma unroll
+    for (int et = 0; et < ET; ++et)
+      *reinterpret_cast<f4*>(&Vt[(16 * et + r) * PC + 16 * W + 4 * gq]) = f.U[et] - P[et];
+    lds_barrier();   // v~ of chunk n written
+#pragma unroll
+    for (int et = 0; et < ET; ++et) {
+      const f8 v0 = exact_bfrag(&Vt[(16 * et + r) * PC + 4 * gq]), v1 = exact_bfrag(&Vt[(16 * et + r) * PC + 32 + 4 * gq]);
+#pragma unroll
+      for (int t = 0; t < DTW; ++t) S[t][et] = mma32(mma32(S[t][et] * f.gc[t], f.L[t][0], v0), f.L[t][1], v1);
+    }
+  };
+  // two fragment sets in fixed registers, each reloaded right after its step
+  ExactChainFrags<DK, ET> f0, f1;
+  if (nchunks > 0) load(f0, 0);
+  if (nchunks > 1) load(f1, 1);
+  for (int n = 0; n < nchunks; n += 2) {
     step(f0, n);
-    if (n + 3 < nchunks) load_frags<DK, DV, EXACT, W>(f0, a, chead_of(n + 3), split, l, gq);
     if (n + 1 >= nchunks) break;
+    load(f0, n + 2);
     step(f1, n + 1);
-    if (n + 4 < nchunks) load_frags<DK, DV, EXACT, W>(f1, a, chead_of(n + 4), split, l, gq);
-    if (n + 2 >= nchunks) break;
-    step(f2, n + 2);
-    if (n + 5 < nchunks) load_frags<DK, DV, EXACT, W>(f2, a, chead_of(n + 5), split, l, gq);
+    load(f1, n + 3);
   }
-
   if (a.ht != nullptr) {
 #pragma unroll
     for (int t = 0; t < DTW; ++t)
 #pragma unroll
-      for (int et = 0; et < 2; ++et)
+      for (int et = 0; et < ET; ++et)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int d = 16 * (W * DTW + t) + 4 * gq + i;
-          const int e = 32 * split + 16 * et + r;
+          const int e = 16 * (ET * split + et) + r;
           a.ht[sbase + static_cast<int64_t>(d) * DV + e] = S[t][et][i];
         }
   }
 }
 
-template <int DK, int DV, bool EXACT, int OUT_DT>
-__global__ __launch_bounds__(256, 1)
+template <int DK, int DV, int ET, int OUT_DT, int W>
+__device__ __forceinline__ void exact_out(const StateArgs& a, ExactSmem<DK, ET>& sm, const ChainRef& c, int h, int split) {
+  constexpr int NJ = DK / 32;
+  constexpr int NA = (W < 2) ? 1 : 2;   // Aqk row tile W has no keys past tile W
+  constexpr int PK = ExactSmem<DK, ET>::PK, PC = ExactSmem<DK, ET>::PC;
+  const Geom& G = a.geom;
+  const int H = G.H;
+  const int l = threadIdx.x & 63, r = l & 15, gq = l >> 4;
+  const int nchunks = c.nchunks, seq_len = c.seq_len;
+  auto load = [&](ExactOutFrags<DK>& f, int n) {
+    const int64_t ch = static_cast<int64_t>(chain_unit(G, c, min(n, nchunks - 1))) * H + h;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      f.Q[j] = *reinterpret_cast<const f8*>(static_cast<const float*>(a.GQ) + (ch * 4 * NJ + W * NJ + j) * 512 + l * 8);
+#pragma unroll
+    for (int jj = 0; jj < NA; ++jj)
+      f.A[jj] = *reinterpret_cast<const f8*>(static_cast<const float*>(a.AQ) + (ch * 8 + W * 2 + jj) * 512 + l * 8);
+  };
+  f4 O[ET];
+  auto from_s = [&](const ExactOutFrags<DK>& f, int n) {   // (gamma q) S of chunk n
+    const float* const St = sm.St[n & 1];
+#pragma unroll
+    for (int et = 0; et < ET; ++et) O[et] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int et = 0; et < ET; ++et)
+        O[et] = mma32(O[et], f.Q[j], exact_bfrag(&St[(16 * et + r) * PK + 32 * j + 4 * gq]));
+  };
+  auto from_v = [&](const ExactOutFrags<DK>& f, int n) {   // + Aqk v~, stored
+    const float* const Vt = sm.Vt[n & 1];
+#pragma unroll
+    for (int jj = 0; jj < NA; ++jj)
+#pragma unroll
+      for (int et = 0; et < ET; ++et)
+        O[et] = mma32(O[et], f.A[jj], exact_bfrag(&Vt[(16 * et + r) * PC + 32 * jj + 4 * gq]));
+    const int64_t row0 = c.tok0 + static_cast<int64_t>(n) * kC;
+    const int len = min(kC, seq_len - n * kC);
+#pragma unroll
+    for (int et = 0; et < ET; ++et)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int cr = 16 * W + 4 * gq + i;
+        if (cr < len) {
+          const int64_t oi = ((row0 + cr) * H + h) * (int64_t)DV + 16 * (ET * split + et) + r;
+          if constexpr (OUT_DT == 0) static_cast<float*>(a.o)[oi] = O[et][i];
+          else static_cast<u16*>(a.o)[oi] = f32_to_bf16_bits(O[et][i]);
+        }
+      }
+  };
+  // step n's barriers, chunk n - 1's outputs between and after them: its S
+  // buffer is rewritten only after step n's second barrier, its v~ buffer
+  // only after step n + 1's first
+  auto step = [&](const ExactOutFrags<DK>& f, int n) {
+    lds_barrier();
+    if (n > 0) from_s(f, n - 1);
+    lds_barrier();
+    if (n > 0) from_v(f, n - 1);
+  };
+  // chunk n's fragments are in f0 for even n
+  ExactOutFrags<DK> f0, f1;
+  if (nchunks > 0) load(f0, 0);
+  if (nchunks > 1) load(f1, 1);
+  for (int n = 0; n < nchunks; n += 2) {
+    step(f1, n);                        // chunk n - 1 (odd)
+    if (n > 0) load(f1, n + 1);
+    if (n + 1 >= nchunks) break;
+    step(f0, n + 1);                    // chunk n (even)
+    load(f0, n + 2);
+  }
+  if (nchunks > 0) {                    // the last chunk: both buffers were written before the last barrier
+    const ExactOutFrags<DK>& f = (nchunks & 1) ? f0 : f1;
+    from_s(f, nchunks - 1);
+    from_v(f, nchunks - 1);
+  }
+}
+
+template <int DK, int DV, int ET, int OUT_DT>
+__global__ __launch_bounds__(512, 1)
 void kda_state_kernel(StateArgs a) {
-  constexpr int SPLITS = DV / 32;
-  __shared__ StateSmem<DK, DV, EXACT> sm;
+  constexpr int SPLITS = DV / (16 * ET);
+  __shared__ __attribute__((aligned(16))) ExactSmem<DK, ET> sm;
   const Geom& G = a.geom;
   const int H = G.H;
   // XCD-aware mapping: the SPLITS workgroups of one chain share an XCD (and L2)
@@ -1409,12 +1411,17 @@ void kda_state_kernel(StateArgs a) {
   if (chain >= G.N * H) return;
   const int seq_rank = chain / H;
   const int h = chain - seq_rank * H;
-  const int seq = seq_rank;   // the roles look the sequence up (chain_ref)
+  const ChainRef c = chain_ref(G, seq_rank);
+  if (!c.active) return;   // uniform per workgroup
   switch (threadIdx.x >> 6) {
-    case 0: state_chain<DK, DV, EXACT, OUT_DT, 0>(a, sm, seq, h, split); break;
-    case 1: state_chain<DK, DV, EXACT, OUT_DT, 1>(a, sm, seq, h, split); break;
-    case 2: state_chain<DK, DV, EXACT, OUT_DT, 2>(a, sm, seq, h, split); break;
-    default: state_chain<DK, DV, EXACT, OUT_DT, 3>(a, sm, seq, h, split); break;
+    case 0: exact_chain<DK, DV, ET, 0>(a, sm, c, h, split); break;
+    case 1: exact_chain<DK, DV, ET, 1>(a, sm, c, h, split); break;
+    case 2: exact_chain<DK, DV, ET, 2>(a, sm, c, h, split); break;
+    case 3: exact_chain<DK, DV, ET, 3>(a, sm, c, h, split); break;
+    case 4: exact_out<DK, DV, ET, OUT_DT, 0>(a, sm, c, h, split); break;
+    case 5: exact_out<DK, DV, ET, OUT_DT, 1>(a, sm, c, h, split); break;
+    case 6: exact_out<DK, DV, ET, OUT_DT, 2>(a, sm, c, h, split); break;
+    default: exact_out<DK, DV, ET, OUT_DT, 3>(a, sm, c, h, split); break;
   }
 }
 
@@ -2281,10 +2288,14 @@ static hipError_t launch_intra_t(const IntraArgs& a, int grid, hipStream_t s) {
 // config 2 1 569 -> 2 465 us), so calls with fewer chains keep the 32-column
 // slices.
 constexpr int kFullStateMinChains = 256;
+constexpr int kCUs = 256;
 template <int DK, int DV, bool EXACT, int OUT>
 static hipError_t launch_state_t(const StateArgs& a, int grid, hipStream_t s) {
   if constexpr (EXACT) {
-    hipLaunchKernelGGL((kda_state_kernel<DK, DV, EXACT, OUT>), dim3(grid), dim3(256), 0, s, a);
+    if (2 * grid <= kCUs)   // one-tile slices, see the kernel
+      hipLaunchKernelGGL((kda_state_kernel<DK, DV, 1, OUT>), dim3(2 * grid), dim3(512), 0, s, a);
+    else
+      hipLaunchKernelGGL((kda_state_kernel<DK, DV, 2, OUT>), dim3(grid), dim3(512), 0, s, a);
   } else {
     const int64_t chains = static_cast<int64_t>(a.geom.N) * a.geom.H;
     if (DK == 128 && chains >= kFullStateMinChains) {
