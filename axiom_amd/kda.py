@@ -28,6 +28,7 @@ stream; nothing here computes on the CPU.
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 
 import torch
 
@@ -40,15 +41,38 @@ SUPPORTED_HEAD_DIMS = (64, 128)
 CHUNK = 64
 
 
+# The host path of a call is a few microseconds of Python, which is what a small
+# call costs: one decode-layer token took 15.9 us around a 6.3 us kernel with a
+# ctypes object per pointer, a set of device objects, a query of torch's device
+# state, three workspace queries and a formatted name per tensor checked.
 def _ptr(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    """Device address for a c_void_p argument (None: a null pointer)."""
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device):
+    """Handle of the device's current stream (without building a Stream object where torch allows)."""
+    return _raw_stream(device.index) if _raw_stream is not None else torch.cuda.current_stream(device).cuda_stream
 
 
 def _require_gpu(tensors, what: str) -> torch.device:
+    """The one GPU all tensors are on; raises as :func:`_wrong_device` otherwise."""
+    index = dev = None
+    for t in tensors:
+        if t is not None:
+            if not t.is_cuda:
+                return _wrong_device(tensors, what)
+            if index is None:
+                index, dev = t.get_device(), t.device
+            elif t.get_device() != index:
+                return _wrong_device(tensors, what)
+    return dev if dev is not None else _wrong_device(tensors, what)
+
+
+def _wrong_device(tensors, what: str) -> torch.device:
     devs = {t.device for t in tensors if t is not None}
     if len(devs) != 1:
         raise ValueError(f"{what}: all tensors must be on one device, got {sorted(map(str, devs))}")
@@ -63,6 +87,18 @@ def _require_gpu(tensors, what: str) -> torch.device:
 def _contig(name, t):
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
+
+
+def _contig_args(tensors):
+    for i, t in enumerate(tensors):
+        if not t.is_contiguous():
+            raise ValueError(f"arg{i} must be contiguous")
+
+
+@lru_cache(maxsize=1024)
+def _ws_bytes(entry: str, *sizes) -> int:
+    """A workspace query of the library: a function of its whole-number arguments alone."""
+    return int(getattr(_lib.lib(), entry)(*sizes))
 
 
 def _check_dims(dk, dv, what):
@@ -110,7 +146,7 @@ def kda_chunk_fwd(q, k, v, g, beta, initial_state=None, cu_seqlens=None, chunk_s
     if v.dim() != 4 or v.shape[:3] != q.shape[:3]:
         raise ValueError(f"{what}: v must be [B,T,H,dv] matching q")
     dv = v.shape[3]
-    if tuple(beta.shape) != (B, T, H):
+    if beta.shape != (B, T, H):
         raise ValueError(f"{what}: beta must be [B,T,H] = {(B, T, H)}, got {tuple(beta.shape)}")
     if chunk_size != CHUNK:
         raise ValueError(f"{what}: chunk_size={chunk_size} unsupported (this build runs {CHUNK})")
@@ -135,7 +171,7 @@ def kda_chunk_fwd(q, k, v, g, beta, initial_state=None, cu_seqlens=None, chunk_s
         n_seqs = cu_seqlens.numel() - 1
         N = n_seqs
     if initial_state is not None:
-        if initial_state.dtype != torch.float32 or tuple(initial_state.shape) != (N, H, dk, dv):
+        if initial_state.dtype != torch.float32 or initial_state.shape != (N, H, dk, dv):
             raise ValueError(f"{what}: initial_state must be fp32 [{N},{H},{dk},{dv}]")
     for name, t in (("q", q), ("k", k), ("v", v), ("g", g), ("beta", beta),
                     ("initial_state", initial_state), ("cu_seqlens", cu_seqlens)):
@@ -143,20 +179,20 @@ def kda_chunk_fwd(q, k, v, g, beta, initial_state=None, cu_seqlens=None, chunk_s
             _contig(name, t)
     dev = _require_gpu([q, k, v, g, beta, initial_state, cu_seqlens], what)
     L = _lib.lib()
-    ws_bytes = int(L.kda_chunk_fwd_workspace(B, T, H, dk, dv, CHUNK, n_seqs, in_code))
+    ws_bytes = _ws_bytes("kda_chunk_fwd_workspace", B, T, H, dk, dv, CHUNK, n_seqs, in_code)
     if ws_bytes == 0:
         raise ValueError(f"{what}: unsupported configuration")
     # a caller workspace of at least the minimum is used as it is (a large
     # varlen call then runs in the segments that fit it); else a new one of
     # the fastest schedule's size
-    ws_min = int(L.kda_chunk_fwd_workspace_min(B, T, H, dk, dv, CHUNK, n_seqs, in_code))
-    if workspace is not None and workspace.numel() * workspace.element_size() >= ws_min:
+    if workspace is not None and workspace.numel() * workspace.element_size() >= _ws_bytes(
+            "kda_chunk_fwd_workspace_min", B, T, H, dk, dv, CHUNK, n_seqs, in_code):
         _contig("workspace", workspace)
         ws_bytes = min(ws_bytes, workspace.numel() * workspace.element_size())
     else:
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     if out is not None:
-        if tuple(out.shape) != (B, T, H, dv) or out.dtype != out_dtype or out.device != dev:
+        if out.shape != (B, T, H, dv) or out.dtype != out_dtype or out.device != dev:
             raise ValueError(f"{what}: out must be {out_dtype} [{B},{T},{H},{dv}] on {dev}")
         _contig("out", out)
         o = out
@@ -165,7 +201,7 @@ def kda_chunk_fwd(q, k, v, g, beta, initial_state=None, cu_seqlens=None, chunk_s
     if not output_final_state:
         ht = None
     elif final_state is not None:
-        if tuple(final_state.shape) != (N, H, dk, dv) or final_state.dtype != torch.float32 \
+        if final_state.shape != (N, H, dk, dv) or final_state.dtype != torch.float32 \
                 or final_state.device != dev:
             raise ValueError(f"{what}: final_state must be fp32 [{N},{H},{dk},{dv}] on {dev}")
         _contig("final_state", final_state)
@@ -217,7 +253,7 @@ def _chunk_bwd(q, k, v, g, beta, do, dht, initial_state, scale, chunk_size, need
     if v.dim() != 4 or v.shape[:3] != q.shape[:3]:
         raise ValueError(f"{what}: v must be [B,T,H,dv] matching q")
     dv = v.shape[3]
-    if tuple(beta.shape) != (B, T, H):
+    if beta.shape != (B, T, H):
         raise ValueError(f"{what}: beta must be [B,T,H] = {(B, T, H)}, got {tuple(beta.shape)}")
     if chunk_size != CHUNK:
         raise ValueError(f"{what}: chunk_size={chunk_size} unsupported (this build runs {CHUNK})")
@@ -230,10 +266,10 @@ def _chunk_bwd(q, k, v, g, beta, do, dht, initial_state, scale, chunk_size, need
         in_code = _lib.KDA_DTYPE_BF16_F32GATES
     else:
         raise ValueError(f"{what}: g/beta dtype must equal q's, or be fp32 with bf16 q/k/v")
-    if tuple(do.shape) != (B, T, H, dv) or do.dtype not in _OUT_CODES:
+    if do.shape != (B, T, H, dv) or do.dtype not in _OUT_CODES:
         raise ValueError(f"{what}: do must be fp32 or bf16 [{B},{T},{H},{dv}]")
     for name, st in (("dht", dht), ("initial_state", initial_state)):
-        if st is not None and (st.dtype != torch.float32 or tuple(st.shape) != (B, H, dk, dv)):
+        if st is not None and (st.dtype != torch.float32 or st.shape != (B, H, dk, dv)):
             raise ValueError(f"{what}: {name} must be fp32 [{B},{H},{dk},{dv}]")
     for name, t in (("q", q), ("k", k), ("v", v), ("g", g), ("beta", beta), ("do", do),
                     ("dht", dht), ("initial_state", initial_state)):
@@ -241,7 +277,7 @@ def _chunk_bwd(q, k, v, g, beta, do, dht, initial_state, scale, chunk_size, need
             _contig(name, t)
     dev = _require_gpu([q, k, v, g, beta, do, dht, initial_state], what)
     L = _lib.lib()
-    ws_bytes = int(L.kda_chunk_bwd_workspace(B, T, H, dk, dv, CHUNK))
+    ws_bytes = _ws_bytes("kda_chunk_bwd_workspace", B, T, H, dk, dv, CHUNK)
     if ws_bytes == 0:
         raise ValueError(f"{what}: unsupported configuration")
     if workspace is None or workspace.numel() * workspace.element_size() < ws_bytes:
@@ -267,6 +303,7 @@ class _KDAChunk(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, g, beta, initial_state, scale):
         o, ht = kda_chunk_fwd(q, k, v, g, beta, initial_state=initial_state, scale=scale)
+        ctx.set_materialize_grads(False)   # an unused output's cotangent stays None: no zero tensor
         ctx.save_for_backward(q, k, v, g, beta, initial_state)
         ctx.scale = scale
         return o, ht
@@ -396,15 +433,14 @@ def kda_prologue(qp, kp, vp, wq, wk, wv, num_heads: int, conv_state=None, return
         raise ValueError(f"{what}: projections and out_dtype must be fp32 or bf16")
     K = wq.shape[0]
     for name, w in (("wq", wq), ("wk", wk), ("wv", wv)):
-        if w.dtype != torch.float32 or tuple(w.shape) != (K, HD):
+        if w.dtype != torch.float32 or w.shape != (K, HD):
             raise ValueError(f"{what}: {name} must be fp32 [{K},{HD}]")
     if conv_state is not None:
         for st in conv_state:
-            if st.dtype != torch.float32 or tuple(st.shape) != (B, K - 1, HD):
+            if st.dtype != torch.float32 or st.shape != (B, K - 1, HD):
                 raise ValueError(f"{what}: conv_state buffers must be fp32 [{B},{K - 1},{HD}]")
     tensors = [qp, kp, vp, wq, wk, wv] + list(conv_state or [])
-    for i, t in enumerate(tensors):
-        _contig(f"arg{i}", t)
+    _contig_args(tensors)
     dev = _require_gpu(tensors, what)
     q = torch.empty((B, T, H, d), dtype=out_dtype, device=dev)
     k = torch.empty_like(q)
@@ -429,7 +465,7 @@ def kda_epilogue(o, gate, eps: float = 1e-6, out_dtype=torch.bfloat16):
     if o.dim() != 4:
         raise ValueError(f"{what}: o must be [B,T,H,dv]")
     B, T, H, dv = o.shape
-    if tuple(gate.shape) != (B, T, H * dv):
+    if gate.shape != (B, T, H * dv):
         raise ValueError(f"{what}: gate must be [{B},{T},{H * dv}]")
     if dv not in SUPPORTED_HEAD_DIMS:
         raise ValueError(f"{what}: dv={dv} unsupported ({SUPPORTED_HEAD_DIMS})")
@@ -456,9 +492,9 @@ def kda_decode_layer_step(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state, sta
     """
     what = "kda_decode_layer_step"
     B, H, d = g.shape
-    if tuple(qp.shape) != (B, H * d) or kp.shape != qp.shape or vp.shape != qp.shape or gate.shape != qp.shape:
+    if qp.shape != (B, H * d) or kp.shape != qp.shape or vp.shape != qp.shape or gate.shape != qp.shape:
         raise ValueError(f"{what}: qp, kp, vp, gate must be [{B},{H * d}]")
-    if tuple(beta.shape) != (B, H) or tuple(state.shape) != (B, H, d, d) or state.dtype != torch.float32:
+    if beta.shape != (B, H) or state.shape != (B, H, d, d) or state.dtype != torch.float32:
         raise ValueError(f"{what}: beta [B,H], state fp32 [B,H,d,d] expected")
     dt = qp.dtype
     if dt not in _UT_CODES or any(t.dtype != dt for t in (kp, vp, g, beta, gate)):
@@ -466,11 +502,10 @@ def kda_decode_layer_step(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state, sta
     K = wq.shape[0]
     bq, bk, bv = conv_state
     tensors = [qp, kp, vp, g, beta, gate, wq, wk, wv, bq, bk, bv, state]
-    for i, t in enumerate(tensors):
-        _contig(f"arg{i}", t)
+    _contig_args(tensors)
     dev = _require_gpu(tensors, what)
     L = _lib.lib()
-    need = int(L.kda_decode_layer_workspace(B, H, d, _UT_CODES[dt]))
+    need = _ws_bytes("kda_decode_layer_workspace", B, H, d, _UT_CODES[dt])
     if need == 0:
         raise ValueError(f"{what}: unsupported configuration")
     if workspace is None or workspace.numel() * workspace.element_size() < need:
@@ -509,7 +544,7 @@ def kda_layer_fwd(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state=None, initia
     if g.dim() != 4:
         raise ValueError(f"{what}: g must be [B,T,H,d]")
     B, T, H, d = g.shape
-    if tuple(qp.shape) != (B, T, H * d) or tuple(beta.shape) != (B, T, H):
+    if qp.shape != (B, T, H * d) or beta.shape != (B, T, H):
         raise ValueError(f"{what}: qp [B,T,H*d], beta [B,T,H] expected for g {tuple(g.shape)}")
     _check_dims(d, d, what)
     if any(t.dtype != qp.dtype for t in (kp, vp)) or beta.dtype != g.dtype:
@@ -526,24 +561,23 @@ def kda_layer_fwd(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state=None, initia
         raise ValueError(f"{what}: gate and out_dtype must be fp32 or bf16")
     K = wq.shape[0]
     for name, w in (("wq", wq), ("wk", wk), ("wv", wv)):
-        if w.dtype != torch.float32 or tuple(w.shape) != (K, H * d):
+        if w.dtype != torch.float32 or w.shape != (K, H * d):
             raise ValueError(f"{what}: {name} must be fp32 [{K},{H * d}]")
     if conv_state is not None:
         for st in conv_state:
-            if st.dtype != torch.float32 or tuple(st.shape) != (B, K - 1, H * d):
+            if st.dtype != torch.float32 or st.shape != (B, K - 1, H * d):
                 raise ValueError(f"{what}: conv_state buffers must be fp32 [{B},{K - 1},{H * d}]")
     if initial_state is not None and (initial_state.dtype != torch.float32 or
-                                      tuple(initial_state.shape) != (B, H, d, d)):
+                                      initial_state.shape != (B, H, d, d)):
         raise ValueError(f"{what}: initial_state must be fp32 [{B},{H},{d},{d}]")
-    if o_out is not None and (o_out.dtype != torch.float32 or tuple(o_out.shape) != (B, T, H, d)):
+    if o_out is not None and (o_out.dtype != torch.float32 or o_out.shape != (B, T, H, d)):
         raise ValueError(f"{what}: o_out must be fp32 [{B},{T},{H},{d}]")
     tensors = [qp, kp, vp, g, beta, gate, wq, wk, wv] + list(conv_state or []) + \
         ([initial_state] if initial_state is not None else []) + ([o_out] if o_out is not None else [])
-    for i, t in enumerate(tensors):
-        _contig(f"arg{i}", t)
+    _contig_args(tensors)
     dev = _require_gpu(tensors, what)
     L = _lib.lib()
-    need = int(L.kda_layer_fwd_workspace(B, T, H, d, K, code))
+    need = _ws_bytes("kda_layer_fwd_workspace", B, T, H, d, K, code)
     if need == 0:
         raise ValueError(f"{what}: unsupported configuration")
     if workspace is None or workspace.numel() * workspace.element_size() < need:
@@ -588,7 +622,7 @@ def _prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state, workspace, dx_
     if dq.dim() != 4:
         raise ValueError(f"{what}: dq must be [B,T,H,d]")
     H, d = dq.shape[2], dq.shape[3]
-    if tuple(dq.shape) != (B, T, H, d) or H * d != HD or dk.shape != dq.shape or dv.shape != dq.shape:
+    if dq.shape != (B, T, H, d) or H * d != HD or dk.shape != dq.shape or dv.shape != dq.shape:
         raise ValueError(f"{what}: dq, dk, dv must be [{B},{T},H,d] with H*d = {HD}")
     if any(t.dtype != torch.float32 for t in (dq, dk, dv)):
         raise ValueError(f"{what}: dq, dk, dv must be fp32")
@@ -598,18 +632,17 @@ def _prologue_bwd(qp, kp, vp, wq, wk, wv, dq, dk, dv, conv_state, workspace, dx_
         raise ValueError(f"{what}: projections must be fp32 or bf16")
     K = wq.shape[0]
     for name, w in (("wq", wq), ("wk", wk), ("wv", wv)):
-        if w.dtype != torch.float32 or tuple(w.shape) != (K, HD):
+        if w.dtype != torch.float32 or w.shape != (K, HD):
             raise ValueError(f"{what}: {name} must be fp32 [{K},{HD}]")
     if conv_state is not None:
         for st in conv_state:
-            if st.dtype != torch.float32 or tuple(st.shape) != (B, K - 1, HD):
+            if st.dtype != torch.float32 or st.shape != (B, K - 1, HD):
                 raise ValueError(f"{what}: conv_state buffers must be fp32 [{B},{K - 1},{HD}]")
     tensors = [qp, kp, vp, wq, wk, wv, dq, dk, dv] + list(conv_state or [])
-    for i, t in enumerate(tensors):
-        _contig(f"arg{i}", t)
+    _contig_args(tensors)
     dev = _require_gpu(tensors, what)
     L = _lib.lib()
-    need = int(L.kda_prologue_bwd_workspace(B, T, H, d, K))
+    need = _ws_bytes("kda_prologue_bwd_workspace", B, T, H, d, K)
     if need == 0:
         raise ValueError(f"{what}: unsupported configuration")
     if workspace is None or workspace.numel() * workspace.element_size() < need:
@@ -638,7 +671,7 @@ def kda_epilogue_bwd(o, gate, dy, eps: float = 1e-6, dgate_dtype=None):
     if o.dim() != 4:
         raise ValueError(f"{what}: o must be [B,T,H,dv]")
     B, T, H, dv = o.shape
-    if tuple(gate.shape) != (B, T, H * dv) or tuple(dy.shape) != (B, T, H * dv):
+    if gate.shape != (B, T, H * dv) or dy.shape != (B, T, H * dv):
         raise ValueError(f"{what}: gate and dy must be [{B},{T},{H * dv}]")
     if dv not in SUPPORTED_HEAD_DIMS:
         raise ValueError(f"{what}: dv={dv} unsupported ({SUPPORTED_HEAD_DIMS})")
@@ -671,6 +704,7 @@ class _KDALayer(torch.autograd.Function):
         y, ht, _ = kda_layer_fwd(qp, kp, vp, g, beta, gate, wq, wk, wv, conv_state=conv_state,
                                  initial_state=initial_state, scale=scale, eps=eps, return_conv_state=False,
                                  out_dtype=qp.dtype, o_out=o)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(qp, kp, vp, g, beta, gate, wq, wk, wv, bq, bk, bv, initial_state, o)
         ctx.scale, ctx.eps = scale, eps
         return y, ht
@@ -732,12 +766,12 @@ def kda_recurrent_step(q, k, v, g, beta, state, scale: float = 1.0, out_dtype=to
     if v.dim() != 3 or v.shape[:2] != q.shape[:2]:
         raise ValueError(f"{what}: v must be [B,H,dv]")
     dv = v.shape[2]
-    if tuple(beta.shape) != (B, H):
+    if beta.shape != (B, H):
         raise ValueError(f"{what}: beta must be [B,H]")
     _check_dims(dk, dv, what)
     if q.dtype not in _IN_CODES or any(t.dtype != q.dtype for t in (k, v, g, beta)):
         raise ValueError(f"{what}: q, k, v, g, beta must share a dtype in bf16/fp16/fp32")
-    if state.dtype != torch.float32 or tuple(state.shape) != (B, H, dk, dv):
+    if state.dtype != torch.float32 or state.shape != (B, H, dk, dv):
         raise ValueError(f"{what}: state must be fp32 [{B},{H},{dk},{dv}]")
     if out_dtype not in _OUT_CODES:
         raise ValueError(f"{what}: out_dtype must be fp32 or bf16")
@@ -778,9 +812,9 @@ def _cc_check(q, k, v, alpha, beta32, S, tile, chunk, what, dtype_msg):
     if not (1 <= int(tile) <= 16):
         raise ValueError(f"{what}: tile={tile} outside [1, 16]")
     _check_dims(dk, dv, what)
-    if (tuple(q.shape) != lead + (H * dk,) or tuple(k.shape) != lead + (H * dk,) or k.dtype != dt
-            or tuple(v.shape) != lead + (H * dv,) or tuple(alpha.shape) != lead + (H * dk,)
-            or tuple(beta32.shape) != lead + (H * 32,)):
+    if (q.shape != lead + (H * dk,) or k.shape != lead + (H * dk,) or k.dtype != dt
+            or v.shape != lead + (H * dv,) or alpha.shape != lead + (H * dk,)
+            or beta32.shape != lead + (H * 32,)):
         raise ValueError(f"{what}: shapes must be q,k,alpha ([B,] T,H*dk), v ([B,] T,H*dv), "
                          "beta32 ([B,] T,H*32)")
     if alpha.dtype != torch.float32 or beta32.dtype != torch.float32 or S.dtype != torch.float32:
@@ -796,7 +830,7 @@ def _cc_scan_fwd(q, k, v, alpha, beta32, S, tile, chunk):
     dev = _require_gpu([q, k, v, alpha, beta32, S], "cc_scan")
     L = _lib.lib()
     nb = max(B, 1)
-    ws_bytes = int(L.kda_cc_scan_batched_workspace(nb, T, H, dk, dv, C))
+    ws_bytes = _ws_bytes("kda_cc_scan_batched_workspace", nb, T, H, dk, dv, C)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     o = torch.empty(q.shape[:-1] + (H * dv,), dtype=torch.float32, device=dev)
     S_new = torch.empty_like(S)
@@ -825,13 +859,13 @@ def cc_scan_bwd(q, k, v, alpha, beta32, S, do, dS=None, tile: int = 16, chunk: i
     do = do.float().contiguous()
     if dS is None:
         dS = torch.zeros_like(S)
-    if tuple(dS.shape) != tuple(S.shape):
+    if dS.shape != S.shape:
         raise ValueError(f"{what}: dS must be shaped as S ([B,] H, dk, dv)")
     dS = dS.float().contiguous()
     dev = _require_gpu([q, k, v, alpha, beta32, S, do, dS], what)
     L = _lib.lib()
     nb = max(B, 1)
-    ws_bytes = int(L.kda_cc_scan_bwd_batched_workspace(nb, T, H, dk, dv, C))
+    ws_bytes = _ws_bytes("kda_cc_scan_bwd_batched_workspace", nb, T, H, dk, dv, C)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     dq = torch.empty_like(q)
     dk_ = torch.empty_like(k)
@@ -854,6 +888,7 @@ class _CCScan(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, alpha, beta32, S, tile, chunk):
         o, S_new = _cc_scan_fwd(q, k, v, alpha, beta32, S, tile, chunk)
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(q, k, v, alpha, beta32, S)
         ctx.tile, ctx.chunk = tile, chunk
         return o, S_new
