@@ -1335,15 +1335,17 @@ int kda_layer_fwd(hipStream_t stream, const void* qp, const void* kp, const void
   p.bq_in = bq_in; p.bk_in = bk_in; p.bv_in = bv_in; p.bq_out = bq_out; p.bk_out = bk_out; p.bv_out = bv_out;
   p.B = B; p.T = T; p.H = H; p.K = K;
   const int pdt = in_dtype == KDA_DTYPE_F32 ? 0 : 1;
+  const int gdt = gate_dtype == KDA_DTYPE_F32 ? 0 : 1, ydt = out_dtype == KDA_DTYPE_F32 ? 0 : 1;
+  kda::EpilogueArgs ep{};
+  ep.o = o; ep.gate = gate; ep.y = y; ep.B = B; ep.T = T; ep.H = H; ep.eps = eps;
   hipError_t e;
   if (layer_fused(K, in_dtype)) {
     FusedPrologue fp{{wq, wk, wv}, {bq_in, bk_in, bv_in}, K};
     const int rc = chunk_fwd_impl(stream, qp, kp, vp, g, beta, h0, nullptr, 0, o, ht, B, T, H, d, d, 64, scale,
                                   in_dtype, KDA_DTYPE_F32, ws, chunk_bytes, &fp);
     if (rc != KDA_OK) return rc;
-    // the buffers are rewritten after every read of the old ones
-    e = kda::launch_prologue_buffers(p, d, pdt, stream);
-    if (e != hipSuccess) return hip_fail(e, "layer conv buffer launch");
+    // the buffers are rewritten after every read of the old ones, beside the epilogue
+    e = kda::launch_epilogue_buffers(ep, p, d, gdt, ydt, stream);
   } else {
     const size_t n = static_cast<size_t>(B) * T * H * d;
     const size_t es = in_dtype == KDA_DTYPE_F32 ? 4 : 2;
@@ -1355,10 +1357,8 @@ int kda_layer_fwd(hipStream_t stream, const void* qp, const void* kp, const void
     const int rc = chunk_fwd_impl(stream, p.q, p.k, p.v, g, beta, h0, nullptr, 0, o, ht, B, T, H, d, d, 64, scale,
                                   in_dtype, KDA_DTYPE_F32, ws, chunk_bytes);
     if (rc != KDA_OK) return rc;
+    e = kda::launch_epilogue(ep, d, 0, gdt, ydt, stream);
   }
-  kda::EpilogueArgs ep{};
-  ep.o = o; ep.gate = gate; ep.y = y; ep.B = B; ep.T = T; ep.H = H; ep.eps = eps;
-  e = kda::launch_epilogue(ep, d, 0, gate_dtype == KDA_DTYPE_F32 ? 0 : 1, out_dtype == KDA_DTYPE_F32 ? 0 : 1, stream);
   if (e != hipSuccess) return hip_fail(e, "layer epilogue launch");
   return KDA_OK;
 }

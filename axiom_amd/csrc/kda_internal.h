@@ -211,8 +211,10 @@ hipError_t launch_prologue(const PrologueArgs& a, int d, int in_dt, int out_dt, 
 hipError_t launch_prologue_bwd(const PrologueBwdArgs& a, int d, int in_dt, int dx_dt, hipStream_t s);
 hipError_t launch_epilogue_bwd(const EpilogueBwdArgs& a, int d, int o_dt, int g_dt, int dy_dt, int dg_dt,
                                hipStream_t s);
-// only the conv buffer update of launch_prologue (the last K-1 inputs)
-hipError_t launch_prologue_buffers(const PrologueArgs& a, int d, int in_dt, hipStream_t s);
+// launch_epilogue (fp32 o) and the conv buffer update of launch_prologue (the
+// last K-1 inputs; bf16 projections) in one launch
+hipError_t launch_epilogue_buffers(const EpilogueArgs& a, const PrologueArgs& p, int d, int g_dt, int y_dt,
+                                   hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs& a, int d, int o_dt, int g_dt, int y_dt, hipStream_t s);
 // in_dtype: a kda_dtype_t, or kInAlphaGates (the cc_scan seam: bf16 q, k, v,
 // fp32 do; g = alpha, beta = beta32 [token-head][32], dg = dalpha, dbeta =

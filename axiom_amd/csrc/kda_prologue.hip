@@ -175,30 +175,54 @@ __global__ __launch_bounds__(64 * kRowsPerBlock) void kda_prologue_kernel(Prolog
 
 // new conv buffers: the last K-1 inputs of (old buffer ++ x), one thread per
 // (tensor, b, channel); every old value a thread needs is read before it writes.
-template <int DI, int D>
-__global__ __launch_bounds__(256) void kda_prologue_buf_kernel(PrologueArgs a) {
-  const int HD = a.H * D;
-  const int64_t n = 3LL * a.B * HD;
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (id >= n) return;
-  const int tensor = static_cast<int>(id / (static_cast<int64_t>(a.B) * HD));
-  const int64_t rem = id - tensor * static_cast<int64_t>(a.B) * HD;
-  const int b = static_cast<int>(rem / HD), c = static_cast<int>(rem - static_cast<int64_t>(b) * HD);
-  const void* x = tensor == 0 ? a.qp : tensor == 1 ? a.kp : a.vp;
-  const float* bin = tensor == 0 ? a.bq_in : tensor == 1 ? a.bk_in : a.bv_in;
-  float* bout = tensor == 0 ? a.bq_out : tensor == 1 ? a.bk_out : a.bv_out;
+constexpr int kBufThreads = 256;
+
+template <int DI>
+__device__ __forceinline__ void conv_buf_column(const void* x, const float* bin, float* bout, int b, int c, int T, int K,
+                                                int HD) {
   if (bout == nullptr) return;
   constexpr int KMAX = 8;
-  float v[KMAX - 1];
-  const int km1 = a.K - 1;
-  for (int j = 0; j < km1; ++j) {
-    const int src = a.T - km1 + j;                 // row of (old ++ x) relative to x
-    float val = 0.f;
-    if (src >= 0) val = pl_ld<DI>(x, (static_cast<int64_t>(b) * a.T + src) * HD + c);
-    else if (bin != nullptr) val = bin[(static_cast<int64_t>(b) * km1 + (km1 + src)) * HD + c];
-    v[j] = val;
+  float v[KMAX - 1];                               // (unrolled: in registers)
+  const int km1 = K - 1;
+#pragma unroll
+  for (int j = 0; j < KMAX - 1; ++j) {
+    const int src = T - km1 + j;                 // row of (old ++ x) relative to x
+    v[j] = 0.f;
+    if (j < km1) {
+      if (src >= 0) v[j] = pl_ld<DI>(x, (static_cast<int64_t>(b) * T + src) * HD + c);
+      else if (bin != nullptr) v[j] = bin[(static_cast<int64_t>(b) * km1 + (km1 + src)) * HD + c];
+    }
   }
-  for (int j = 0; j < km1; ++j) bout[(static_cast<int64_t>(b) * km1 + j) * HD + c] = v[j];
+#pragma unroll
+  for (int j = 0; j < KMAX - 1; ++j)
+    if (j < km1) bout[(static_cast<int64_t>(b) * km1 + j) * HD + c] = v[j];
+}
+
+template <int DI, int D>
+__device__ __forceinline__ void prologue_buf_block(const PrologueArgs& a, int block) {
+  const int HD = a.H * D;
+  const int64_t n = 3LL * a.B * HD;
+  const int64_t id = static_cast<int64_t>(block) * kBufThreads + threadIdx.x;
+  if (id >= n) return;
+  // (B H D is a multiple of 64: a wave stays within one tensor, so the three
+  // branches below are scalar and no pointer is selected through memory)
+  const int tensor = __builtin_amdgcn_readfirstlane(static_cast<int>(id / (static_cast<int64_t>(a.B) * HD)));
+  const int64_t rem = id - tensor * static_cast<int64_t>(a.B) * HD;
+  const int b = static_cast<int>(rem / HD), c = static_cast<int>(rem - static_cast<int64_t>(b) * HD);
+  if (tensor == 0) conv_buf_column<DI>(a.qp, a.bq_in, a.bq_out, b, c, a.T, a.K, HD);
+  else if (tensor == 1) conv_buf_column<DI>(a.kp, a.bk_in, a.bk_out, b, c, a.T, a.K, HD);
+  else conv_buf_column<DI>(a.vp, a.bv_in, a.bv_out, b, c, a.T, a.K, HD);
+}
+
+template <int D>
+int prologue_buf_blocks(const PrologueArgs& a) {
+  if (!(a.bq_out || a.bk_out || a.bv_out) || a.K <= 1) return 0;
+  return static_cast<int>((3LL * a.B * a.H * D + kBufThreads - 1) / kBufThreads);
+}
+
+template <int DI, int D>
+__global__ __launch_bounds__(kBufThreads) void kda_prologue_buf_kernel(PrologueArgs a) {
+  prologue_buf_block<DI, D>(a, blockIdx.x);
 }
 
 // Four consecutive channels per lane: a row of D channels is D/4 lanes (a
@@ -232,13 +256,13 @@ __device__ __forceinline__ void ep_st4(void* p, int64_t i, const f4& v) {
 }
 
 template <int DO_, int DG, int DY, int D>
-__global__ __launch_bounds__(kEpiThreads) void kda_epilogue_kernel(EpilogueArgs a) {
+__device__ __forceinline__ void epilogue_rows(const EpilogueArgs& a, int block, int nblocks) {
   constexpr int LPR = D / 4;                    // lanes per row
   constexpr int RPB = kEpiThreads / LPR;        // rows per workgroup step
   const int64_t rows = static_cast<int64_t>(a.B) * a.T * a.H;
   const int sub = threadIdx.x % LPR;
-  for (int64_t r = static_cast<int64_t>(blockIdx.x) * RPB + threadIdx.x / LPR; r < rows;
-       r += static_cast<int64_t>(gridDim.x) * RPB) {   // a row's lanes share r: uniform per group
+  for (int64_t r = static_cast<int64_t>(block) * RPB + threadIdx.x / LPR; r < rows;
+       r += static_cast<int64_t>(nblocks) * RPB) {   // a row's lanes share r: uniform per group
     const int64_t i = r * D + 4 * sub;
     const f4 o = ep_ld4<DO_>(a.o, i);
     const f4 g = ep_ld4<DG>(a.gate, i);
@@ -253,6 +277,24 @@ __global__ __launch_bounds__(kEpiThreads) void kda_epilogue_kernel(EpilogueArgs 
     for (int e = 0; e < 4; ++e) y[e] = sigmoid_f32(g[e]) * o[e] * inv;
     ep_st4<DY>(a.y, i, y);
   }
+}
+
+template <int DO_, int DG, int DY, int D>
+__global__ __launch_bounds__(kEpiThreads) void kda_epilogue_kernel(EpilogueArgs a) {
+  epilogue_rows<DO_, DG, DY, D>(a, blockIdx.x, gridDim.x);
+}
+
+// The fused layer's epilogue (fp32 o) and its conv buffer update (bf16
+// projections) in one launch: the update waits for the scan only because the
+// buffers may be rewritten in place, and a launch of its own costs a small call
+// more than its work (B1 T333 H16 d128: 3.6 of 34.8 us).  The first nbuf
+// workgroups update the buffers.
+template <int DG, int DY, int D>
+__global__ __launch_bounds__(kEpiThreads) void kda_epilogue_buf_kernel(EpilogueArgs a, PrologueArgs p, int nbuf) {
+  static_assert(kEpiThreads == kBufThreads, "one workgroup size");
+  const int x = blockIdx.x;
+  if (x < nbuf) prologue_buf_block<1, D>(p, x);
+  else epilogue_rows<0, DG, DY, D>(a, x - nbuf, gridDim.x - nbuf);
 }
 
 template <int D, int KW, int RW, bool BUF>
@@ -286,33 +328,38 @@ hipError_t launch_prologue_d(const PrologueArgs& a, int in_dt, int out_dt, hipSt
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  if ((a.bq_out || a.bk_out || a.bv_out) && a.K > 1) {
-    const int64_t n = 3LL * a.B * a.H * D;
-    const int g = static_cast<int>((n + 255) / 256);
-    if (in_dt == 0) hipLaunchKernelGGL((kda_prologue_buf_kernel<0, D>), dim3(g), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((kda_prologue_buf_kernel<1, D>), dim3(g), dim3(256), 0, s, a);
+  if (const int g = prologue_buf_blocks<D>(a)) {
+    if (in_dt == 0) hipLaunchKernelGGL((kda_prologue_buf_kernel<0, D>), dim3(g), dim3(kBufThreads), 0, s, a);
+    else hipLaunchKernelGGL((kda_prologue_buf_kernel<1, D>), dim3(g), dim3(kBufThreads), 0, s, a);
     return hipGetLastError();
   }
   return hipSuccess;
 }
 
 template <int D>
-hipError_t launch_prologue_buffers_d(const PrologueArgs& a, int in_dt, hipStream_t s) {
-  if (!(a.bq_out || a.bk_out || a.bv_out) || a.K <= 1) return hipSuccess;
-  const int64_t n = 3LL * a.B * a.H * D;
-  const int g = static_cast<int>((n + 255) / 256);
-  if (in_dt == 0) hipLaunchKernelGGL((kda_prologue_buf_kernel<0, D>), dim3(g), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((kda_prologue_buf_kernel<1, D>), dim3(g), dim3(256), 0, s, a);
+int epilogue_blocks(const EpilogueArgs& a) {
+  const int64_t rows = static_cast<int64_t>(a.B) * a.T * a.H;
+  constexpr int RPB = kEpiThreads / (D / 4);
+  const int64_t need = (rows + RPB - 1) / RPB;
+  return static_cast<int>(need < 8192 ? need : 8192);   // 32 workgroups per CU, grid-strided
+}
+
+template <int D>
+hipError_t launch_epilogue_buffers_d(const EpilogueArgs& a, const PrologueArgs& p, int g_dt, int y_dt, hipStream_t s) {
+  const int nbuf = prologue_buf_blocks<D>(p);
+  const dim3 grid(nbuf + epilogue_blocks<D>(a)), blk(kEpiThreads);
+  if (grid.x == 0) return hipSuccess;
+  if (g_dt == 0 && y_dt == 0) hipLaunchKernelGGL((kda_epilogue_buf_kernel<0, 0, D>), grid, blk, 0, s, a, p, nbuf);
+  else if (g_dt == 0) hipLaunchKernelGGL((kda_epilogue_buf_kernel<0, 1, D>), grid, blk, 0, s, a, p, nbuf);
+  else if (y_dt == 0) hipLaunchKernelGGL((kda_epilogue_buf_kernel<1, 0, D>), grid, blk, 0, s, a, p, nbuf);
+  else hipLaunchKernelGGL((kda_epilogue_buf_kernel<1, 1, D>), grid, blk, 0, s, a, p, nbuf);
   return hipGetLastError();
 }
 
 template <int D>
 hipError_t launch_epilogue_d(const EpilogueArgs& a, int o_dt, int g_dt, int y_dt, hipStream_t s) {
-  const int64_t rows = static_cast<int64_t>(a.B) * a.T * a.H;
-  if (rows == 0) return hipSuccess;
-  constexpr int RPB = kEpiThreads / (D / 4);
-  const int64_t need = (rows + RPB - 1) / RPB;
-  const int grid = static_cast<int>(need < 8192 ? need : 8192);   // 32 workgroups per CU, grid-strided
+  const int grid = epilogue_blocks<D>(a);
+  if (grid == 0) return hipSuccess;
   const int code = o_dt * 4 + g_dt * 2 + y_dt;
   switch (code) {
     case 0: hipLaunchKernelGGL((kda_epilogue_kernel<0, 0, 0, D>), dim3(grid), dim3(kEpiThreads), 0, s, a); break;
@@ -694,8 +741,9 @@ hipError_t launch_prologue(const PrologueArgs& a, int d, int in_dt, int out_dt, 
   return d == 128 ? launch_prologue_d<128>(a, in_dt, out_dt, s) : launch_prologue_d<64>(a, in_dt, out_dt, s);
 }
 
-hipError_t launch_prologue_buffers(const PrologueArgs& a, int d, int in_dt, hipStream_t s) {
-  return d == 128 ? launch_prologue_buffers_d<128>(a, in_dt, s) : launch_prologue_buffers_d<64>(a, in_dt, s);
+hipError_t launch_epilogue_buffers(const EpilogueArgs& a, const PrologueArgs& p, int d, int g_dt, int y_dt,
+                                   hipStream_t s) {
+  return d == 128 ? launch_epilogue_buffers_d<128>(a, p, g_dt, y_dt, s) : launch_epilogue_buffers_d<64>(a, p, g_dt, y_dt, s);
 }
 
 hipError_t launch_epilogue(const EpilogueArgs& a, int d, int o_dt, int g_dt, int y_dt, hipStream_t s) {
