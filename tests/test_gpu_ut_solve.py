@@ -94,3 +94,37 @@ def test_autograd_function_routes_through_the_backward_rule(cuda):
         da, db = axiom_amd.ut_solve_bwd(at.detach(), x.detach(), dx, transpose=tr)
         torch.cuda.synchronize()
         assert torch.equal(at.grad, da) and torch.equal(bt.grad, db)
+
+
+@pytest.mark.parametrize("H,C,N", [(1, 1, 1), (3, 15, 63), (2, 16, 64), (5, 17, 65), (2, 33, 130), (1, 48, 200), (3, 64, 7)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_backward_tiles(cuda, H, C, N, dtype, transpose):
+    """(dA, dB) at the edges of the 16-row and 64-column tiles, against 64 bits on the same x.
+
+    fp32: at most C + N = 248 rounded sums, 248 * 2^-24 = 1.5e-5 if every rounding went the same way;
+    bf16: half a unit, 2^-9 of each value stored (dA from the db before its rounding or after it).
+    The call whose dB is written over dX solves with two launches: the same dB.
+    """
+    import axiom_amd
+    from axiom_amd import _lib
+    a, b = _inputs(H, C, N, seed=31 * C + N)
+    dx = np.random.default_rng(5).standard_normal((H, C, N)).astype(np.float32)
+    at, bt, dxt = (torch.from_numpy(v).to(cuda, dtype) for v in (a, b, dx))
+    x = axiom_amd.ut_solve(at, bt, transpose=transpose)
+    da, db = axiom_amd.ut_solve_bwd(at, x, dxt, transpose=transpose)
+    da2, db2 = torch.full_like(at, float("nan")), dxt.clone()
+    code = _lib.KDA_DTYPE_F32 if dtype == torch.float32 else _lib.KDA_DTYPE_BF16
+    assert _lib.lib().kda_ut_solve_bwd(torch.cuda.current_stream().cuda_stream, at.data_ptr(), x.data_ptr(),
+                                       db2.data_ptr(), da2.data_ptr(), db2.data_ptr(), H, C, N, code,
+                                       int(transpose)) == 0
+    torch.cuda.synchronize()
+    db_ref = _exact(at.double().cpu(), dxt.double().cpu(), not transpose)
+    x64 = x.double().cpu()
+    da_ref = -torch.tril(x64 @ db_ref.transpose(1, 2) if transpose else db_ref @ x64.transpose(1, 2), -1)
+    bound = 1.5e-5 if dtype == torch.float32 else 2.0 ** -8
+    for got in (da, da2):
+        assert torch.count_nonzero(torch.triu(got)) == 0
+        assert float((got.double().cpu() - da_ref).norm()) <= bound * max(float(da_ref.norm()), 1e-30)
+    assert float((db.double().cpu() - db_ref).norm()) <= bound * float(db_ref.norm())
+    assert torch.equal(db, db2)
