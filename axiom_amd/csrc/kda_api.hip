@@ -1004,13 +1004,20 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   // from the chunk kernel) when every pointer allows their 16-byte (dq, dk,
   // dv: 4-byte) accesses; a pass before and one after the dense backward
   // cost 42 and 126 us at B2 T8192 H12 d128.  Other pointers keep those two
-  // passes, whose element-wise forms take any alignment.
+  // passes, whose element-wise forms take any alignment, and so do gradients
+  // over inputs: there every input is read before the last pass writes.
   const uintptr_t a16 = reinterpret_cast<uintptr_t>(alpha) | reinterpret_cast<uintptr_t>(beta32) |
                         reinterpret_cast<uintptr_t>(dbeta32);
   const uintptr_t a4 = reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) |
                        reinterpret_cast<uintptr_t>(dv) | reinterpret_cast<uintptr_t>(dalpha);
   const int64_t nt = (T + kC - 1) / kC;
-  if (T > 0 && (a16 & 15) == 0 && (a4 & 3) == 0 && static_cast<int64_t>(B) * nt * H <= 0x7FFFFFFFLL &&
+  const int64_t bh = static_cast<int64_t>(th) * dk_dim * 2, bf = 2 * bh, b32n = static_cast<int64_t>(th) * 128;
+  const struct { const void* p; int64_t n; } in[] = {{q, bh}, {k, bh}, {v, bh}, {alpha, bf}, {beta32, b32n}, {d_o, bf}},
+                                             grad[] = {{dq, bh}, {dk, bh}, {dv, bh}, {dalpha, bf}, {dbeta32, b32n}};
+  bool apart = true;
+  for (const auto& x : grad)
+    for (const auto& y : in) apart = apart && !kda::overlaps(x.p, x.n, y.p, y.n);
+  if (T > 0 && apart && (a16 & 15) == 0 && (a4 & 3) == 0 && static_cast<int64_t>(B) * nt * H <= 0x7FFFFFFFLL &&
       th * dk_dim < (1ULL << 40)) {
     kda::BwdArgs a{};
     a.B = B; a.T = T; a.H = H; a.NT = static_cast<int>(nt);
@@ -1345,7 +1352,14 @@ int kda_layer_fwd(hipStream_t stream, const void* qp, const void* kp, const void
                                   in_dtype, KDA_DTYPE_F32, ws, chunk_bytes, &fp);
     if (rc != KDA_OK) return rc;
     // the buffers are rewritten after every read of the old ones, beside the epilogue
-    e = kda::launch_epilogue_buffers(ep, p, d, gdt, ydt, stream);
+    const int64_t nx = static_cast<int64_t>(B) * T * H * d * 2, ny = ydt == 0 ? 2 * nx : nx;   // bf16 projections
+    if (kda::overlaps(y, ny, qp, nx) || kda::overlaps(y, ny, kp, nx) || kda::overlaps(y, ny, vp, nx)) {
+      e = kda::launch_epilogue_buffers(kda::EpilogueArgs{}, p, d, gdt, ydt, stream);   // the buffers alone
+      if (e != hipSuccess) return hip_fail(e, "layer conv buffer launch");
+      e = kda::launch_epilogue(ep, d, 0, gdt, ydt, stream);
+    } else {
+      e = kda::launch_epilogue_buffers(ep, p, d, gdt, ydt, stream);
+    }
   } else {
     const size_t n = static_cast<size_t>(B) * T * H * d;
     const size_t es = in_dtype == KDA_DTYPE_F32 ? 4 : 2;

@@ -2070,7 +2070,7 @@ struct Col4 {
 };
 
 // ---------------------------------------------------------------------------
-// per chunk-head adjoint: one 512-thread workgroup per chunk-head, four
+// per chunk-head adjoint: one workgroup per chunk-head (ChunkThreads), four
 // phases separated by workgroup barriers, every phase in the same thread
 // mapping so the partial dq, dk, dG stay in registers and each output is
 // stored once:
@@ -2804,11 +2804,20 @@ hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t s) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int scan_grid = (chains + 7) / 8 * 8 * (D / 32);   // workgroups of either scan
-  if constexpr (DTQ != 0)
-    hipLaunchKernelGGL((kda_bwd_scans16_kernel<D, DO>), dim3(2 * scan_grid), dim3(64 * (2 + kRsProducers)), 0, s, a, scan_grid);
-  else
-    hipLaunchKernelGGL((kda_bwd_scans_kernel<D, DO>), dim3(2 * scan_grid), dim3(ScanThreads<D>::value), 0, s, a, scan_grid);
-  e = hipGetLastError();
+  auto scans = [&](int grid, int nblk) {   // the first nblk workgroups run the reverse scan
+    if constexpr (DTQ != 0)
+      hipLaunchKernelGGL((kda_bwd_scans16_kernel<D, DO>), dim3(grid), dim3(64 * (2 + kRsProducers)), 0, s, a, nblk);
+    else
+      hipLaunchKernelGGL((kda_bwd_scans_kernel<D, DO>), dim3(grid), dim3(ScanThreads<D>::value), 0, s, a, nblk);
+    return hipGetLastError();
+  };
+  const int64_t state_bytes = static_cast<int64_t>(chains) * D * D * 4;
+  if (overlaps(a.dh0, state_bytes, a.h0, state_bytes)) {   // dh0 over h0: the forward scan reads h0 first
+    e = scans(scan_grid, 0);
+    if (e == hipSuccess) e = scans(scan_grid, scan_grid);
+  } else {
+    e = scans(2 * scan_grid, scan_grid);
+  }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((kda_bwd_chunk_kernel<D, DTQ, DTG, DO>), dim3(chunk_heads), dim3(ChunkThreads<D>::value), 0, s, a);
   return hipGetLastError();

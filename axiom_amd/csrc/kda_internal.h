@@ -146,6 +146,13 @@ struct BwdArgs {
 };
 
 // Standalone unit-triangular solve (kda_ut.hip); a [H][C][C], b/x/xf [H][C][N].
+// Whether two byte ranges share memory (never where one has no address).  Launches
+// that were joined keep their order for calls whose outputs lie over their inputs.
+inline bool overlaps(const void* p, int64_t pn, const void* q, int64_t qn) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
+  return p != nullptr && q != nullptr && x < y + static_cast<uintptr_t>(qn) && y < x + static_cast<uintptr_t>(pn);
+}
+
 struct UtArgs {
   const void* a;
   const void* b;    // right-hand side (the cotangent dX in the backward rule)

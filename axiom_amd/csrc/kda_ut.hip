@@ -250,11 +250,6 @@ __global__ __launch_bounds__(kUtThreads) void kda_ut_bwd_kernel(UtArgs a) {
   }
 }
 
-bool overlaps(const void* p, int64_t pn, const void* q, int64_t qn) {
-  const uintptr_t x = reinterpret_cast<uintptr_t>(p), y = reinterpret_cast<uintptr_t>(q);
-  return x < y + static_cast<uintptr_t>(qn) && y < x + static_cast<uintptr_t>(pn);
-}
-
 template <int DT>
 hipError_t launch_ut_t(const UtArgs& a, bool transpose, bool with_da, hipStream_t s) {
   if (with_da) {
