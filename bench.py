@@ -275,7 +275,7 @@ def bench_backward(args, fwd_inputs, device):
                 roofline={"bound": "hbm", "achieved": gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                           "frac": gbps / HBM_PEAK_GBPS, "algorithmic_bytes_per_call": nbytes,
                           "traffic": measured_traffic("backward_traffic_bytes_per_call")},
-                kernels="kda_bwd_prep + kda_bwd_fscan16 + kda_bwd_rscan16 + kda_bwd_chunk (fp16 forward-side "
+                kernels="kda_bwd_prep + kda_bwd_scans16 + kda_bwd_chunk (fp16 forward-side "
                         "workspace, fp32 cotangents; fp16 and bf16 hi/lo products)",
                 config="B4 T4096 H16 d128 bf16 inputs, fp32 do and dht, zero h0")
 
