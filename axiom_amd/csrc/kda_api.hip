@@ -1005,15 +1005,17 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   // dv: 4-byte) accesses; a pass before and one after the dense backward
   // cost 42 and 126 us at B2 T8192 H12 d128.  Other pointers keep those two
   // passes, whose element-wise forms take any alignment, and so do gradients
-  // over inputs: there every input is read before the last pass writes.
+  // over inputs: there every input is read before the last pass writes, and
+  // beta32 before the scans write dS_in.
   const uintptr_t a16 = reinterpret_cast<uintptr_t>(alpha) | reinterpret_cast<uintptr_t>(beta32) |
                         reinterpret_cast<uintptr_t>(dbeta32);
   const uintptr_t a4 = reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) |
                        reinterpret_cast<uintptr_t>(dv) | reinterpret_cast<uintptr_t>(dalpha);
   const int64_t nt = (T + kC - 1) / kC;
   const int64_t bh = static_cast<int64_t>(th) * dk_dim * 2, bf = 2 * bh, b32n = static_cast<int64_t>(th) * 128;
+  const int64_t st = static_cast<int64_t>(B) * H * dk_dim * dv_dim * 4;
   const struct { const void* p; int64_t n; } in[] = {{q, bh}, {k, bh}, {v, bh}, {alpha, bf}, {beta32, b32n}, {d_o, bf}},
-                                             grad[] = {{dq, bh}, {dk, bh}, {dv, bh}, {dalpha, bf}, {dbeta32, b32n}};
+                                             grad[] = {{dq, bh}, {dk, bh}, {dv, bh}, {dalpha, bf}, {dbeta32, b32n}, {dS_in, st}};
   bool apart = true;
   for (const auto& x : grad)
     for (const auto& y : in) apart = apart && !kda::overlaps(x.p, x.n, y.p, y.n);

@@ -37,8 +37,6 @@ def test_dh0_over_h0(cuda, B, H, d, prec):
         assert torch.equal(a, w), i
 
 
-
-
 @pytest.mark.parametrize("T,H,d", [(96, 2, 128), (64, 3, 64)])
 def test_seam_gradients_over_their_primals(cuda, T, H, d):
     import axiom_amd
@@ -62,6 +60,32 @@ def test_seam_gradients_over_their_primals(cuda, T, H, d):
     assert rc == 0
     for i, (a, w) in enumerate(zip(ops, want)):
         assert a.dtype == w.dtype and torch.equal(a, w), i
+
+
+@pytest.mark.parametrize("T,H,d,skip", [(512, 1, 128, 0), (1024, 2, 128, 64), (256, 3, 64, 0)])
+def test_seam_state_gradient_over_beta(cuda, T, H, d, skip):
+    """dS_in over part of beta32 (from element ``skip`` on): beta32 is read before the scans write dS_in."""
+    import axiom_amd
+    from axiom_amd import _lib, kda
+    x = inputs.make_inputs(1, T, H, d, d, seed=T, dtype="bf16", h0_std=0.05)
+    ops = [to_dev(x[n][0].reshape(T, H * d), torch.bfloat16, cuda) for n in ("q", "k", "v")]
+    ops.append(to_dev(np.exp(x["g"][0]).reshape(T, H * d), torch.float32, cuda))
+    ops.append(to_dev(np.repeat(x["beta"][0], 32, axis=-1), torch.float32, cuda))
+    ops.append(to_dev(x["h0"][0], torch.float32, cuda))
+    do, dS = torch.randn(T, H * d, device=cuda), torch.randn(H, d, d, device=cuda)
+    want = axiom_amd.cc_scan_bwd(*ops, do, dS, chunk=32)
+    outs = [torch.empty_like(t) for t in want[:5]]
+    dS_in = ops[4].view(-1)[skip:skip + H * d * d]
+    assert dS_in.numel() == H * d * d
+    ws = torch.empty(kda._ws_bytes("kda_cc_scan_bwd_batched_workspace", 1, T, H, d, d, 32), dtype=torch.uint8,
+                     device=cuda)
+    p = [t.data_ptr() for t in (*ops, do, dS, *outs, dS_in)]
+    rc = _lib.lib().kda_cc_scan_bwd_batched(kda._stream(do.device), *p, 1, T, H, d, d, 16, 32, ws.data_ptr(),
+                                            ws.numel())
+    torch.cuda.synchronize()
+    assert rc == 0
+    for i, (a, w) in enumerate(zip((*outs, dS_in.view(H, d, d)), want)):
+        assert torch.equal(a, w), i
 
 
 @pytest.mark.parametrize("T,over", [(2, 0), (333, 1), (130, 2)])
