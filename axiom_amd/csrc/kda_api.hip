@@ -1353,9 +1353,17 @@ int kda_layer_fwd(hipStream_t stream, const void* qp, const void* kp, const void
     const int rc = chunk_fwd_impl(stream, qp, kp, vp, g, beta, h0, nullptr, 0, o, ht, B, T, H, d, d, 64, scale,
                                   in_dtype, KDA_DTYPE_F32, ws, chunk_bytes, &fp);
     if (rc != KDA_OK) return rc;
-    // the buffers are rewritten after every read of the old ones, beside the epilogue
-    const int64_t nx = static_cast<int64_t>(B) * T * H * d * 2, ny = ydt == 0 ? 2 * nx : nx;   // bf16 projections
-    if (kda::overlaps(y, ny, qp, nx) || kda::overlaps(y, ny, kp, nx) || kda::overlaps(y, ny, vp, nx)) {
+    // the buffers are rewritten after every read of the old ones, beside the
+    // epilogue unless either part writes what the other reads or writes: then
+    // the buffers first (bf16 projections; the old buffers are read if T < K - 1)
+    const int64_t n = static_cast<int64_t>(B) * T * H * d, nb = static_cast<int64_t>(B) * (K - 1) * H * d * 4;
+    const int64_t ny = n * (ydt == 0 ? 4 : 2), ng = n * (gdt == 0 ? 4 : 2);
+    bool apart = true;
+    for (const void* x : {qp, kp, vp}) apart = apart && !kda::overlaps(y, ny, x, 2 * n);
+    for (const float* x : {bq_in, bk_in, bv_in}) apart = apart && !kda::overlaps(y, ny, x, nb);
+    for (const float* x : {bq_out, bk_out, bv_out})
+      apart = apart && !kda::overlaps(x, nb, y, ny) && !kda::overlaps(x, nb, gate, ng) && !kda::overlaps(x, nb, o, 4 * n);
+    if (!apart) {
       e = kda::launch_epilogue_buffers(kda::EpilogueArgs{}, p, d, gdt, ydt, stream);   // the buffers alone
       if (e != hipSuccess) return hip_fail(e, "layer conv buffer launch");
       e = kda::launch_epilogue(ep, d, 0, gdt, ydt, stream);

@@ -109,3 +109,28 @@ def test_layer_output_over_a_projection(cuda, T, over):
     assert torch.equal(xs[over], y) and torch.equal(ht2, ht)
     for a, b in zip(bufs, new):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("K,T,over", [(4, 1, 0), (4, 2, 2), (3, 1, 1)])
+@pytest.mark.parametrize("B,H,d", [(1, 2, 64), (4, 16, 128)])
+def test_layer_output_over_an_incoming_buffer(cuda, K, T, over, B, H, d):
+    """A call of fewer than K - 1 tokens reads the old buffers; y lies over one, the new ones are elsewhere."""
+    from axiom_amd import _lib, kda
+    xs = [torch.randn(B, T, H * d, device=cuda).to(torch.bfloat16) for _ in range(4)]
+    gb = [(-torch.rand(B, T, H, d, device=cuda)).to(torch.bfloat16), torch.rand(B, T, H, device=cuda).to(torch.bfloat16)]
+    w = [torch.randn(K, H * d, device=cuda) * 0.4 for _ in range(3)]
+    bufs = [torch.randn(B, K - 1, H * d, device=cuda) for _ in range(3)]
+    y, ht, new = kda.kda_layer_fwd(*xs[:3], *gb, xs[3], *w, conv_state=tuple(bufs))
+    ws = torch.empty(kda._ws_bytes("kda_layer_fwd_workspace", B, T, H, d, K, _lib.KDA_DTYPE_BF16), dtype=torch.uint8,
+                     device=cuda)
+    ht2, new2 = torch.empty_like(ht), [torch.empty_like(b) for b in bufs]
+    p = [t.data_ptr() for t in (*xs[:3], *gb, xs[3], *w, *bufs, *new2)]
+    rc = _lib.lib().kda_layer_fwd(kda._stream(y.device), *p, None, ht2.data_ptr(), bufs[over].data_ptr(), None,
+                                  B, T, H, d, K, 1.0, 1e-6, _lib.KDA_DTYPE_BF16, _lib.KDA_DTYPE_BF16,
+                                  _lib.KDA_DTYPE_BF16, ws.data_ptr(), ws.numel())
+    torch.cuda.synchronize()
+    assert rc == 0
+    got = bufs[over].view(torch.bfloat16).view(-1)[:y.numel()].view(y.shape)
+    assert torch.equal(got, y) and torch.equal(ht2, ht)
+    for a, b in zip(new2, new):
+        assert torch.equal(a, b)
