@@ -10,7 +10,7 @@
 // and the B tile go to LDS (all of a thread's loads in flight together),
 // T = (I + L)^-1 is formed there (kda_tri.h), and X = T B (or T^T B) runs on
 // the fp32 matrix cores.  Padding rows/columns beyond C and N are zero and
-// never stored.  The backward rule is one launch of its own kernel (below).
+// never stored.  The backward rule of few heads is one launch of its own kernel (below).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -78,7 +78,8 @@ __device__ __forceinline__ void ut_tile_load(float* dst, const void* src, int64_
   ut_tile_store(dst, v);
 }
 
-// X = T B (or T^T B; the backward rule's dB with B = dX) on the fp32 matrix cores: wave w owns row tile w and the four column tiles.
+// X = T B (or T^T B; the backward rule's dB with B = dX) on the fp32 matrix
+// cores: wave w owns row tile w and the four column tiles.
 template <int DT, bool TR>
 __global__ __launch_bounds__(kUtThreads) void kda_ut_solve_kernel(UtArgs a) {
   __shared__ float sL[kN * kPC], sT[kN * kPC], sB[kN * kPC], tmp[768];
@@ -250,16 +251,27 @@ __global__ __launch_bounds__(kUtThreads) void kda_ut_bwd_kernel(UtArgs a) {
   }
 }
 
+constexpr int kUtOneRound = 512;   // two workgroups (LDS) on each of 256 CUs
+
 template <int DT>
 hipError_t launch_ut_t(const UtArgs& a, bool transpose, bool with_da, hipStream_t s) {
   if (with_da) {
-    // One launch unless an output shares memory with an input: workgroups of one
+    // One launch while its workgroups (16 rows of a head each) run in one round, two
+    // a CU, or, with at most 32 rows, form no more inverses than the solve's column
+    // tiles would: past that each row tile's own inverse and reads of X and dX cost
+    // more than the second launch.  us in two launches and in one, fp32: C 64 N 64,
+    // 128 heads 12.8 and 10.6, 192 13.1 and 18.2, 1 024 34.0 and 69.2; C 64 N 1 024,
+    // 128 heads 72.5 and 67.3, 192 84.8 and 105; C 32, 1 024 heads, N 64 28.5 and
+    // 33.7, N 128 48.9 and 43.1, N 512 174 and 99; C 16 N 64, 1 024 heads 26.0 and 17.9.
+    // Two launches also where an output shares memory with an input: workgroups of one
     // head read all of a, dX and X while others write, where the two launches
     // read a head's a and a column's dX before they write over them.
+    const int rtiles = (a.C + 15) / 16;
+    const bool one = static_cast<int64_t>(a.H) * rtiles <= kUtOneRound || (rtiles <= 2 && rtiles <= a.ntiles);
     const int64_t es = DT == 0 ? 4 : 2, na = es * a.H * a.C * a.C, nb = es * a.H * a.C * a.N;
     auto apart = [&](const void* in, int64_t n) { return !overlaps(a.x, nb, in, n) && !overlaps(a.da, na, in, n); };
-    if (apart(a.a, na) && apart(a.b, nb) && apart(a.xf, nb)) {
-      const dim3 grid(a.H * ((a.C + 15) / 16));
+    if (one && apart(a.a, na) && apart(a.b, nb) && apart(a.xf, nb)) {
+      const dim3 grid(a.H * rtiles);
       if (transpose) hipLaunchKernelGGL((kda_ut_bwd_kernel<DT, true>), grid, dim3(kUtThreads), 0, s, a);
       else hipLaunchKernelGGL((kda_ut_bwd_kernel<DT, false>), grid, dim3(kUtThreads), 0, s, a);
       return hipGetLastError();

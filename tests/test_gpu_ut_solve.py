@@ -128,3 +128,33 @@ def test_backward_tiles(cuda, H, C, N, dtype, transpose):
         assert float((got.double().cpu() - da_ref).norm()) <= bound * max(float(da_ref.norm()), 1e-30)
     assert float((db.double().cpu() - db_ref).norm()) <= bound * float(db_ref.norm())
     assert torch.equal(db, db2)
+
+
+@pytest.mark.parametrize("H,C,N,two", [(128, 64, 64, False), (129, 64, 64, True), (171, 48, 200, True), (256, 32, 64, False),
+                                       (257, 32, 64, True), (257, 32, 65, False), (600, 16, 64, False), (600, 64, 7, True)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_backward_of_many_heads(cuda, H, C, N, two, transpose):
+    """The rule between one launch and two, at its edges.  Two launches form dA from dB as stored, one
+    from dB before its rounding to bf16: the same dA bits as the call whose dB lies over dX (always two
+    launches) tell which ran.  The bounds as in ``test_backward_tiles``."""
+    import axiom_amd
+    from axiom_amd import _lib
+    g = torch.Generator(device=cuda).manual_seed(H + N)
+    R = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    at = (torch.eye(C, device=cuda) + torch.tril(0.1 * R(H, C, C), -1)).bfloat16()
+    bt, dxt = R(H, C, N).bfloat16(), R(H, C, N).bfloat16()
+    x = axiom_amd.ut_solve(at, bt, transpose=transpose)
+    da, db = axiom_amd.ut_solve_bwd(at, x, dxt, transpose=transpose)
+    da2, db2 = torch.full_like(at, float("nan")), dxt.clone()
+    assert _lib.lib().kda_ut_solve_bwd(torch.cuda.current_stream().cuda_stream, at.data_ptr(), x.data_ptr(),
+                                       db2.data_ptr(), da2.data_ptr(), db2.data_ptr(), H, C, N, _lib.KDA_DTYPE_BF16,
+                                       int(transpose)) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(db, db2)
+    assert torch.equal(da, da2) == two
+    db_ref = _exact(at.double().cpu(), dxt.double().cpu(), not transpose)
+    x64 = x.double().cpu()
+    da_ref = -torch.tril(x64 @ db_ref.transpose(1, 2) if transpose else db_ref @ x64.transpose(1, 2), -1)
+    assert torch.count_nonzero(torch.triu(da)) == 0
+    for got, ref in ((da, da_ref), (db, db_ref)):
+        assert float((got.double().cpu() - ref).norm()) <= 2.0 ** -8 * float(ref.norm())
