@@ -1985,6 +1985,21 @@ __global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_scans_kernel(Bw
   else fscan_block<D, false>(a, x - nblk, *reinterpret_cast<FscanLds<D>*>(sm));
 }
 
+// The forward scan alone, in LDS of its own size: at d = 64 two workgroups of it
+// fit a CU, where a workgroup of the joined launch reserves the reverse scan's
+// 99 KiB and has a CU to itself.  That only tells where a chain is one chunk, so
+// that no next chunk's loads are in flight beside the step, and with workgroups
+// for many rounds (fp32, d = 64, one chunk a chain, whole backward joined and
+// apart: 512 chains 98 and 98 us, 1 024 196 and 195, 2 048 392 and 378, 4 096 758
+// and 732; 2 048 chains of 16 tokens 349 and 335).  Longer chains are faster
+// joined (132 chains of 16 chunks 392 and 444) or the same, as are 16-bit inputs.
+template <int D>
+__global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_fscan_kernel(BwdArgs a) {
+  __shared__ FscanLds<D> L;
+  fscan_block<D, false>(a, blockIdx.x, L);
+}
+constexpr int kForwardApart = 2048;   // forward scan workgroups
+
 // A 16 x 16 accumulator tile (lane (r, gq): rows 4 gq + i, column r) into
 // row-major hi / lo bf16 planes of pitch PB at (row0, col0): lanes r and r ^ 1
 // swap one value of each row pair, so each lane writes packed column pairs
@@ -2812,8 +2827,18 @@ hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t s) {
     return hipGetLastError();
   };
   const int64_t state_bytes = static_cast<int64_t>(chains) * D * D * 4;
-  if (overlaps(a.dh0, state_bytes, a.h0, state_bytes)) {   // dh0 over h0: the forward scan reads h0 first
-    e = scans(scan_grid, 0);
+  auto forward = [&]() {   // the forward scan alone
+    if constexpr (D == 64 && DTQ == 0) {
+      hipLaunchKernelGGL(kda_bwd_fscan_kernel<D>, dim3(scan_grid), dim3(ScanThreads<D>::value), 0, s, a);
+      return hipGetLastError();
+    } else {
+      return scans(scan_grid, 0);
+    }
+  };
+  // apart: see kda_bwd_fscan_kernel; and with dh0 over h0 the forward scan reads h0 first
+  if ((D == 64 && DTQ == 0 && a.NT == 1 && scan_grid >= kForwardApart) ||
+      overlaps(a.dh0, state_bytes, a.h0, state_bytes)) {
+    e = forward();
     if (e == hipSuccess) e = scans(scan_grid, scan_grid);
   } else {
     e = scans(2 * scan_grid, scan_grid);

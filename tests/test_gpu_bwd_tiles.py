@@ -52,3 +52,22 @@ def test_bwd_at_tile_edges_with_mixed_decay(cuda, T, prec, d):
         rel, mx = K.rel_l2(a, b), K.max_abs(a, b)
         print(f"  {n}: rel_l2={rel:.2e} max_abs={mx:.2e}")
         assert rel <= rel_tol and mx <= abs_tol * max(1.0, float(np.abs(b).max())), n
+
+
+@pytest.mark.parametrize("B,T", [(31, 64), (32, 64), (32, 37), (32, 65)])
+def test_many_one_chunk_chains(cuda, B, T):
+    """fp32, d = 64: the forward scan in a launch of its own from 1 024 one-chunk chains on.  A chain's
+    gradients do not depend on the others: the same bits as in a call of one batch row."""
+    import axiom_amd
+    H, d = 32, 64
+    x = inputs.make_inputs(B, T, H, d, d, seed=T, dtype="fp32", h0_std=0.1)
+    t = {n: to_dev(x[n], torch.float32, cuda) for n in x}
+    g = torch.Generator(device=cuda).manual_seed(1)
+    do, dht = torch.randn(B, T, H, d, device=cuda, generator=g), torch.randn(B, H, d, d, device=cuda, generator=g)
+    ops = [t[n] for n in ("q", "k", "v", "g", "beta")]
+    got = axiom_amd.kda_chunk_bwd(*ops, do, dht=dht, initial_state=t["h0"])
+    for b in (0, B // 2, B - 1):
+        s = slice(b, b + 1)
+        one = axiom_amd.kda_chunk_bwd(*(y[s] for y in ops), do[s], dht=dht[s], initial_state=t["h0"][s])
+        for i, (u, v) in enumerate(zip(got, one)):
+            assert torch.equal(u[s], v), (b, i)
