@@ -1,9 +1,10 @@
 """Build the gfx950 KDA library in-tree: ``axiom_amd/libkda_mi355x.so``.
 
 Every HIP source under ``axiom_amd/csrc`` is compiled with hipcc for gfx950
-only, then linked into one shared library whose exported symbols are exactly
-the C ABI of ``include/kda_mi355x.h``.  Run ``python -m axiom_amd.build`` or
-call :func:`build`.
+only, then linked into one shared library whose exported functions are the C
+ABI of ``include/kda_mi355x.h`` and the package's own entry points
+(``_lib._PRIVATE``, declared in ``csrc/kda_internal.h``).  Run ``python -m
+axiom_amd.build`` or call :func:`build`.
 """
 
 from __future__ import annotations

@@ -145,7 +145,6 @@ struct BwdArgs {
   void* FLT;            // [ch][dk/16][2][64][8]  (lambda k)^T (M channels, K rows)
 };
 
-// Standalone unit-triangular solve (kda_ut.hip); a [H][C][C], b/x/xf [H][C][N].
 // Whether two byte ranges share memory (never where one has no address).  Launches
 // that were joined keep their order for calls whose outputs lie over their inputs.
 inline bool overlaps(const void* p, int64_t pn, const void* q, int64_t qn) {
@@ -153,6 +152,7 @@ inline bool overlaps(const void* p, int64_t pn, const void* q, int64_t qn) {
   return p != nullptr && q != nullptr && x < y + static_cast<uintptr_t>(qn) && y < x + static_cast<uintptr_t>(pn);
 }
 
+// Standalone unit-triangular solve (kda_ut.hip); a [H][C][C], b/x/xf [H][C][N].
 struct UtArgs {
   const void* a;
   const void* b;    // right-hand side (the cotangent dX in the backward rule)
