@@ -104,12 +104,11 @@ __device__ __forceinline__ ChunkRows chunk_rows(const BwdArgs& a, int u) {
   return r;
 }
 
-// ROWS x COLS block of a row-major fp32 array (row stride src_ld floats,
-// first column col0) into LDS rows of pitch PITCH.  All of a thread's 16-byte
-// loads are issued before its LDS writes, so they are in flight together.
-// The two halves of lds_load: the loads into registers (a thread's share,
-// Tile::PER pieces of four elements) and the LDS writes.  Split, a scan kernel
-// issues the next chunk's loads before the current chunk's arithmetic.
+// ROWS x COLS block of a row-major array (row stride src_ld elements, first
+// column col0) into LDS rows, in two halves: the loads into registers (fetch; a
+// thread's share, Tile::PER pieces of four elements) and the LDS writes (put).
+// Apart, a scan kernel issues the next chunk's loads before the current chunk's
+// arithmetic.
 //
 // Workspace arrays are fp32 (ET 0) or fp16 (ET 2, see BwdWs); an fp16 tile
 // loads 8 bytes per piece and converts when it is written to LDS, so the wait
@@ -214,13 +213,6 @@ struct Tile {
   }
 };
 
-template <int ROWS, int COLS, int PITCH, int NTH = kThreads>
-__device__ __forceinline__ void lds_load(float* dst, const float* src, int src_ld, int col0) {
-  Tile<ROWS, COLS, NTH> t;
-  t.fetch(src, src_ld, col0);
-  t.template put<PITCH>(dst);
-}
-
 // Largest in-tile decay (log2 units, one channel) at which the chunk
 // kernel's diagonal score-adjoint tiles run on the matrix cores anchored at
 // the tile's first row: the key factors reach 2^kDiagAnchorLog2, which leaves
@@ -239,57 +231,10 @@ __device__ __forceinline__ bool scan_slot(int x, int nchains, int& chain, int& s
   return chain < nchains;
 }
 
-// Eight consecutive elements of an input tensor (DT 0 fp32, 1 bf16, 2 fp16)
-// as fp32.
-template <int DT>
-__device__ __forceinline__ void ld8(const void* p, int64_t i, float (&o)[8]) {
-  if constexpr (DT == 0) {
-    const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i);
-    const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + i + 4);
-    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
-    o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
-  } else {
-    const uint4 w = *reinterpret_cast<const uint4*>(static_cast<const u16*>(p) + i);
-    const f4 lo = unpack4<DT>(make_uint2(w.x, w.y)), hi = unpack4<DT>(make_uint2(w.z, w.w));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { o[e] = lo[e]; o[4 + e] = hi[e]; }
-  }
-}
-
-// Columns [col0, col0 + COLS) of the 64 rows of a chunk of a token-major
-// input tensor [*, H, D] (rows past `len` read as zero), times mul, into LDS
-// rows of pitch PITCH.  Loads issued together, 8 elements per load.
-template <int DT, int D, int COLS, int PITCH, int NTH = kThreads>
-__device__ __forceinline__ void lds_load_in(float* dst, const void* src, int64_t row0, int len, int H, int h,
-                                            int col0, float mul) {
-  constexpr int V = COLS / 8;
-  constexpr int N = kC * V;
-  constexpr int PER = (N + NTH - 1) / NTH;
-  static_assert(COLS % 8 == 0, "8-element loads");
-  // every thread loads (masked ones from row 0 of the chunk) and zeroes
-  // where it stores, so no load sits inside a branch
-  float tmp[PER][8];
-#pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    const int e = fresh_tid() + p * NTH;
-    const int r = e / V, c8 = e - r * V;
-    const bool ok = (N % NTH == 0 || e < N) && r < len;
-    ld8<DT>(src, ((row0 + (ok ? r : 0)) * H + h) * D + col0 + 8 * (ok ? c8 : 0), tmp[p]);
-  }
-#pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    const int e = fresh_tid() + p * NTH;
-    if (N % NTH == 0 || e < N) {
-      const int r = e / V, c8 = e - r * V;
-      const bool ok = r < len;
-#pragma unroll
-      for (int x = 0; x < 8; ++x) dst[r * PITCH + 8 * c8 + x] = ok ? tmp[p][x] * mul : 0.f;
-    }
-  }
-}
-
-// lds_load_in split into its loads (fetch) and its LDS writes (put), so a
-// kernel can issue the loads of a later phase before this phase's arithmetic.
+// Columns [col0, col0 + COLS) of the 64 rows of a chunk of a token-major input
+// tensor [*, H, D] (DT 0 fp32, 1 bf16, 2 fp16; rows past `len` read as zero),
+// 8 elements per load: the loads (fetch) and the LDS writes (put) are apart, so
+// a kernel can issue the loads of a later phase before this phase's arithmetic.
 template <int DT, int D, int COLS, int NTH>
 struct InTile {
   static constexpr int V = COLS / 8;
@@ -918,11 +863,8 @@ struct TTile {
 // (r, gq) holding K values 8 gq .. 8 gq + 7 of each 32-wide block): W and
 // (lambda k)^T, the state slice S^T and v~^T are kept in LDS as hi and lo
 // bf16 planes with the K index contiguous, so each fragment is one 16-byte
-// read.  The state itself stays fp32 in the accumulators.  With 16-bit inputs
-// every operand of both products is forward-side and fp16 (W and lambda k as
-// stored; S rounded as it is stored, v~ rounded for the product and stored
-// in fp32), so each product is one fp16 MFMA per K block, the forward
-// kernels' operand precision.
+// read.  The state itself stays fp32 in the accumulators.  (fp32 inputs; with
+// 16-bit ones fscan16_block and rscan16_block run.)
 template <int D>
 struct alignas(16) FscanLds {
   static constexpr int PW = D + 8;     // bf16 pitch of rows whose K index is a channel
@@ -934,9 +876,8 @@ struct alignas(16) FscanLds {
   float U[kC * kPB], GC[D];
 };
 
-template <int D, bool WS16>
+template <int D>
 __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLds<D>& L) {
-  constexpr int EF = BwdWs<WS16>::F;   // W, lambda k in; S_in out
   constexpr int NTH = ScanThreads<D>::value;
   constexpr int NS = D / 32;
   constexpr int NST = (D / 8) / (NTH / 64);   // state tiles per wave (D / 8 tiles of the 32-column slice)
@@ -966,7 +907,7 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
                     : 0.f;
   // chunk n's W, lambda*k and U slice are loaded into registers during
   // chunk n-1's arithmetic
-  typedef Tile<kC, D, NTH, EF> TD;
+  typedef Tile<kC, D, NTH> TD;
   TD tW;
   Tile<kC, 32, NTH> tU;
   // lambda*k, fetched for its transposed store: thread t holds rows 2 rp and
@@ -976,21 +917,20 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
   constexpr int KCG = NTH / 32;                    // column groups per pass
   constexpr int KPER = (D / 4) / KCG;              // float4 column groups per thread
   static_assert((D / 4) % KCG == 0, "lambda*k column groups");
-  typename WsPiece<EF>::t kq[KPER][2];
+  float4 kq[KPER][2];
   const int rp = t & 31, cg = t >> 5;
   float pgc;   // gamma_C of the chunk, loaded with its operands (every thread; t < D stores it)
   auto fetch = [&](int n) {
     const int64_t ch = (static_cast<int64_t>(b) * a.NT + n) * H + h;
     pgc = a.GCV[ch * D + (t & (D - 1))];
-    tW.fetch(ws_at<EF>(a.WM, ch * kC * D), D, 0);
-    const void* KLp = ws_at<EF>(a.KL, ch * kC * D);
+    tW.fetch(a.WM + ch * kC * D, D, 0);
+    const float* KLp = a.KL + ch * kC * D;
 #pragma unroll
     for (int j = 0; j < KPER; ++j)
 #pragma unroll
       for (int y = 0; y < 2; ++y) {
         const int i = (2 * rp + y) * D + 4 * (cg + KCG * j);
-        if constexpr (EF == 0) kq[j][y] = *reinterpret_cast<const float4*>(static_cast<const float*>(KLp) + i);
-        else kq[j][y] = *reinterpret_cast<const uint2*>(static_cast<const u16*>(KLp) + i);
+        kq[j][y] = *reinterpret_cast<const float4*>(KLp + i);
       }
     tU.fetch(a.UM + ch * kC * D, D, c0);
   };
@@ -1001,56 +941,37 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
     for (int q = 0; q < NST; ++q) {
       const int m0 = 16 * rt[q] + 4 * gq, col = 16 * cs[q] + r;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ws_st<EF>(a.SI, ch * D * D + (m0 + i) * D + c0 + col, S[q][i]);
-      if constexpr (WS16) {
-        *reinterpret_cast<uint2*>(&sSh[col * PW + m0]) = pack_f16x4(S[q]);
-      } else {
-        uint2 hh, ll;
-        split2_bf16(S[q][0], S[q][1], hh.x, ll.x);
-        split2_bf16(S[q][2], S[q][3], hh.y, ll.y);
-        *reinterpret_cast<uint2*>(&sSh[col * PW + m0]) = hh;
-        *reinterpret_cast<uint2*>(&sSl[col * PW + m0]) = ll;
-      }
+      for (int i = 0; i < 4; ++i) a.SI[ch * D * D + (m0 + i) * D + c0 + col] = S[q][i];
+      uint2 hh, ll;
+      split2_bf16(S[q][0], S[q][1], hh.x, ll.x);
+      split2_bf16(S[q][2], S[q][3], hh.y, ll.y);
+      *reinterpret_cast<uint2*>(&sSh[col * PW + m0]) = hh;
+      *reinterpret_cast<uint2*>(&sSl[col * PW + m0]) = ll;
     }
-    // W row-major and lambda*k transposed, as hi / lo planes (16-bit
-    // workspace: one fp16 plane each, the stored values as they are)
+    // W row-major and lambda*k transposed, as hi / lo planes
 #pragma unroll
     for (int p = 0; p < TD::PER; ++p) {
       const int e = t + p * NTH;
       const int row = e / TD::V, c4 = e - row * TD::V;
-      if constexpr (WS16) {
-        *reinterpret_cast<uint2*>(&sWh[row * PW + 4 * c4]) = tW.r[p];
-      } else {
-        const float4 w = tW.get(p);
-        uint2 hh, ll;
-        split2_bf16(w.x, w.y, hh.x, ll.x);
-        split2_bf16(w.z, w.w, hh.y, ll.y);
-        *reinterpret_cast<uint2*>(&sWh[row * PW + 4 * c4]) = hh;
-        *reinterpret_cast<uint2*>(&sWl[row * PW + 4 * c4]) = ll;
-      }
+      const float4 w = tW.get(p);
+      uint2 hh, ll;
+      split2_bf16(w.x, w.y, hh.x, ll.x);
+      split2_bf16(w.z, w.w, hh.y, ll.y);
+      *reinterpret_cast<uint2*>(&sWh[row * PW + 4 * c4]) = hh;
+      *reinterpret_cast<uint2*>(&sWl[row * PW + 4 * c4]) = ll;
     }
 #pragma unroll
     for (int j = 0; j < KPER; ++j) {
       const int ch4 = 4 * (cg + KCG * j);
-      if constexpr (WS16) {
-        // channel ch4 + e of rows 2 rp, 2 rp + 1: the e-th halves of the two
-        // rows' pieces, packed low / high
-        const uint2 w0 = kq[j][0], w1 = kq[j][1];
-        const unsigned pr[4] = {(w0.x & 0xFFFFu) | (w1.x << 16), (w0.x >> 16) | (w1.x & 0xFFFF0000u),
-                                (w0.y & 0xFFFFu) | (w1.y << 16), (w0.y >> 16) | (w1.y & 0xFFFF0000u)};
+      const float4 y0 = kq[j][0], y1 = kq[j][1];
+      const float k0[4] = {y0.x, y0.y, y0.z, y0.w};
+      const float k1[4] = {y1.x, y1.y, y1.z, y1.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) *reinterpret_cast<unsigned*>(&sKh[(ch4 + e) * PK + 2 * rp]) = pr[e];
-      } else {
-        const float4 y0 = ws_unpack<EF>(kq[j][0]), y1 = ws_unpack<EF>(kq[j][1]);
-        const float k0[4] = {y0.x, y0.y, y0.z, y0.w};
-        const float k1[4] = {y1.x, y1.y, y1.z, y1.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          unsigned hh, ll;
-          split2_bf16(k0[e], k1[e], hh, ll);     // rows 2 rp, 2 rp + 1 of channel ch4 + e
-          *reinterpret_cast<unsigned*>(&sKh[(ch4 + e) * PK + 2 * rp]) = hh;
-          *reinterpret_cast<unsigned*>(&sKl[(ch4 + e) * PK + 2 * rp]) = ll;
-        }
+      for (int e = 0; e < 4; ++e) {
+        unsigned hh, ll;
+        split2_bf16(k0[e], k1[e], hh, ll);     // rows 2 rp, 2 rp + 1 of channel ch4 + e
+        *reinterpret_cast<unsigned*>(&sKh[(ch4 + e) * PK + 2 * rp]) = hh;
+        *reinterpret_cast<unsigned*>(&sKl[(ch4 + e) * PK + 2 * rp]) = ll;
       }
     }
     tU.template put<kPB>(sU);
@@ -1064,13 +985,9 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
       for (int kb = 0; kb < D / 32; ++kb) {
         const int ka = (16 * mt + r) * PW + 32 * kb + 8 * gq, kbb = (16 * ct + r) * PW + 32 * kb + 8 * gq;
         f4& acc = (kb & 1) ? acc1 : acc0;
-        if constexpr (WS16) {
-          acc = mma32(acc, *reinterpret_cast<const h8*>(&sWh[ka]), *reinterpret_cast<const h8*>(&sSh[kbb]));
-        } else {
-          const b8 ah = *reinterpret_cast<const b8*>(&sWh[ka]), al = *reinterpret_cast<const b8*>(&sWl[ka]);
-          const b8 bh = *reinterpret_cast<const b8*>(&sSh[kbb]), bl = *reinterpret_cast<const b8*>(&sSl[kbb]);
-          acc = mma3_bf16(acc, ah, al, bh, bl);
-        }
+        const b8 ah = *reinterpret_cast<const b8*>(&sWh[ka]), al = *reinterpret_cast<const b8*>(&sWl[ka]);
+        const b8 bh = *reinterpret_cast<const b8*>(&sSh[kbb]), bl = *reinterpret_cast<const b8*>(&sSl[kbb]);
+        acc = mma3_bf16(acc, ah, al, bh, bl);
       }
       float v[4];
 #pragma unroll
@@ -1079,15 +996,11 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
         v[i] = sU[row * kPB + col] - (acc0[i] + acc1[i]);
         a.VT[ch * kC * D + row * D + c0 + col] = v[i];
       }
-      if constexpr (WS16) {
-        *reinterpret_cast<uint2*>(&sVh[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = pack_f16x4(f4{v[0], v[1], v[2], v[3]});
-      } else {
-        uint2 hh, ll;
-        split2_bf16(v[0], v[1], hh.x, ll.x);
-        split2_bf16(v[2], v[3], hh.y, ll.y);
-        *reinterpret_cast<uint2*>(&sVh[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = hh;
-        *reinterpret_cast<uint2*>(&sVl[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = ll;
-      }
+      uint2 hh, ll;
+      split2_bf16(v[0], v[1], hh.x, ll.x);
+      split2_bf16(v[2], v[3], hh.y, ll.y);
+      *reinterpret_cast<uint2*>(&sVh[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = hh;
+      *reinterpret_cast<uint2*>(&sVl[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = ll;
     }
     __syncthreads();
     // S <- gamma_C S + (lambda k)^T v~
@@ -1100,11 +1013,8 @@ __device__ __forceinline__ void fscan_block(const BwdArgs& a, int block, FscanLd
 #pragma unroll
       for (int q = 0; q < NST; ++q) {
         const int ka = (16 * rt[q] + r) * PK + 32 * kb + 8 * gq, kbb = (16 * cs[q] + r) * PK + 32 * kb + 8 * gq;
-        if constexpr (WS16)
-          S[q] = mma32(S[q], *reinterpret_cast<const h8*>(&sKh[ka]), *reinterpret_cast<const h8*>(&sVh[kbb]));
-        else
-          S[q] = mma3_bf16(S[q], *reinterpret_cast<const b8*>(&sKh[ka]), *reinterpret_cast<const b8*>(&sKl[ka]),
-                           *reinterpret_cast<const b8*>(&sVh[kbb]), *reinterpret_cast<const b8*>(&sVl[kbb]));
+        S[q] = mma3_bf16(S[q], *reinterpret_cast<const b8*>(&sKh[ka]), *reinterpret_cast<const b8*>(&sKl[ka]),
+                         *reinterpret_cast<const b8*>(&sVh[kbb]), *reinterpret_cast<const b8*>(&sVl[kbb]));
       }
     __syncthreads();
   }
@@ -1140,9 +1050,8 @@ struct alignas(16) RscanLds {
   float GC[D];
 };
 
-template <int D, int DO, bool WS16>
+template <int D, int DO>
 __device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLds<D>& L) {
-  constexpr int EF = BwdWs<WS16>::F;    // lambda k, Aqk, gamma q, W in
   constexpr int NTH = ScanThreads<D>::value;
   constexpr int NS = D / 32;
   constexpr int NST = (D / 8) / (NTH / 64);
@@ -1177,9 +1086,9 @@ __device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLd
   // each: a set is reloaded right after it is staged, so every load has a
   // whole chunk step to arrive.  The do slice is held as loaded (raw words),
   // so that no wait falls at its load.
-  Tile<kC, D, NTH, EF> tL;
-  TTile<kC, kScanThreads, EF> tA;   // threads t < kScanThreads
-  TTile<D, NTH, EF> tQ, tW;
+  Tile<kC, D, NTH> tL;
+  TTile<kC, kScanThreads> tA;   // threads t < kScanThreads
+  TTile<D, NTH> tQ, tW;
   const bool a_thread = t < kScanThreads;
   float pgc;   // gamma_C of the chunk (every thread; t < D stages it)
   // do^T of the slice, spread over every thread: thread t holds rows 2 rp,
@@ -1200,9 +1109,9 @@ __device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLd
   auto fetch_a = [&](int n) {   // lambda k, Aqk, gamma q, gamma_C and do of chunk n
     const int u = b * a.NT + n;
     const int64_t ch = chead(n);
-    tL.fetch(ws_at<EF>(a.KL, ch * kC * D), D, 0);
-    if (a_thread) tA.fetch(ws_at<EF>(a.AQ, ch * kC * kC), kC, 0);
-    tQ.fetch(ws_at<EF>(a.QG, ch * kC * D), D, 0);
+    tL.fetch(a.KL + ch * kC * D, D, 0);
+    if (a_thread) tA.fetch(a.AQ + ch * kC * kC, kC, 0);
+    tQ.fetch(a.QG + ch * kC * D, D, 0);
     pgc = a.GCV[ch * D + (t & (D - 1))];
     const ChunkRows crn = chunk_rows(a, u);
 #pragma unroll
@@ -1233,7 +1142,7 @@ __device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLd
   };
   if (a.NT > 0) {
     fetch_a(a.NT - 1);
-    tW.fetch(ws_at<EF>(a.WM, chead(a.NT - 1) * kC * D), D, 0);
+    tW.fetch(a.WM + chead(a.NT - 1) * kC * D, D, 0);
     put_a(a.NT - 1);
     if (a.NT > 1) fetch_a(a.NT - 2);
     __syncthreads();
@@ -1294,7 +1203,7 @@ __device__ __forceinline__ void rscan_block(const BwdArgs& a, int block, RscanLd
       *reinterpret_cast<uint2*>(&sVl[(16 * ct + r) * PK + 16 * mt + 4 * gq]) = ll;
     }
     tW.template put_hl<PK>(sWh, sWl);
-    if (n > 0) tW.fetch(ws_at<EF>(a.WM, chead(n - 1) * kC * D), D, 0);
+    if (n > 0) tW.fetch(a.WM + chead(n - 1) * kC * D, D, 0);
     __syncthreads();
     // ---- C: dS <- dS - W^T dv~; the next chunk's lambda k, Aqk^T, do^T,
     // (gamma q)^T and gamma_C staged while the products run
@@ -1981,8 +1890,8 @@ __global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_scans_kernel(Bw
   constexpr size_t N = sizeof(RscanLds<D>) > sizeof(FscanLds<D>) ? sizeof(RscanLds<D>) : sizeof(FscanLds<D>);
   __shared__ __attribute__((aligned(16))) unsigned char sm[N];
   const int x = blockIdx.x;
-  if (x < nblk) rscan_block<D, DO, false>(a, x, *reinterpret_cast<RscanLds<D>*>(sm));
-  else fscan_block<D, false>(a, x - nblk, *reinterpret_cast<FscanLds<D>*>(sm));
+  if (x < nblk) rscan_block<D, DO>(a, x, *reinterpret_cast<RscanLds<D>*>(sm));
+  else fscan_block<D>(a, x - nblk, *reinterpret_cast<FscanLds<D>*>(sm));
 }
 
 // The forward scan alone, in LDS of its own size: at d = 64 two workgroups of it
@@ -1996,7 +1905,7 @@ __global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_scans_kernel(Bw
 template <int D>
 __global__ __launch_bounds__(ScanThreads<D>::value) void kda_bwd_fscan_kernel(BwdArgs a) {
   __shared__ FscanLds<D> L;
-  fscan_block<D, false>(a, blockIdx.x, L);
+  fscan_block<D>(a, blockIdx.x, L);
 }
 constexpr int kForwardApart = 2048;   // forward scan workgroups
 
