@@ -77,11 +77,13 @@ _SIGNATURES = {
 
 # Entry points of this binding's own, outside the C ABI of the header: the two
 # backward calls whose outputs may be rounded to the primals' 16-bit types by
-# the kernels that form them (axiom_amd/csrc/kda_internal.h)
+# the kernels that form them, and the seam's backward with the workspace its
+# direct form needs (axiom_amd/csrc/kda_internal.h)
 _PRIVATE = {
     "axiom_chunk_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                              _vp, _vp, _vp, _vp, _vp, _vp,
                              _i, _i, _i, _i, _i, _i, _f, _i, _i, _i, _i, _vp, _sz]),
+    "axiom_cc_scan_bwd": (_i, [_vp] * 15 + [_i, _i, _i, _i, _i, _i, _i, _vp, _sz]),
     "axiom_prologue_bwd": (_i, [_vp] * 22 + [_i, _i, _i, _i, _i, _i, _i, _vp, _sz]),
 }
 

@@ -857,7 +857,7 @@ int kda_cc_scan_batched(hipStream_t stream, const void* q, const void* k, const 
   // The (B, T, H*d) operands are the [B, T, H, d] layout of the chunked
   // forward; its intra kernel takes the log-decay of alpha (log2 alpha, in
   // its own units) and beta = mean(beta32) (in kda_adapt_kernel's column
-  // order; the backward runs that adapter) itself.  The workspace keeps the
+  // order) itself.  The workspace keeps the
   // adapter's g and beta areas unused, so both directions size it the same
   // way.
   void* rest = static_cast<char*>(workspace) + g_bytes + b_bytes;
@@ -960,12 +960,15 @@ size_t kda_cc_scan_bwd_workspace(int T, int H, int dk, int dv, int chunk) {
   return kda_cc_scan_bwd_batched_workspace(1, T, H, dk, dv, chunk);
 }
 
-int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, const void* v,
+// The seam's backward.  own_workspace: the caller brings the dense backward's
+// workspace alone where the direct form runs (the package's binding), else
+// kda_cc_scan_bwd_batched_workspace's bytes whichever form runs.
+static int cc_scan_bwd_impl(hipStream_t stream, const void* q, const void* k, const void* v,
                             const float* alpha, const float* beta32, const float* S_in,
                             const float* d_o, const float* dS, void* dq, void* dk, void* dv,
                             float* dalpha, float* dbeta32, float* dS_in,
                             int B, int T, int H, int dk_dim, int dv_dim, int tile, int chunk,
-                            void* workspace, size_t workspace_bytes) {
+                            void* workspace, size_t workspace_bytes, bool own_workspace) {
   g_err[0] = '\0';
   if (B < 1) return fail(KDA_ERR_INVALID_ARGUMENT, "B=%d must be >= 1", B);
   if (!q || !k || !v || !alpha || !beta32 || !S_in || !d_o || !dS || !dq || !dk || !dv || !dalpha ||
@@ -982,23 +985,7 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   if (int rc = require_aligned(16, "q, k, v, S_in, do, dS, dS_in and the workspace",
                                {q, k, v, S_in, d_o, dS, dS_in, workspace}))
     return rc;
-  const size_t need = kda_cc_scan_bwd_batched_workspace(B, T, H, dk_dim, dv_dim, chunk);
-  if (workspace == nullptr || workspace_bytes < need)
-    return fail(KDA_ERR_WORKSPACE, "workspace of %zu bytes is too small (need %zu)", workspace_bytes, need);
   const size_t th = static_cast<size_t>(B) * T * H;
-  unsigned char* ws = static_cast<unsigned char*>(workspace);
-  float* g32 = reinterpret_cast<float*>(ws);
-  ws += align_up(th * dk_dim * 4);
-  float* b32 = reinterpret_cast<float*>(ws);
-  ws += align_up(th * 4);
-  float* f[4];
-  for (int i = 0; i < 4; ++i) {
-    f[i] = reinterpret_cast<float*>(ws);
-    ws += align_up(th * dk_dim * 4);
-  }
-  float* dbeta = reinterpret_cast<float*>(ws);
-  ws += align_up(th * 4);
-  const size_t rest = workspace_bytes - static_cast<size_t>(ws - static_cast<unsigned char*>(workspace));
   // The kernels take the seam's operands as they are (log alpha and the mean
   // of beta32 in the prep and chunk kernels, bf16 / dalpha / dbeta32 outputs
   // from the chunk kernel) when every pointer allows their 16-byte (dq, dk,
@@ -1019,8 +1006,13 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   bool apart = true;
   for (const auto& x : grad)
     for (const auto& y : in) apart = apart && !kda::overlaps(x.p, x.n, y.p, y.n);
-  if (T > 0 && apart && (a16 & 15) == 0 && (a4 & 3) == 0 && static_cast<int64_t>(B) * nt * H <= 0x7FFFFFFFLL &&
-      th * dk_dim < (1ULL << 40)) {
+  const bool direct = T > 0 && apart && (a16 & 15) == 0 && (a4 & 3) == 0 &&
+                      static_cast<int64_t>(B) * nt * H <= 0x7FFFFFFFLL && th * dk_dim < (1ULL << 40);
+  const size_t need = direct && own_workspace ? bwd_layout(B, T, H, dk_dim).total
+                                              : kda_cc_scan_bwd_batched_workspace(B, T, H, dk_dim, dv_dim, chunk);
+  if (workspace == nullptr || workspace_bytes < need)
+    return fail(KDA_ERR_WORKSPACE, "workspace of %zu bytes is too small (need %zu)", workspace_bytes, need);
+  if (direct) {
     kda::BwdArgs a{};
     a.B = B; a.T = T; a.H = H; a.NT = static_cast<int>(nt);
     a.q = q; a.k = k; a.v = v; a.g = alpha; a.beta = beta32;
@@ -1028,11 +1020,24 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
     a.dq = dq; a.dk = dk; a.dv = dv; a.dg = dalpha; a.dbeta = dbeta32; a.dh0 = dS_in;
     a.qkv_out = KDA_DTYPE_BF16;
     a.g_out = KDA_DTYPE_F32;
-    bwd_workspace(a, bwd_layout(B, T, H, dk_dim), ws);
+    bwd_workspace(a, bwd_layout(B, T, H, dk_dim), static_cast<unsigned char*>(workspace));
     const hipError_t e = kda::launch_bwd(a, dk_dim, kda::kInAlphaGates, 0, stream);
     if (e != hipSuccess) return hip_fail(e, "cc_scan backward launch");
     return KDA_OK;
   }
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  float* g32 = reinterpret_cast<float*>(ws);
+  ws += align_up(th * dk_dim * 4);
+  float* b32 = reinterpret_cast<float*>(ws);
+  ws += align_up(th * 4);
+  float* f[4];
+  for (int i = 0; i < 4; ++i) {
+    f[i] = reinterpret_cast<float*>(ws);
+    ws += align_up(th * dk_dim * 4);
+  }
+  float* dbeta = reinterpret_cast<float*>(ws);
+  ws += align_up(th * 4);
+  const size_t rest = workspace_bytes - static_cast<size_t>(ws - static_cast<unsigned char*>(workspace));
   kda::AdaptArgs aa{};
   aa.alpha = alpha; aa.beta32 = beta32; aa.g_out = g32; aa.beta_out = b32;
   aa.n_tok_heads = static_cast<int64_t>(th);
@@ -1051,6 +1056,26 @@ int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, co
   e = kda::launch_cc_finish(fa, stream);
   if (e != hipSuccess) return hip_fail(e, "cc_scan backward finish launch");
   return KDA_OK;
+}
+
+int kda_cc_scan_bwd_batched(hipStream_t stream, const void* q, const void* k, const void* v,
+                            const float* alpha, const float* beta32, const float* S_in,
+                            const float* d_o, const float* dS, void* dq, void* dk, void* dv,
+                            float* dalpha, float* dbeta32, float* dS_in,
+                            int B, int T, int H, int dk_dim, int dv_dim, int tile, int chunk,
+                            void* workspace, size_t workspace_bytes) {
+  return cc_scan_bwd_impl(stream, q, k, v, alpha, beta32, S_in, d_o, dS, dq, dk, dv, dalpha, dbeta32, dS_in, B, T, H,
+                          dk_dim, dv_dim, tile, chunk, workspace, workspace_bytes, false);
+}
+
+int axiom_cc_scan_bwd(hipStream_t stream, const void* q, const void* k, const void* v,
+                      const float* alpha, const float* beta32, const float* S_in,
+                      const float* d_o, const float* dS, void* dq, void* dk, void* dv,
+                      float* dalpha, float* dbeta32, float* dS_in,
+                      int B, int T, int H, int dk_dim, int dv_dim, int tile, int chunk,
+                      void* workspace, size_t workspace_bytes) {
+  return cc_scan_bwd_impl(stream, q, k, v, alpha, beta32, S_in, d_o, dS, dq, dk, dv, dalpha, dbeta32, dS_in, B, T, H,
+                          dk_dim, dv_dim, tile, chunk, workspace, workspace_bytes, true);
 }
 
 int kda_cc_scan_bwd(hipStream_t stream, const void* q, const void* k, const void* v,

@@ -295,8 +295,16 @@ hipError_t launch_cc_finish(const CcFinishArgs& a, hipStream_t s);
 // the caller.  dq, dk, dv in qkv_grad_dtype (KDA_DTYPE_F32 or the dtype of q,
 // k, v), dg and dbeta in gate_grad_dtype (F32 or the dtype of g, beta); dqp,
 // dkp, dvp in dx_dtype (F32 or in_dtype).  A 16-bit gradient is the fp32 one
-// rounded to nearest even by the kernel that forms it.
+// rounded to nearest even by the kernel that forms it.  And
+// kda_cc_scan_bwd_batched for fresh outputs: where alpha and beta32 are aligned
+// to 16 bytes and T > 0 it needs kda_chunk_bwd_workspace's bytes only (the seam's
+// own query keeps room for the two-pass form: at B2 T8192 H12 d128 half a GB more).
 extern "C" {
+__attribute__((visibility("default"))) int axiom_cc_scan_bwd(
+    hipStream_t stream, const void* q, const void* k, const void* v, const float* alpha, const float* beta32,
+    const float* S_in, const float* d_o, const float* dS, void* dq, void* dk, void* dv, float* dalpha, float* dbeta32,
+    float* dS_in, int B, int T, int H, int dk_dim, int dv_dim, int tile, int chunk, void* workspace,
+    size_t workspace_bytes);
 __attribute__((visibility("default"))) int axiom_chunk_bwd(
     hipStream_t stream, const void* q, const void* k, const void* v, const void* g, const void* beta, const float* h0,
     const void* dout, const float* dht, void* dq, void* dk, void* dv, void* dg, void* dbeta, float* dh0, int B, int T,

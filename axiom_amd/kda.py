@@ -865,7 +865,11 @@ def cc_scan_bwd(q, k, v, alpha, beta32, S, do, dS=None, tile: int = 16, chunk: i
     dev = _require_gpu([q, k, v, alpha, beta32, S, do, dS], what)
     L = _lib.lib()
     nb = max(B, 1)
-    ws_bytes = _ws_bytes("kda_cc_scan_bwd_batched_workspace", nb, T, H, dk, dv, C)
+    # fresh outputs and 16-byte-aligned gates: the form without passes of its own
+    if T > 0 and (alpha.data_ptr() | beta32.data_ptr()) % 16 == 0:
+        ws_bytes = _ws_bytes("kda_chunk_bwd_workspace", nb, T, H, dk, dv, CHUNK)
+    else:
+        ws_bytes = _ws_bytes("kda_cc_scan_bwd_batched_workspace", nb, T, H, dk, dv, C)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     dq = torch.empty_like(q)
     dk_ = torch.empty_like(k)
@@ -873,10 +877,10 @@ def cc_scan_bwd(q, k, v, alpha, beta32, S, do, dS=None, tile: int = 16, chunk: i
     dalpha = torch.empty_like(alpha)
     dbeta32 = torch.empty_like(beta32)
     dS_in = torch.empty_like(S)
-    rc = L.kda_cc_scan_bwd_batched(_stream(dev), _ptr(q), _ptr(k), _ptr(v), _ptr(alpha), _ptr(beta32), _ptr(S),
-                                   _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dalpha),
-                                   _ptr(dbeta32), _ptr(dS_in), nb, T, H, dk, dv, int(tile), C,
-                                   _ptr(workspace), ws_bytes)
+    rc = L.axiom_cc_scan_bwd(_stream(dev), _ptr(q), _ptr(k), _ptr(v), _ptr(alpha), _ptr(beta32), _ptr(S),
+                             _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk_), _ptr(dv_), _ptr(dalpha),
+                             _ptr(dbeta32), _ptr(dS_in), nb, T, H, dk, dv, int(tile), C,
+                             _ptr(workspace), ws_bytes)
     _lib.check(rc, what)
     return dq, dk_, dv_, dalpha, dbeta32, dS_in
 

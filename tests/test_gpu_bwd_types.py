@@ -75,3 +75,21 @@ def test_seam_backward_of_misaligned_gates_matches(cuda, T, H, d, which):
     torch.cuda.synchronize()
     for i, (a, b) in enumerate(zip(got, want)):
         assert a.dtype == b.dtype and torch.equal(a, b), i
+
+
+def test_seam_backward_brings_the_dense_workspace_alone(cuda):
+    """Beside its outputs a call with aligned gates allocates what the dense backward needs, no room for
+    the two-pass form's fp32 gradients and gates (blocks are rounded up to 512 bytes)."""
+    import axiom_amd
+    from axiom_amd import kda
+    T, H, d = 1024, 2, 128
+    q, k, v = (torch.randn(T, H * d, device=cuda).to(torch.bfloat16) * 0.1 for _ in range(3))
+    alpha, beta32 = torch.rand(T, H * d, device=cuda) * 0.5 + 0.5, torch.rand(T, H * 32, device=cuda)
+    S, do, dS = torch.randn(H, d, d, device=cuda), torch.randn(T, H * d, device=cuda), torch.randn(H, d, d, device=cuda)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = axiom_amd.cc_scan_bwd(q, k, v, alpha, beta32, S, do, dS, chunk=32)
+    used = torch.cuda.max_memory_allocated() - before
+    need = kda._ws_bytes("kda_chunk_bwd_workspace", 1, T, H, d, d, 64) + sum(t.numel() * t.element_size() for t in out)
+    assert need <= used <= need + 512 * (len(out) + 1)
