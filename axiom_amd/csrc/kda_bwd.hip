@@ -367,11 +367,12 @@ __device__ __forceinline__ int fa_frag(int it, int kb) { return (it < 2) ? 2 * i
 // gamma k (kept in registers for W).  The scores read their operands 16 bytes
 // at a time, four channels per lane for four v_mfma_f32_16x16x4f32, and a tile
 // pair costs one factor 2^(Ga_R - Ge_s) per channel.
-// Bound by its phases' latencies beside its traffic (200 KiB per chunk-head at
-// d = 128, 16-bit inputs: 160 us of 4 096 chunk-heads at the copy rate).  4 096
-// chunk-heads, 16-bit inputs: 267 us with each decay factor formed per operand
-// and tile pair, element-wise LDS reads and the first half's k, g staged again
-// for W; 212 now; 3 072 with the seam's gates 227 -> 167; 256 in fp32 29 -> 24.
+// Bound by its phases' latencies beside its traffic (192 KiB per chunk-head at
+// d = 128, 16-bit inputs: 155 us of 4 096 chunk-heads at the copy rate).  4 096
+// chunk-heads, 16-bit inputs, traced medians: 273 us with each decay factor
+// formed per operand and tile pair, element-wise LDS reads and the first half's
+// k, g staged again for W; 214 now (within a training step of the layer 291 and
+// 234); 3 072 of the seam's 229 (and an adapter pass) and 185; 256 in fp32 30 and 25.
 template <int D, int DTQ, int DTG>
 __global__ __launch_bounds__(kPrepThreads, 4) void kda_bwd_prep_kernel(BwdArgs a) {
   constexpr int EF = BwdWs<DTQ != 0>::F;   // gamma q, lambda k, Aqk, T, W
@@ -1872,7 +1873,8 @@ __device__ __forceinline__ void fscan16_block(const BwdArgs& a, int block, Fscan
 // ones, come first: with more workgroups than CUs the forward ones fill in as
 // CUs free up.  Whole backward against the two scans one after the other
 // (d = 128, 16-bit inputs): 24 chains of 128 chunks 1 137 -> 974 us, 48 of 64
-// 935 -> 896, 64 of 64 1 120 -> 1 117; fp32, 16 of 16 176 -> 138; the same bits.
+// 935 -> 896, 64 of 64 1 120 -> 1 117; fp32, 16 of 16 176 -> 138; d = 64, 16-bit
+// inputs, 132 of 16 345 -> 315, 512 of 8 576 -> 569; the same bits.
 // ---------------------------------------------------------------------------
 static_assert(kRsProducers == kFsProducers, "one workgroup size");
 
@@ -2005,12 +2007,14 @@ struct Col4 {
 //   3  dL = -(Yw W^T + Yu U^T)
 //   4  the score adjoints of the wave's row tile (row side) and key tile
 //      (column side); dg's reverse cumsum; dq, dk, dg, dbeta stored
-// Bound by the phases' latencies at one workgroup per CU (LDS) beside the 480
-// KiB it moves per chunk-head (d = 128, 16-bit inputs: 380 us of a 4 096
+// Bound by the phases' latencies at one workgroup per CU (LDS) beside the 447
+// KiB it moves per chunk-head (d = 128, 16-bit inputs: 360 us of a 4 096
 // chunk-head call at the copy rate).  d = 128, 4 096 chunk-heads, 16-bit
-// inputs: 658 us with two waves per SIMD, a decay factor formed per operand
-// and tile pair and the operands read element by element from LDS in phase 4,
-// and two-byte column reads of q, k, v, g from memory; 561 us now.
+// inputs, traced medians: 657 us with two waves per SIMD, a decay factor formed
+// per operand and tile pair and the operands read element by element from LDS in
+// phase 4, and two-byte column reads of q, k, v, g from memory; 559 us now
+// (within a training step of the layer 691 and 588); 3 072 of the seam's 511 and
+// 472, 256 in fp32 48 and 42.
 // ---------------------------------------------------------------------------
 template <int D, int DTQ, int DTG, int DO>
 __global__ __launch_bounds__(ChunkThreads<D>::value) void kda_bwd_chunk_kernel(BwdArgs a) {

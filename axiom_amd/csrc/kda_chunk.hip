@@ -1196,8 +1196,9 @@ void kda_intra_kernel(IntraArgs a) {
 // slices on twice the CUs; past that they only add reads and barriers.
 // Four waves doing all of it on two-tile slices: 24.3 us (B1 T512 H4 d64) and
 // 77 us (B2 T1024 H8 d128) of state launch; one-tile slices 16.2 and 51, the
-// output waves too 15.4 and 49.6.  Where slices stay two-tile the output waves
-// gain 1 to 8 % of the call (B8 T2048 H32 d64 575 -> 533 us).
+// output waves too 14.9 and 47.8.  Where slices stay two-tile the whole call
+// takes 0.89 to 0.97 of the four-wave form's time at d = 64 (B16 T512 H32 328 and
+// 293 us) and 0.96 to 1.00 at d = 128 (878 and 881).
 // ----------------------------------------------------------------------------
 template <int DK, int ET>
 struct ExactChainFrags {

@@ -384,7 +384,7 @@ def bench_layer(args, fwd_inputs, device):
     return dict(us_per_call=t_call * 1e6, tokens_per_s=B * T / t_call, unfused_us_per_call=t_unfused * 1e6,
                 roofline={"bound": "hbm", "achieved": gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                           "frac": gbps / HBM_PEAK_GBPS, "algorithmic_bytes_per_call": nbytes},
-                kernels="kda_intra_kernel with the fused short conv + kda_state_col_kernel + kda_epilogue_kernel",
+                kernels="kda_intra_kernel with the fused short conv + kda_state_col_kernel + kda_epilogue_buf_kernel",
                 config="B4 T4096 H16 d128 K4, bf16 projections, gates and y, fp32 o inside, zero h0")
 
 
