@@ -46,3 +46,20 @@ def test_exact_packed_sequences(cuda):
             assert torch.equal(o[:, s:e], oi) and torch.equal(ht[i:i + 1], hi), i
         else:
             assert torch.equal(ht[i], t["h0"][i])
+
+
+@pytest.mark.parametrize("T", [64, 128, 192, 300])
+def test_many_chains_in_short_segments(cuda, T):
+    """512 chains run in segments of one to a few chunks, where a segment ends while fragments would still
+    be loaded ahead; a row of the batch by itself runs in one.  The same bits."""
+    import axiom_amd
+    B, H, d = 16, 32, 128
+    g = torch.Generator(device=cuda).manual_seed(T)
+    R = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    q, k = (torch.nn.functional.normalize(R(B, T, H, d), dim=-1) for _ in range(2))
+    ops = [q, k, R(B, T, H, d), -torch.nn.functional.softplus(R(B, T, H, d)), torch.sigmoid(R(B, T, H))]
+    h0 = R(B, H, d, d) * 0.1
+    o, ht = axiom_amd.kda_chunk_fwd(*ops, initial_state=h0)
+    for b in (0, B - 1):
+        one, h1 = axiom_amd.kda_chunk_fwd(*(x[b:b + 1] for x in ops), initial_state=h0[b:b + 1])
+        assert torch.equal(o[b:b + 1], one) and torch.equal(ht[b:b + 1], h1)
